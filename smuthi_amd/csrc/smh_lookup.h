@@ -6,6 +6,8 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "smh_op.h"
@@ -27,7 +29,10 @@ struct KernelInfo {
 
 // Receiver chunk of a precision: as many receivers (at most 512, the pair
 // record's receiver field) as the LDS accumulator [Rc][SY] and one counter
-// int per receiver fit in one workgroup's LDS, less 1 KiB.
+// int per receiver fit in one workgroup's LDS, less 1 KiB, evened out over the
+// chunks that takes: a chunk never covers receivers that do not exist, whose
+// accumulators every work item would zero, write and have summed (50 particles
+// at l_max 3 in FP32: 336 -> 50 receivers).
 inline int chunk_size(const smh_op* op, size_t real_size, int sy, size_t& lds) {
   const size_t limit = std::min<size_t>(op->ctx->lds_per_block ? op->ctx->lds_per_block : 65536, 163840) - 1024;
   const size_t per = (size_t)sy * real_size + sizeof(int);
@@ -36,26 +41,69 @@ inline int chunk_size(const smh_op* op, size_t real_size, int sy, size_t& lds) {
     lds = 0;
     return 0;
   }
+  const int64_t chunks = (op->n_part + rc - 1) / rc;
+  rc = (int)((op->n_part + chunks - 1) / chunks);
   lds = (size_t)rc * per + 16;
   return rc;
 }
 
-// Sum the work-item accumulators of each receiver chunk in fixed order
-// (y = sum, or y += sum when accumulate is set).
+// Strands of the partial-sum reductions: the items of a chunk are cut into
+// runs of strand_len, each summed by its own threads in item order, and the
+// runs added in order. Launches with few results would otherwise leave the
+// chip to a few threads that each wait for one item's value after the other:
+// 50 spheres, l_max 3 (1500 results, 648 items): 166 us with one strand. With
+// 128k results and more, one strand per result fills the chip.
+struct Strands {
+  int count, len;
+};
+inline Strands reduce_strands(int64_t results, int max_chunk_items) {
+  const int want = results <= 16384 ? 16 : (results <= 131072 ? 4 : 1);
+  const int count = std::max(1, std::min(want, max_chunk_items / 4));
+  return {count, std::max(1, (max_chunk_items + count - 1) / count)};
+}
+inline dim3 reduce_block(Strands st) { return st.count == 1 ? dim3(256, 1) : dim3(64, st.count); }
+inline int reduce_blocks(Strands st, int64_t results) { return blocks_for(results, st.count == 1 ? 256 : 64); }
+constexpr int kMaxStrands = 16;
+
+// Add the strands' sums in order; the first strand's threads get the total.
 template <typename Real>
-__global__ void reduce_kernel(const Real* __restrict__ ypart, const int* __restrict__ chunk_items, int Rc, int B,
-                              int64_t n_part, typename Vec2<Real>::t* y, int accumulate) {
+__device__ inline void add_strands(Real& re, Real& im) {
+  __shared__ Real part[kMaxStrands][2][64];
+  if (blockDim.y == 1) return;
+  part[threadIdx.y][0][threadIdx.x] = re;
+  part[threadIdx.y][1][threadIdx.x] = im;
+  __syncthreads();
+  if (threadIdx.y == 0)
+    for (int k = 1; k < (int)blockDim.y; ++k) {
+      re += part[k][0][threadIdx.x];
+      im += part[k][1][threadIdx.x];
+    }
+}
+
+// Sum the work-item accumulators of each receiver chunk in fixed order
+// (y = sum, or y += sum when accumulate is set). HBM-bound on the partials
+// once enough loads are in flight (strands, eight items unrolled).
+template <typename Real>
+__global__ void reduce_kernel(const Real* __restrict__ ypart, const int* __restrict__ chunk_items, int strand_len,
+                              int Rc, int B, int64_t n_part, typename Vec2<Real>::t* y, int accumulate) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n_part * B) return;
-  const int64_t i1 = j / B;
-  const int n1 = (int)(j - i1 * B);
-  const int c = (int)(i1 / Rc), il = (int)(i1 - (int64_t)c * Rc);
+  const bool act = j < n_part * B;
   Real re = 0, im = 0;
-  for (int w = chunk_items[c]; w < chunk_items[c + 1]; ++w) {
-    const Real* p = ypart + ((size_t)w * Rc + il) * 2 * B;
-    re += p[n1];
-    im += p[B + n1];
+  if (act) {
+    const int64_t i1 = j / B;
+    const int n1 = (int)(j - i1 * B);
+    const int c = (int)(i1 / Rc), il = (int)(i1 - (int64_t)c * Rc);
+    const int w0 = chunk_items[c] + threadIdx.y * strand_len;
+    const int w1 = min(chunk_items[c + 1], w0 + strand_len);
+#pragma unroll 8
+    for (int w = w0; w < w1; ++w) {
+      const Real* p = ypart + ((size_t)w * Rc + il) * 2 * B;
+      re += p[n1];
+      im += p[B + n1];
+    }
   }
+  add_strands(re, im);
+  if (!act || threadIdx.y > 0) return;
   if (accumulate) {
     re += y[j].x;
     im += y[j].y;
@@ -64,31 +112,58 @@ __global__ void reduce_kernel(const Real* __restrict__ ypart, const int* __restr
 }
 
 // Sum the work items of each chunk for the kBatch-RHS kernels: partial
-// [Rc][kBatch][2][S] (slot order when slot is given, else S = B) -> y
-// [n_part][B][kBatch] (y = sum, or y += sum when accumulate is set).
+// [Rc][kBatch][2][S] (slot order when n_of is given, else S = B) -> y
+// [n_part][B][kBatch] (y = sum, or y += sum when accumulate is set). Threads
+// run along the slots, so the partials are read in whole lines; each result
+// is written once, scattered.
 template <typename Real>
-__global__ void reduce_batch_kernel(const Real* __restrict__ ypart, const int* __restrict__ chunk_items, int Rc,
-                                    int B, int S, const int* __restrict__ slot, int64_t n_part,
-                                    typename Vec2<Real>::t* y, int accumulate) {
+__global__ void reduce_batch_kernel(const Real* __restrict__ ypart, const int* __restrict__ chunk_items,
+                                    int strand_len, int Rc, int B, int S, const int* __restrict__ n_of,
+                                    int64_t n_part, typename Vec2<Real>::t* y, int accumulate) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n_part * B * kBatchRhs) return;
-  const int r = (int)(j % kBatchRhs);
-  const int64_t in = j / kBatchRhs;
-  const int64_t i1 = in / B;
-  const int n1 = (int)(in - i1 * B);
-  const int k1 = slot ? slot[n1] : n1;
-  const int c = (int)(i1 / Rc), il = (int)(i1 - (int64_t)c * Rc);
+  const int64_t i1 = j / (S * kBatchRhs);
+  const int k = (int)(j - i1 * (S * kBatchRhs));
+  const int r = k / S, sl = k - r * S;
+  const int n1 = i1 >= n_part ? -1 : (n_of ? n_of[sl] : sl);
   Real re = 0, im = 0;
-  for (int w = chunk_items[c]; w < chunk_items[c + 1]; ++w) {
-    const Real* p = ypart + ((size_t)w * Rc + il) * 2 * kBatchRhs * S + (size_t)(2 * r) * S;
-    re += p[k1];
-    im += p[S + k1];
+  if (n1 >= 0) {
+    const int c = (int)(i1 / Rc), il = (int)(i1 - (int64_t)c * Rc);
+    const int w0 = chunk_items[c] + threadIdx.y * strand_len;
+    const int w1 = min(chunk_items[c + 1], w0 + strand_len);
+#pragma unroll 8
+    for (int w = w0; w < w1; ++w) {
+      const Real* p = ypart + (((size_t)w * Rc + il) * kBatchRhs + r) * 2 * S + sl;
+      re += p[0];
+      im += p[S];
+    }
   }
+  add_strands(re, im);
+  if (n1 < 0 || threadIdx.y > 0) return;
+  const int64_t o = (i1 * B + n1) * kBatchRhs + r;
   if (accumulate) {
-    re += y[j].x;
-    im += y[j].y;
+    re += y[o].x;
+    im += y[o].y;
   }
-  y[j] = typename Vec2<Real>::t{re, im};
+  y[o] = typename Vec2<Real>::t{re, im};
+}
+
+// Launch the reduction of one binning's partials.
+template <typename Real>
+inline void launch_reduce(const smh_op* op, const smh_op::Binning& bn, void* y, int accumulate, hipStream_t s) {
+  const int64_t n = op->n_part * op->B;
+  const Strands st = reduce_strands(n, bn.max_chunk_items);
+  hipLaunchKernelGGL(reduce_kernel<Real>, dim3(reduce_blocks(st, n)), reduce_block(st), 0, s,
+                     (const Real*)op->d_ypart, bn.d_chunk_items, st.len, bn.Rc, op->B, op->n_part,
+                     (typename Vec2<Real>::t*)y, accumulate);
+}
+template <typename Real>
+inline void launch_reduce_batch(const smh_op* op, const smh_op::Binning& bn, int S, const int* n_of, void* y,
+                                int accumulate, hipStream_t s) {
+  const int64_t n = op->n_part * S * kBatchRhs;
+  const Strands st = reduce_strands(n, bn.max_chunk_items);
+  hipLaunchKernelGGL(reduce_batch_kernel<Real>, dim3(reduce_blocks(st, n)), reduce_block(st), 0, s,
+                     (const Real*)op->d_ypart, bn.d_chunk_items, st.len, bn.Rc, op->B, S, n_of, op->n_part,
+                     (typename Vec2<Real>::t*)y, accumulate);
 }
 
 // Row sums of tap rows: rowsum[row] = max_n1 sum_n2 (|Re| + |Im|) of row
@@ -177,7 +252,29 @@ __global__ void item_count_kernel(const Rec* __restrict__ recs, const int4* __re
 // Largest |Re x| + |Im x| of an input, in two passes: kXmaxBlocks workgroups
 // write their maxima after xmax[0], one workgroup takes the largest (times a
 // headroom factor) into xmax[0]. The buffer holds 1 + kXmaxBlocks floats.
+// Inputs of at most kXmaxSmall entries take one workgroup and one launch (16
+// entries a thread, about the time of the second pass alone).
 constexpr int kXmaxBlocks = 256;
+constexpr int64_t kXmaxSmall = 16384;
+template <typename V2>
+__global__ void __launch_bounds__(1024) xmax_small_kernel(const V2* __restrict__ x, int n, float* xmax,
+                                                          float headroom) {
+  __shared__ float red[16];
+  float m = 0.f;
+#pragma unroll 4
+  for (int j = threadIdx.x; j < n; j += 1024) {
+    const V2 v = x[j];
+    m = fmaxf(m, (float)(fabs((double)v.x) + fabs((double)v.y)));
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int k = 1; k < 16; ++k) m = fmaxf(m, red[k]);
+    xmax[0] = m * headroom;
+  }
+}
 template <typename V2>
 __global__ void __launch_bounds__(256) xmax_part_kernel(const V2* __restrict__ x, int64_t n, float* xmax) {
   __shared__ float red[256];
@@ -204,16 +301,23 @@ __global__ void __launch_bounds__(kXmaxBlocks) xmax_final_kernel(float* xmax, fl
   }
   if (threadIdx.x == 0) xmax[0] = red[0] * headroom;
 }
+template <typename V2>
+inline void launch_xmax_scaled(const V2* x, int64_t n, float* xmax, float headroom, hipStream_t s) {
+  if (n <= kXmaxSmall) {
+    hipLaunchKernelGGL(xmax_small_kernel<V2>, dim3(1), dim3(1024), 0, s, x, (int)n, xmax, headroom);
+    return;
+  }
+  hipLaunchKernelGGL(xmax_part_kernel<V2>, dim3(kXmaxBlocks), dim3(256), 0, s, x, n, xmax);
+  hipLaunchKernelGGL(xmax_final_kernel, dim3(1), dim3(kXmaxBlocks), 0, s, xmax, headroom);
+}
 // FP32 input: the bound of the fixed-point scales.
 inline void launch_xmax(const float2* x, int64_t n, float* xmax, hipStream_t s) {
-  hipLaunchKernelGGL(xmax_part_kernel<float2>, dim3(kXmaxBlocks), dim3(256), 0, s, x, n, xmax);
-  hipLaunchKernelGGL(xmax_final_kernel, dim3(1), dim3(kXmaxBlocks), 0, s, xmax, 1.f);
+  launch_xmax_scaled(x, n, xmax, 1.f, s);
 }
 // FP64 input (the FP16-operand kernel's input is scaled by it while being
 // converted): one ulp of headroom, so the scaled inputs stay inside [-1, 1].
 inline void launch_xmax(const double2* x, int64_t n, float* xmax, hipStream_t s) {
-  hipLaunchKernelGGL(xmax_part_kernel<double2>, dim3(kXmaxBlocks), dim3(256), 0, s, x, n, xmax);
-  hipLaunchKernelGGL(xmax_final_kernel, dim3(1), dim3(kXmaxBlocks), 0, s, xmax, 1.f + 1.2e-7f);
+  launch_xmax_scaled(x, n, xmax, 1.f + 1.2e-7f, s);
 }
 
 // FP64 padded [n_part][B][kBatchRhs] -> FP64 input of the FP64 slot-order
@@ -240,9 +344,25 @@ inline void fill_zero(void* p, size_t bytes, hipStream_t s) {
 }
 
 // Work items per compute unit: items of one receiver chunk run one after the
-// other on a CU's single workgroup slot, so ~16 rounds keep the last,
-// partly filled round short. The autotuner (smh_op_autotune) may regroup.
-constexpr int kItemsPerCu = 16;
+// other on a CU's single workgroup slot, so ~16 rounds keep the last, partly
+// filled round of a large operator short. Every item also zeroes its
+// accumulator and writes it as a partial that the reduction reads back, worth
+// about kItemCost units of an entry's cost (4 us against 1.2 us for a 16-pair
+// tile, 4-8 us against 0.2-0.6 us for a pair of the kBatch-RHS kernels). With W units
+// per CU in k items each, a CU spends W + k kItemCost and waits about half an
+// item at the end: the sum is least at k = sqrt(W / (2 kItemCost)) (1023
+// spheres, l_max 2, FP64: 4 items per CU, where 16 write and read 260 MB of
+// partials). The FP64 kBatch-RHS kernel keeps small items: it adds with FP64
+// atomics in no fixed order, and where an item holds few pairs of a receiver
+// the residuals that certify a solve repeat to the last bit. The autotuner
+// (smh_op_autotune) may regroup.
+constexpr int kMaxItemsPerCu = 16;
+constexpr double kItemCost = 8.0, kItemCostBatch = 12.0;
+inline int default_items_per_cu(double cost_per_cu, bool batch, bool fp64) {
+  if (batch && fp64) return kMaxItemsPerCu;
+  const double k = std::sqrt(cost_per_cu / (2.0 * (batch ? kItemCostBatch : kItemCost)));
+  return std::max(1, std::min(kMaxItemsPerCu, (int)std::lround(k)));
+}
 
 // Launch the item statistics that depend on the grouping: the most pairs per
 // receiver (always) and the largest tap-row sum (once the table is set).
@@ -266,8 +386,8 @@ inline void set_item_lsum(smh_op::Binning& bn, const float* rowsum, int T, int v
 }
 
 // Host: group the binning's entries (h_entries, in (chunk, bin) order) into
-// work items of similar cost, about items_per_cu per compute unit and never
-// spanning two receiver chunks, and upload them with their launch order and
+// work items of similar cost, about items_per_cu per compute unit (0: the
+// default) and never spanning two receiver chunks, and upload them with their launch order and
 // statistics (replacing an earlier grouping). Cost of an entry: single-vector
 // kernels one unit per tile of 16 pairs plus 1/4 for loading the bin's taps;
 // the kBatch-RHS kernels one unit per pair plus one for the taps.
@@ -284,6 +404,7 @@ inline int group_work_items(smh_op* op, smh_op::Binning& bn, int items_per_cu, i
   const std::vector<int>& ent_chunk = bn.h_ent_chunk;
   double total = 0;
   for (const int4& e : entries) total += cost(e.z);
+  if (items_per_cu <= 0) items_per_cu = default_items_per_cu(total / ctx->num_cu, batch, bn.fp64);
   const int64_t target_items = std::max<int64_t>((int64_t)items_per_cu * ctx->num_cu, bn.n_chunks);
   const double budget = std::max(1.0, total / (double)target_items);
   // row bands: n_bands equal ranges of the entries' first tap rows
@@ -307,6 +428,8 @@ inline int group_work_items(smh_op* op, smh_op::Binning& bn, int items_per_cu, i
   }
   while (cur_chunk < bn.n_chunks) chunk_items[++cur_chunk] = (int)items.size();
   const int ni = (int)items.size();
+  bn.max_chunk_items = 0;
+  for (int c = 0; c < bn.n_chunks; ++c) bn.max_chunk_items = std::max(bn.max_chunk_items, chunk_items[c + 1] - chunk_items[c]);
   // Launch order (order_mode 1): items sorted by their first table row;
   // blocks are dealt to the XCDs round-robin (XCD = block mod kXcds), so XCD x
   // gets the x-th contiguous share of the sorted list and its CUs run items of
@@ -381,6 +504,7 @@ int build_work_items(smh_op* op, smh_op::Binning& bn, const std::vector<int>& cn
     }
   bn.n_entries = (int)bn.h_entries.size();
   bn.batch = batch;
+  bn.fp64 = std::is_same<Rec, PairRec<double>>::value || std::is_same<Rec, PairRec2<double>>::value;
   bn.count_items = [](smh_op::Binning& b, hipStream_t st) {
     hipLaunchKernelGGL(item_count_kernel<Rec>, dim3(b.n_items), dim3(256), 0, st, (const Rec*)b.d_rec, b.d_entries,
                        b.d_items, b.n_items, b.n_entries, b.d_item_en);
@@ -389,7 +513,7 @@ int build_work_items(smh_op* op, smh_op::Binning& bn, const std::vector<int>& cn
       hipMemcpyAsync(bn.d_entries, bn.h_entries.data(), bn.h_entries.size() * sizeof(int4), hipMemcpyHostToDevice,
                      s) != hipSuccess)
     return smh_fail(ctx, SMH_ERR_HIP, "device allocation failed (bin entries)");
-  return group_work_items(op, bn, kItemsPerCu, 1);
+  return group_work_items(op, bn, 0, 1);
 }
 
 }  // namespace

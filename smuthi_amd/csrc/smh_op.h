@@ -66,8 +66,9 @@ struct smh_op {
     // bands)
     std::vector<int4> h_entries;
     std::vector<int> h_ent_chunk;
-    bool batch = false;
+    bool batch = false, fp64 = false;
     int items_per_cu = 0;
+    int max_chunk_items = 0;  // most items of one chunk
     int order_mode = 1;
     void (*count_items)(Binning&, hipStream_t) = nullptr;  // item_count_kernel for the record type
     // item_lsum_kernel arguments once the table is set (rows == nullptr: not yet)

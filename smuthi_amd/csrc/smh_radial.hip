@@ -488,12 +488,14 @@ int op_reserve_packed(smh_op* op, int64_t nrhs) {
 int op_unpack(smh_op* op, int precision, const double2* pk, void* pad) {
   hipStream_t s = op->ctx->stream;
   const int64_t n_pad = op->n_part * op->B;
+  // particles below the operator's cut-offs leave padded entries that nothing writes
+  const bool holes = op->n_unk != n_pad;
   if (precision == SMH_FP32) {
-    SMH_HIP(op->ctx, hipMemsetAsync(pad, 0, n_pad * sizeof(float2), s));
+    if (holes) SMH_HIP(op->ctx, hipMemsetAsync(pad, 0, n_pad * sizeof(float2), s));
     hipLaunchKernelGGL(scatter_kernel<float>, dim3(blocks_for(op->n_unk)), dim3(256), 0, s, pk, op->d_pk2pad,
                        op->n_unk, (float2*)pad);
   } else {
-    SMH_HIP(op->ctx, hipMemsetAsync(pad, 0, n_pad * sizeof(double2), s));
+    if (holes) SMH_HIP(op->ctx, hipMemsetAsync(pad, 0, n_pad * sizeof(double2), s));
     hipLaunchKernelGGL(scatter_kernel<double>, dim3(blocks_for(op->n_unk)), dim3(256), 0, s, pk, op->d_pk2pad,
                        op->n_unk, (double2*)pad);
   }
@@ -637,13 +639,10 @@ int op_apply(smh_op* op, int precision, const void* x_pad, void* y_pad, bool tim
     SMH_HIP(ctx, hipLaunchKernel(k.fn, dim3(bn.n_items), dim3(k.threads), args, bn.lds, s));
     if (time_kernel) SMH_HIP(ctx, hipEventRecord(ctx->ev1, s));
   }
-  const int64_t n = op->n_part * op->B;
   if (pi == 0)
-    hipLaunchKernelGGL(reduce_kernel<float>, dim3(blocks_for(n)), dim3(256), 0, s, (const float*)op->d_ypart,
-                       bn.d_chunk_items, bn.Rc, op->B, op->n_part, (float2*)y_pad, 0);
+    launch_reduce<float>(op, bn, y_pad, 0, s);
   else
-    hipLaunchKernelGGL(reduce_kernel<double>, dim3(blocks_for(n)), dim3(256), 0, s, (const double*)op->d_ypart,
-                       bn.d_chunk_items, bn.Rc, op->B, op->n_part, (double2*)y_pad, 0);
+    launch_reduce<double>(op, bn, y_pad, 0, s);
   SMH_HIP(ctx, hipGetLastError());
   if (time_kernel && bn.n_items > 0) {
     SMH_HIP(ctx, hipEventSynchronize(ctx->ev1));
@@ -843,9 +842,7 @@ int op_apply_batch(smh_op* op, int precision, const void* x_pad, void* y_pad, bo
   a.row_s = op->s_mode;
   a.row_o = op->o_mode;
   if (int rc_ = op_set_lds(op, fn, bn.lds)) return rc_;
-  const int64_t nx = op->n_part * op->B * kBatch;
   const int S = slots ? k.slots : op->B;
-  const int* slot = slots ? op->d_b32_tab : nullptr;
   // (the FP16 input was scaled by the xmax its conversion wrote)
   if (pi == 0 && !half)
     launch_xmax((const float2*)x_pad, op->n_part * S * kBatch, op->d_xmax, s);
@@ -859,13 +856,11 @@ int op_apply_batch(smh_op* op, int precision, const void* x_pad, void* y_pad, bo
                                  bn.lds, s));
     if (time_kernel) SMH_HIP(ctx, hipEventRecord(ctx->ev1, s));
   }
+  const int* n_of = slots ? op->d_b32_tab + op->B : nullptr;
   if (pi == 0)
-    hipLaunchKernelGGL(reduce_batch_kernel<float>, dim3(blocks_for(nx)), dim3(256), 0, s, (const float*)op->d_ypart,
-                       bn.d_chunk_items, bn.Rc, op->B, S, slot, op->n_part, (float2*)y_pad, 0);
+    launch_reduce_batch<float>(op, bn, S, n_of, y_pad, 0, s);
   else
-    hipLaunchKernelGGL(reduce_batch_kernel<double>, dim3(blocks_for(nx)), dim3(256), 0, s,
-                       (const double*)op->d_ypart, bn.d_chunk_items, bn.Rc, op->B, S, slot, op->n_part,
-                       (double2*)y_pad, 0);
+    launch_reduce_batch<double>(op, bn, S, n_of, y_pad, 0, s);
   SMH_HIP(ctx, hipGetLastError());
   if (time_kernel && bn.n_items > 0) {
     SMH_HIP(ctx, hipEventSynchronize(ctx->ev1));
@@ -1255,26 +1250,35 @@ extern "C" int smh_op_matvec(smh_op* op, const double* x, double* y, int64_t nrh
 }
 
 namespace {
-// Sum the partials of items [k0, k1) of every receiver chunk onto y, in item
-// order (partial of item w at ypart[w - k0]); with y zero before the first
-// range, a sequence of ranges adds exactly what reduce_kernel adds at once.
+// Sum the partials of items [k0, k1) of every receiver chunk onto y (partial
+// of item w at ypart[w - k0]); with y and cur zero before the first range, a
+// sequence of ranges adds exactly what reduce_kernel adds at once: the strand
+// being summed is kept in cur and added to y when it ends (one strand, cur
+// null: straight onto y).
 template <typename Real>
-__global__ void reduce_range_kernel(const Real* __restrict__ ypart, const int* __restrict__ chunk_items, int k0, int k1,
-                                    int Rc, int B, int64_t n_part, typename Vec2<Real>::t* y) {
+__global__ void reduce_range_kernel(const Real* __restrict__ ypart, const int* __restrict__ chunk_items,
+                                    int strand_len, int k0, int k1, int Rc, int B, int64_t n_part,
+                                    typename Vec2<Real>::t* y, typename Vec2<Real>::t* cur) {
   const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n_part * B) return;
   const int64_t i1 = j / B;
   const int n1 = (int)(j - i1 * B);
   const int c = (int)(i1 / Rc), il = (int)(i1 - (int64_t)c * Rc);
-  const int w0 = max(chunk_items[c], k0), w1 = min(chunk_items[c + 1], k1);
+  const int c0 = chunk_items[c], c1 = chunk_items[c + 1];
+  const int w0 = max(c0, k0), w1 = min(c1, k1);
   if (w0 >= w1) return;
-  Real re = y[j].x, im = y[j].y;
+  typename Vec2<Real>::t* sum = cur ? cur : y;
+  Real re = sum[j].x, im = sum[j].y;
   for (int w = w0; w < w1; ++w) {
     const Real* p = ypart + ((size_t)(w - k0) * Rc + il) * 2 * B;
     re += p[n1];
     im += p[B + n1];
+    if (cur && ((w - c0 + 1) % strand_len == 0 || w + 1 == c1)) {
+      y[j] = typename Vec2<Real>::t{y[j].x + re, y[j].y + im};
+      re = im = Real(0);
+    }
   }
-  y[j] = typename Vec2<Real>::t{re, im};
+  sum[j] = typename Vec2<Real>::t{re, im};
 }
 
 // Synthetic input: n entries into whichever of x32 / x64 is given.
@@ -1393,22 +1397,27 @@ extern "C" int smh_op_matvec_noalloc(smh_op* op, const double* x, double* y, int
   // partials of as many work items as fit (launched in ranges of that size)
   const size_t rs = pi == 0 ? sizeof(float) : sizeof(double);
   const int64_t n_pad = op->n_part * op->B;
+  // (operators of several strands, at most 128k padded unknowns: and their running strand)
+  const Strands st = reduce_strands(n_pad, bn.max_chunk_items);
   const size_t head = 4096, vec = ((size_t)n_pad * 2 * rs + 255) / 256 * 256;
+  const size_t vecs = (st.count > 1 ? 3 : 2) * vec;
   const size_t per_item = (size_t)bn.Rc * 2 * op->B * rs;
-  SMH_CHECK(ctx, head + 2 * vec + per_item <= kScratchBytes, SMH_ERR_ARG,
+  SMH_CHECK(ctx, head + vecs + per_item <= kScratchBytes, SMH_ERR_ARG,
             "operator too large for the fixed scratch: %zu bytes needed (%lld padded unknowns, %zu per work item), "
             "%zu available",
-            head + 2 * vec + per_item, (long long)n_pad, per_item, kScratchBytes);
-  const int range = (int)std::min<size_t>((kScratchBytes - head - 2 * vec) / per_item, (size_t)1 << 20);
+            head + vecs + per_item, (long long)n_pad, per_item, kScratchBytes);
+  const int range = (int)std::min<size_t>((kScratchBytes - head - vecs) / per_item, (size_t)1 << 20);
   SMH_HIP(ctx, hipSetDevice(ctx->device));
   hipStream_t s = ctx->stream;
   char* base = ctx->scratch;
   float* xmax = reinterpret_cast<float*>(base);
   void* xp = base + head;
   void* yp = base + head + vec;
-  void* part = base + head + 2 * vec;
+  void* cur = st.count > 1 ? base + head + 2 * vec : nullptr;
+  void* part = base + head + vecs;
   fill_zero(xp, (size_t)n_pad * 2 * rs, s);
   fill_zero(yp, (size_t)n_pad * 2 * rs, s);
+  if (cur) fill_zero(cur, (size_t)n_pad * 2 * rs, s);
   if (pi == 0)
     hipLaunchKernelGGL(scatter_kernel<float>, dim3(blocks_for(op->n_unk)), dim3(256), 0, s, (const double2*)x,
                        op->d_pk2pad, op->n_unk, (float2*)xp);
@@ -1439,10 +1448,10 @@ extern "C" int smh_op_matvec_noalloc(smh_op* op, const double* x, double* y, int
     SMH_HIP(ctx, hipLaunchKernel(k.fn, dim3(k1 - k0), dim3(k.threads), args, bn.lds, s));
     if (pi == 0)
       hipLaunchKernelGGL(reduce_range_kernel<float>, dim3(blocks_for(n_pad)), dim3(256), 0, s, (const float*)part,
-                         bn.d_chunk_items, k0, k1, bn.Rc, op->B, op->n_part, (float2*)yp);
+                         bn.d_chunk_items, st.len, k0, k1, bn.Rc, op->B, op->n_part, (float2*)yp, (float2*)cur);
     else
       hipLaunchKernelGGL(reduce_range_kernel<double>, dim3(blocks_for(n_pad)), dim3(256), 0, s, (const double*)part,
-                         bn.d_chunk_items, k0, k1, bn.Rc, op->B, op->n_part, (double2*)yp);
+                         bn.d_chunk_items, st.len, k0, k1, bn.Rc, op->B, op->n_part, (double2*)yp, (double2*)cur);
   }
   if (pi == 0)
     hipLaunchKernelGGL(pack_kernel<float>, dim3(blocks_for(op->n_unk)), dim3(256), 0, s, (const float2*)yp,

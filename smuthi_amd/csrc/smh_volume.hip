@@ -849,13 +849,10 @@ int vol_apply(smh_op* op, int precision, const void* x_pad, void* y_pad, bool ti
       }
       // the first launch writes y, the others add to it
       const int accumulate = (t > 0 || sl > 0) ? 1 : 0;
-      const int64_t n = op->n_part * op->B;
       if (pi == 0)
-        hipLaunchKernelGGL(reduce_kernel<float>, dim3(blocks_for(n)), dim3(256), 0, s, (const float*)op->d_ypart,
-                           bn.d_chunk_items, bn.Rc, op->B, op->n_part, (float2*)y_pad, accumulate);
+        launch_reduce<float>(op, bn, y_pad, accumulate, s);
       else
-        hipLaunchKernelGGL(reduce_kernel<double>, dim3(blocks_for(n)), dim3(256), 0, s, (const double*)op->d_ypart,
-                           bn.d_chunk_items, bn.Rc, op->B, op->n_part, (double2*)y_pad, accumulate);
+        launch_reduce<double>(op, bn, y_pad, accumulate, s);
       SMH_HIP(ctx, hipGetLastError());
     }
   }
@@ -907,7 +904,6 @@ int vol_apply_batch(smh_op* op, int precision, const void* x_pad, void* y_pad, b
   }
   double ms_total = 0;
   const int n_slices = op->vmode >= 2 ? 4 : 1;
-  const int64_t nx = op->n_part * op->B * kBatchRhs;
   for (int t = 0; t < 2; ++t) {
     const smh_op::Binning& bn = op->vbbin[t][pi];
     for (int sl = 0; sl < n_slices; ++sl) {
@@ -952,13 +948,9 @@ int vol_apply_batch(smh_op* op, int precision, const void* x_pad, void* y_pad, b
       }
       const int accumulate = (t > 0 || sl > 0) ? 1 : 0;
       if (pi == 0)
-        hipLaunchKernelGGL(reduce_batch_kernel<float>, dim3(blocks_for(nx)), dim3(256), 0, s,
-                           (const float*)op->d_ypart, bn.d_chunk_items, bn.Rc, op->B, S, slot, op->n_part,
-                           (float2*)y_pad, accumulate);
+        launch_reduce_batch<float>(op, bn, S, slots ? slot + op->B : nullptr, y_pad, accumulate, s);
       else
-        hipLaunchKernelGGL(reduce_batch_kernel<double>, dim3(blocks_for(nx)), dim3(256), 0, s,
-                           (const double*)op->d_ypart, bn.d_chunk_items, bn.Rc, op->B, S, slot, op->n_part,
-                           (double2*)y_pad, accumulate);
+        launch_reduce_batch<double>(op, bn, S, slots ? slot + op->B : nullptr, y_pad, accumulate, s);
       SMH_HIP(ctx, hipGetLastError());
     }
   }
