@@ -5,20 +5,18 @@
 // classical Gram-Schmidt applied twice (CGS2) in FP64 with fused multi-dot
 // and multi-axpy kernels.
 //
-// Two drivers share the stopping rules below:
-// * one right-hand side at a time (operators without the kBatch-RHS kernels,
-//   e.g. the explicit matrix, and single right-hand sides): the small
-//   (restart+1) x restart least-squares problem is solved on the host;
-// * kBatch right-hand sides at a time over every ensemble ("segment") of the
-//   operator: every (segment, right-hand side) pair is a system of its own
-//   (its own Arnoldi scalars, Givens rotations and convergence), all systems
-//   share each coupling matvec launch, and the Givens rotations, the
-//   back-substitution and the restart bookkeeping run on the device. One
-//   Arnoldi step (matvec, CGS2, norm, rotation, normalisation) is a fixed
-//   launch sequence that is captured once per (step, precision,
-//   preconditioner) in a hipGraph and replayed; the host reads one counter
-//   of still-active systems per step. With a right block preconditioner P
-//   (op->d_P) the steps apply M P and the update is x += P V y.
+// One driver for KB = 1 right-hand side (single right-hand sides, operators
+// without the kBatch-RHS kernels) and for KB = kBatch right-hand sides at a
+// time over every ensemble ("segment") of the operator: every (segment,
+// right-hand side) pair is a system of its own (its own Arnoldi scalars, Givens
+// rotations and convergence), all systems share each coupling matvec launch,
+// and the Givens rotations, the back-substitution and the restart bookkeeping
+// run on the device. One Arnoldi step (matvec, CGS2, norm, rotation,
+// normalisation) is a fixed launch sequence that is captured once per (step,
+// precision, preconditioner) in a hipGraph and replayed; the last kernel of a
+// step writes the count of still-active systems to pinned host memory, the one
+// value the host waits for. With a right block preconditioner P (op->d_P) the
+// steps apply M P and the update is x += P V y.
 //
 // SMH_SOLVE_FP64: restarted GMRES with FP64 coupling matvecs, x0 = rhs and
 //   stopping rule ||rhs - M x|| <= tol ||rhs|| (smuthi's scipy call,
@@ -37,17 +35,16 @@
 //   digits, so tolerances near 1e-6 take two sweeps. Between sweeps the
 //   residual comes from the FP32 matvec; the FP64 residual certifies the
 //   result once that meets the tolerance.
+#include <algorithm>
 #include <chrono>
 #include <cmath>
-#include <complex>
 #include <cstdlib>
 #include <map>
+#include <set>
 
 #include "smh_op.h"
 
 namespace {
-
-typedef std::complex<double> zd;
 
 int blocks_for(int64_t n, int t = 256) { return (int)((n + t - 1) / t); }
 
@@ -59,98 +56,6 @@ constexpr double kInnerRel16 = 1e-3;  // the same for FP16-operand matvecs
 // FP32 residuals drive FP16 sweeps while above this fraction of ||b|| (about
 // 30 times the FP32 matvec's error)
 constexpr double kFp32ResidualFloor = 1e-5;
-
-// ---------------------------------------------------------------------------
-// single right-hand side
-// ---------------------------------------------------------------------------
-
-// partial[b][j] = sum over this block's slice of conj(V_j) . w
-__global__ void multi_dot_kernel(const double2* __restrict__ V, int64_t ld, int nv, const double2* __restrict__ w,
-                                 int64_t n, double2* partial) {
-  __shared__ double2 red[kDotThreads];
-  for (int j = 0; j < nv; ++j) {
-    const double2* v = V + (size_t)j * ld;
-    double re = 0, im = 0;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-      const double2 a = v[i], b = w[i];
-      re += a.x * b.x + a.y * b.y;
-      im += a.x * b.y - a.y * b.x;
-    }
-    red[threadIdx.x] = make_double2(re, im);
-    __syncthreads();
-    for (int s = blockDim.x / 2; s > 0; s >>= 1) {
-      if (threadIdx.x < s) {
-        red[threadIdx.x].x += red[threadIdx.x + s].x;
-        red[threadIdx.x].y += red[threadIdx.x + s].y;
-      }
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[(size_t)blockIdx.x * kMaxBasis + j] = red[0];
-    __syncthreads();
-  }
-}
-
-__global__ void reduce_partials_kernel(const double2* __restrict__ partial, int nblocks, int nv, double2* out) {
-  const int j = threadIdx.x;
-  if (j >= nv) return;
-  double re = 0, im = 0;
-  for (int b = 0; b < nblocks; ++b) {
-    re += partial[(size_t)b * kMaxBasis + j].x;
-    im += partial[(size_t)b * kMaxBasis + j].y;
-  }
-  out[j] = make_double2(re, im);
-}
-
-// w -= sum_j V_j c_j
-__global__ void multi_axpy_kernel(const double2* __restrict__ V, int64_t ld, int nv, const double2* __restrict__ c,
-                                  double2* w, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double2 acc = w[i];
-  for (int j = 0; j < nv; ++j) {
-    const double2 v = V[(size_t)j * ld + i], cj = c[j];
-    acc.x -= v.x * cj.x - v.y * cj.y;
-    acc.y -= v.x * cj.y + v.y * cj.x;
-  }
-  w[i] = acc;
-}
-
-// x += sum_j V_j c_j
-__global__ void multi_update_kernel(const double2* __restrict__ V, int64_t ld, int nv, const double2* __restrict__ c,
-                                    double2* x, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  double2 acc = x[i];
-  for (int j = 0; j < nv; ++j) {
-    const double2 v = V[(size_t)j * ld + i], cj = c[j];
-    acc.x += v.x * cj.x - v.y * cj.y;
-    acc.y += v.x * cj.y + v.y * cj.x;
-  }
-  x[i] = acc;
-}
-
-__global__ void scale_copy_kernel(const double2* __restrict__ src, double s, double2* dst, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = make_double2(src[i].x * s, src[i].y * s);
-}
-
-// out = v - t o y  (master matrix 1 - T W applied after the coupling matvec)
-__global__ void master_fp64_kernel(const double2* __restrict__ v, const double2* __restrict__ t,
-                                   const double2* __restrict__ y, double2* out, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double2 a = t[i], b = y[i];
-  out[i] = make_double2(v[i].x - (a.x * b.x - a.y * b.y), v[i].y - (a.x * b.y + a.y * b.x));
-}
-
-__global__ void master_fp32_kernel(const double2* __restrict__ v, const double2* __restrict__ t,
-                                   const float2* __restrict__ y, double2* out, int64_t n) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double2 a = t[i];
-  const double bx = y[i].x, by = y[i].y;
-  out[i] = make_double2(v[i].x - (a.x * bx - a.y * by), v[i].y - (a.x * by + a.y * bx));
-}
 
 __global__ void to_fp32_kernel(const double2* __restrict__ v, float2* out, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -181,15 +86,16 @@ __global__ void zero_f2_kernel(float2* p, int64_t n) {
 }
 
 // ---------------------------------------------------------------------------
-// kBatch right-hand sides x segments: element e = (particle * B + n) * kB + r
-// of a padded vector; system sys = segment(particle) * kB + r
+// KB right-hand sides x segments: element e = (particle * B + n) * KB + r of a
+// padded vector; system sys = segment(particle) * KB + r
 // ---------------------------------------------------------------------------
 constexpr int kB = smh::kBatchRhs;
 
-// partial[((s * nblk + b) * kMaxBasis + j) * kB + r]: block b's share of
+// partial[((s * nblk + b) * kMaxBasis + j) * KB + r]: block b's share of
 // conj(V_j) . w over segment s and right-hand side r (grid: nblk x n_seg; a
-// thread sees one r, since segments start at multiples of kB elements and
-// the block stride is a multiple of kB)
+// thread sees one r, since segments start at multiples of KB elements and
+// the block stride is a multiple of KB)
+template <int KB>
 __global__ void __launch_bounds__(kDotThreads) sdot_kernel(const double2* __restrict__ V, int64_t ld, int nv,
                                                            const double2* __restrict__ w, int64_t per_part,
                                                            const int64_t* __restrict__ seg_off, double2* partial) {
@@ -206,28 +112,29 @@ __global__ void __launch_bounds__(kDotThreads) sdot_kernel(const double2* __rest
     }
     red[threadIdx.x] = make_double2(re, im);
     __syncthreads();
-    for (int st = blockDim.x / 2; st >= kB; st >>= 1) {  // strides keep e % kB
+    for (int st = blockDim.x / 2; st >= KB; st >>= 1) {  // strides keep e % KB
       if ((int)threadIdx.x < st) {
         red[threadIdx.x].x += red[threadIdx.x + st].x;
         red[threadIdx.x].y += red[threadIdx.x + st].y;
       }
       __syncthreads();
     }
-    if ((int)threadIdx.x < kB)
-      partial[(((size_t)s * nblk + b) * kMaxBasis + j) * kB + threadIdx.x] = red[threadIdx.x];
+    if ((int)threadIdx.x < KB)
+      partial[(((size_t)s * nblk + b) * kMaxBasis + j) * KB + threadIdx.x] = red[threadIdx.x];
     __syncthreads();
   }
 }
 
-// out[(s * kB + r) * ldo + j] = sum over the nblk partials, fixed-order tree;
+// out[(s * KB + r) * ldo + j] = sum over the nblk partials, fixed-order tree;
 // one workgroup per (j, r) and segment
+template <int KB>
 __global__ void __launch_bounds__(256) sreduce_kernel(const double2* __restrict__ partial, int nblk, double2* out,
                                                       int ldo) {
-  const int j = blockIdx.x / kB, r = blockIdx.x % kB, s = blockIdx.y;
+  const int j = blockIdx.x / KB, r = blockIdx.x % KB, s = blockIdx.y;
   __shared__ double2 red[256];
   double re = 0, im = 0;
   for (int b = threadIdx.x; b < nblk; b += blockDim.x) {
-    const double2 p = partial[(((size_t)s * nblk + b) * kMaxBasis + j) * kB + r];
+    const double2 p = partial[(((size_t)s * nblk + b) * kMaxBasis + j) * KB + r];
     re += p.x;
     im += p.y;
   }
@@ -240,21 +147,23 @@ __global__ void __launch_bounds__(256) sreduce_kernel(const double2* __restrict_
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[((size_t)s * kB + r) * ldo + j] = red[0];
+  if (threadIdx.x == 0) out[((size_t)s * KB + r) * ldo + j] = red[0];
 }
 
+template <int KB>
 __device__ inline int sys_of(int64_t e, int64_t per_part, const int* __restrict__ seg_of) {
-  const int r = (int)(e % kB);
-  return (seg_of ? seg_of[e / per_part] : 0) * kB + r;
+  const int r = (int)(e % KB);
+  return (seg_of ? seg_of[e / per_part] : 0) * KB + r;
 }
 
 // w[e] += sgn * sum_j V_j[e] c[sys(e) * ldc + j]
+template <int KB>
 __global__ void saxpy_kernel(const double2* __restrict__ V, int64_t ld, int nv, const double2* __restrict__ c,
                              int ldc, double sgn, double2* w, int64_t n8, int64_t per_part,
                              const int* __restrict__ seg_of) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n8) return;
-  const double2* cs = c + (size_t)sys_of(e, per_part, seg_of) * ldc;
+  const double2* cs = c + (size_t)sys_of<KB>(e, per_part, seg_of) * ldc;
   double2 acc = w[e];
   for (int j = 0; j < nv; ++j) {
     const double2 v = V[(size_t)j * ld + e], cj = cs[j];
@@ -264,20 +173,27 @@ __global__ void saxpy_kernel(const double2* __restrict__ V, int64_t ld, int nv, 
   w[e] = acc;
 }
 
+// dst = src sc[sys]; with `live` the launch also hands the host that count
+// (pinned memory; the kernel that wrote it has ended)
+template <int KB>
 __global__ void sscale_kernel(const double2* __restrict__ src, const double* __restrict__ sc, double2* dst,
-                              int64_t n8, int64_t per_part, const int* __restrict__ seg_of) {
+                              int64_t n8, int64_t per_part, const int* __restrict__ seg_of, const int* live,
+                              int* host_live) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (live && e == 0) *host_live = *live;
   if (e >= n8) return;
-  const double f = sc[sys_of(e, per_part, seg_of)];
+  const double f = sc[sys_of<KB>(e, per_part, seg_of)];
   dst[e] = make_double2(src[e].x * f, src[e].y * f);
 }
 
-// out = v - t o y with t per unknown, shared by the right-hand sides
+// out = v - t o y with t per unknown, shared by the right-hand sides (master
+// matrix 1 - T W applied after the coupling matvec)
+template <int KB>
 __global__ void bmaster_fp64_kernel(const double2* __restrict__ v, const double2* __restrict__ t,
                                     const double2* __restrict__ y, double2* out, int64_t n8) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n8) return;
-  const double2 a = t[e / kB], b = y[e];
+  const double2 a = t[e / KB], b = y[e];
   out[e] = make_double2(v[e].x - (a.x * b.x - a.y * b.y), v[e].y - (a.x * b.y + a.y * b.x));
 }
 
@@ -291,11 +207,12 @@ __global__ void to_fp32_b32_kernel(const double2* __restrict__ v, float2* out, i
   out[smh::b32_index(p, (int)(ip - p * B), r, S, slot)] = make_float2((float)v[e].x, (float)v[e].y);
 }
 
+template <int KB>
 __global__ void bmaster_fp32_kernel(const double2* __restrict__ v, const double2* __restrict__ t,
                                     const float2* __restrict__ y, double2* out, int64_t n8) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n8) return;
-  const double2 a = t[e / kB];
+  const double2 a = t[e / KB];
   const double bx = y[e].x, by = y[e].y;
   out[e] = make_double2(v[e].x - (a.x * bx - a.y * by), v[e].y - (a.x * by + a.y * bx));
 }
@@ -327,40 +244,22 @@ __global__ void cycle_init_kernel(const double2* __restrict__ nrm, const double*
   if (c) atomicAdd(&nlive[restart], 1);
 }
 
-// Arnoldi step k of every live system (one thread per system): the new
-// Hessenberg column h1 + h2 (the two CGS passes) with h_{k+1,k} = ||w||, the
-// previous Givens rotations applied to it, a new rotation zeroing h_{k+1,k},
-// the rotated right-hand side g and the normalisation of w. A system stops
-// when its least-squares residual |g_{k+1}| reaches atol; nlive[k] counts the
-// systems still running after this step.
-__global__ void givens_kernel(int k, const double2* __restrict__ h1, const double2* __restrict__ h2, int ldh,
-                              const double2* __restrict__ hn2, const double* __restrict__ atol, int nsys, int restart,
-                              int* live, double2* H, double2* cs, double2* sn, double2* g, int* kr, double* scale,
-                              int* nlive) {
-  const int sys = blockIdx.x * blockDim.x + threadIdx.x;
-  if (sys >= nsys) return;
-  if (!live[sys]) {
-    scale[sys] = 0.0;
-    return;
-  }
-  const double hn = sqrt(fmax(0.0, hn2[sys].x));
-  double2* Hs = H + (size_t)sys * (restart + 1) * restart;  // H[j][k] at Hs[j * restart + k]
-  double2* css = cs + (size_t)sys * restart;
-  double2* sns = sn + (size_t)sys * restart;
-  double2* gs = g + (size_t)sys * (restart + 1);
-  for (int j = 0; j <= k; ++j) {
-    const double2 a = h1[(size_t)sys * ldh + j], b = h2[(size_t)sys * ldh + j];
-    Hs[(size_t)j * restart + k] = make_double2(a.x + b.x, a.y + b.y);
-  }
+// Arnoldi step k of one live system: the new Hessenberg column col[0..k] (the
+// sum of the two CGS passes) with h_{k+1,k} = hn = ||w||, the previous Givens
+// rotations applied to it, a new rotation zeroing h_{k+1,k} and the rotated
+// right-hand side g. Returns whether the system goes on: it stops when its
+// least-squares residual |g_{k+1}| reaches atol.
+__device__ inline bool givens_step(int k, double2* col, double hn, double atol, int restart, double2* Hs,
+                                   double2* css, double2* sns, double2* gs) {
+  double2 a = col[0];
   for (int j = 0; j < k; ++j) {
-    const double2 a = Hs[(size_t)j * restart + k], b = Hs[(size_t)(j + 1) * restart + k];
+    const double2 b = col[j + 1];
     const double2 c = css[j], s = sns[j];
     const double2 u = cmul2(cconj2(c), a), v = cmul2(cconj2(s), b);
     const double2 p = cmul2(s, a), q = cmul2(c, b);
     Hs[(size_t)j * restart + k] = make_double2(u.x + v.x, u.y + v.y);
-    Hs[(size_t)(j + 1) * restart + k] = make_double2(q.x - p.x, q.y - p.y);
+    a = make_double2(q.x - p.x, q.y - p.y);
   }
-  const double2 a = Hs[(size_t)k * restart + k];
   const double den = sqrt(a.x * a.x + a.y * a.y + hn * hn);
   const double2 c = den > 0 ? make_double2(a.x / den, a.y / den) : make_double2(1.0, 0.0);
   const double2 s = den > 0 ? make_double2(hn / den, 0.0) : make_double2(0.0, 0.0);
@@ -372,13 +271,151 @@ __global__ void givens_kernel(int k, const double2* __restrict__ h1, const doubl
   gs[k] = cmul2(cconj2(c), gk);
   css[k] = c;
   sns[k] = s;
+  const double gr = sqrt(gn.x * gn.x + gn.y * gn.y);
+  return !(gr <= atol || hn == 0.0);
+}
+
+// The step's rotations (one thread per system) and the normalisation of w;
+// nlive[k] counts the systems still running after this step.
+__global__ void givens_kernel(int k, double2* h1, const double2* __restrict__ h2, int ldh,
+                              const double2* __restrict__ hn2, const double* __restrict__ atol, int nsys, int restart,
+                              int* live, double2* H, double2* cs, double2* sn, double2* g, int* kr, double* scale,
+                              int* nlive) {
+  const int sys = blockIdx.x * blockDim.x + threadIdx.x;
+  if (sys >= nsys) return;
+  if (!live[sys]) {
+    scale[sys] = 0.0;
+    return;
+  }
+  const double hn = sqrt(fmax(0.0, hn2[sys].x));
+  double2* col = h1 + (size_t)sys * ldh;
+  for (int j = 0; j <= k; ++j) {
+    const double2 a = col[j], b = h2[(size_t)sys * ldh + j];
+    col[j] = make_double2(a.x + b.x, a.y + b.y);
+  }
+  const bool on = givens_step(k, col, hn, atol[sys], restart, H + (size_t)sys * (restart + 1) * restart,
+                              cs + (size_t)sys * restart, sn + (size_t)sys * restart, g + (size_t)sys * (restart + 1));
   kr[sys] = k + 1;
   scale[sys] = hn > 0 ? 1.0 / hn : 0.0;
-  const double gr = sqrt(gs[k + 1].x * gs[k + 1].x + gs[k + 1].y * gs[k + 1].y);
-  if (gr <= atol[sys] || hn == 0.0)
+  if (!on)
     live[sys] = 0;
   else
     atomicAdd(&nlive[k], 1);
+}
+
+// Everything of an Arnoldi step that follows the matvec, for one system whose
+// vector fits a workgroup's registers (kSmallVector entries): CGS2 against
+// V_0..V_k, the norm, the rotations and V_{k+1}. Bound by the latency of its
+// dependent passes over V from L2 (1500 unknowns, k = 8: about 10 us); the
+// launches it replaces (two dots, two reductions, two updates, norm, rotation,
+// scaling) took 35 us of a step at that size, and spread over more workgroups
+// they are the faster ones above it.
+constexpr int kSmallThreads = 1024, kSmallPer = 4, kSmallVector = kSmallThreads * kSmallPer;
+__global__ void __launch_bounds__(kSmallThreads)
+    arnoldi_small_kernel(int k, double2* V, const double2* __restrict__ wv, int n, const double* __restrict__ atol,
+                         int restart, int* live, double2* H, double2* cs, double2* sn, double2* g, int* kr,
+                         int* nlive, int* host_live) {
+  __shared__ double2 red[kSmallThreads / 64][kMaxBasis + 1];
+  __shared__ double2 h[kMaxBasis + 1], col[kMaxBasis + 1], css[kMaxBasis], sns[kMaxBasis];
+  __shared__ double scale;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  double2 w[kSmallPer];
+#pragma unroll
+  for (int u = 0; u < kSmallPer; ++u) {
+    const int e = u * kSmallThreads + tid;
+    w[u] = e < n ? wv[e] : make_double2(0.0, 0.0);
+  }
+  if (tid < k) {
+    css[tid] = cs[tid];
+    sns[tid] = sn[tid];
+  }
+  // sum of (re, im) over the wave into red[wave][j]
+  auto wave_sum = [&](int j, double re, double im) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      re += __shfl_xor(re, off);
+      im += __shfl_xor(im, off);
+    }
+    if (lane == 0) red[wave][j] = make_double2(re, im);
+  };
+  auto block_sum = [&](int nv) {
+    __syncthreads();
+    if (tid < nv) {
+      double2 s = red[0][tid];
+      for (int q = 1; q < kSmallThreads / 64; ++q) {
+        s.x += red[q][tid].x;
+        s.y += red[q][tid].y;
+      }
+      h[tid] = s;
+    }
+    __syncthreads();
+  };
+  for (int pass = 0; pass < 2; ++pass) {
+#pragma unroll 2
+    for (int j = 0; j <= k; ++j) {
+      double re = 0, im = 0;
+#pragma unroll
+      for (int u = 0; u < kSmallPer; ++u) {
+        const int e = u * kSmallThreads + tid;
+        if (e < n) {
+          const double2 a = V[(size_t)j * n + e];
+          re += a.x * w[u].x + a.y * w[u].y;
+          im += a.x * w[u].y - a.y * w[u].x;
+        }
+      }
+      wave_sum(j, re, im);
+    }
+    block_sum(k + 1);
+    if (tid <= k) {
+      if (pass == 0)
+        col[tid] = h[tid];
+      else
+        col[tid] = make_double2(col[tid].x + h[tid].x, col[tid].y + h[tid].y);
+    }
+#pragma unroll 4
+    for (int j = 0; j <= k; ++j) {
+      const double2 c = h[j];
+#pragma unroll
+      for (int u = 0; u < kSmallPer; ++u) {
+        const int e = u * kSmallThreads + tid;
+        if (e < n) {
+          const double2 v = V[(size_t)j * n + e];
+          w[u].x -= v.x * c.x - v.y * c.y;
+          w[u].y -= v.x * c.y + v.y * c.x;
+        }
+      }
+    }
+    __syncthreads();  // h is read by all before the next sums
+  }
+  double nn = 0;
+#pragma unroll
+  for (int u = 0; u < kSmallPer; ++u) nn += w[u].x * w[u].x + w[u].y * w[u].y;
+  wave_sum(0, nn, 0.0);
+  block_sum(1);
+  if (tid == 0) {
+    double f = 0.0;
+    if (live[0]) {
+      const double hn = sqrt(fmax(0.0, h[0].x));
+      const bool on = givens_step(k, col, hn, atol[0], restart, H, css, sns, g);
+      cs[k] = css[k];
+      sn[k] = sns[k];
+      kr[0] = k + 1;
+      f = hn > 0 ? 1.0 / hn : 0.0;
+      if (!on) live[0] = 0;
+      nlive[k] = on ? 1 : 0;
+      *host_live = on ? 1 : 0;
+    } else {
+      *host_live = nlive[k];
+    }
+    scale = f;
+  }
+  __syncthreads();
+  const double f = scale;
+#pragma unroll
+  for (int u = 0; u < kSmallPer; ++u) {
+    const int e = u * kSmallThreads + tid;
+    if (e < n) V[(size_t)(k + 1) * n + e] = make_double2(w[u].x * f, w[u].y * f);
+  }
 }
 
 // End of a cycle (one thread per system): y = R^{-1} g over the system's
@@ -448,14 +485,8 @@ __global__ void __launch_bounds__(256) precond_kernel(const double2* __restrict_
 }
 
 // ---- per-operator workspace ------------------------------------------------
-struct Ws {
-  // single right-hand side
-  int64_t n1 = 0;
-  int restart1 = 0;
-  double2 *V1 = nullptr, *w1 = nullptr, *t1 = nullptr, *partial1 = nullptr, *coef1 = nullptr, *y1 = nullptr;
-  double2 *b1 = nullptr, *x1 = nullptr, *d1 = nullptr, *r1 = nullptr;
-  float2* x32_1 = nullptr;
-  // batched systems
+// One set of vectors and scalars per KB (single and batched systems).
+struct SolveWs {
   int64_t n8 = 0;
   int restart = 0, nsys = 0, nblk = 0;
   double2 *V = nullptr, *w = nullptr, *t = nullptr, *partial = nullptr, *h1 = nullptr, *h2 = nullptr,
@@ -465,42 +496,34 @@ struct Ws {
   int *live = nullptr, *kr = nullptr, *nlive = nullptr, *active = nullptr;
   float2 *x32 = nullptr, *y32 = nullptr;
   void* x16 = nullptr;
-  int* h_pin = nullptr;  // pinned host word: the live-system count of the last step
+  // pinned host memory: the live-system count of the last step, and the
+  // systems' norms or residuals
+  int* h_live = nullptr;
+  double2* h_val = nullptr;
   std::map<int, hipGraphExec_t> graphs;
-  bool warmed[3][2] = {};
+  std::set<int> ran;  // steps that have run since the graphs were dropped
 
-  void free_single() {
-    void* p[] = {V1, w1, t1, partial1, coef1, y1, b1, x1, d1, r1, x32_1};
-    for (void* q : p)
-      if (q) (void)hipFree(q);
-    V1 = w1 = t1 = partial1 = coef1 = y1 = b1 = x1 = d1 = r1 = nullptr;
-    x32_1 = nullptr;
-    n1 = 0;
-    restart1 = 0;
-  }
   void drop_graphs() {
     for (auto& kv : graphs) (void)hipGraphExecDestroy(kv.second);
     graphs.clear();
-    for (auto& w3 : warmed) w3[0] = w3[1] = false;
+    ran.clear();
   }
-  void free_batch() {
+  void release() {
     drop_graphs();
     void* p[] = {V, w, t, partial, h1, h2, hn, H, cs, sn, g, yv, y64, b, x, d, r, pv, tmp,
                  atol, scale, res, live, kr, nlive, active, x32, y32, x16};
     for (void* q : p)
       if (q) (void)hipFree(q);
-    V = w = t = partial = h1 = h2 = hn = H = cs = sn = g = yv = y64 = b = x = d = r = pv = tmp = nullptr;
-    atol = scale = res = nullptr;
-    live = kr = nlive = active = nullptr;
-    x32 = y32 = nullptr;
-    x16 = nullptr;
-    n8 = 0;
-    restart = nsys = nblk = 0;
+    if (h_live) (void)hipHostFree(h_live);
+    if (h_val) (void)hipHostFree(h_val);
+    *this = SolveWs();
   }
+};
+struct Ws {
+  SolveWs one, batch;
   ~Ws() {
-    free_single();
-    free_batch();
-    if (h_pin) (void)hipHostFree(h_pin);
+    one.release();
+    batch.release();
   }
 };
 
@@ -515,186 +538,36 @@ bool graphs_enabled() {
   return !(e && e[0] == '0');
 }
 
-// Single right-hand side GMRES (host least squares).
+// KB right-hand sides x n_seg segments in lockstep, device-side Givens.
+template <int KB>
 struct Solver {
   smh_op* op;
   smh_ctx* ctx;
   hipStream_t s;
-  Ws* ws;
-  int64_t n;  // padded length
-  int restart;
-  int64_t mv64 = 0, mv32 = 0, iters = 0;
-
-  int init() {
-    if (ws->n1 == n && ws->restart1 >= restart) return SMH_OK;
-    ws->free_single();
-    auto alloc = [&](void** p, size_t bytes) { return hipMalloc(p, bytes) == hipSuccess; };
-    const bool ok = alloc((void**)&ws->V1, (size_t)(restart + 1) * n * sizeof(double2)) &&
-                    alloc((void**)&ws->w1, n * sizeof(double2)) && alloc((void**)&ws->t1, n * sizeof(double2)) &&
-                    alloc((void**)&ws->partial1, (size_t)kDotBlocks * kMaxBasis * sizeof(double2)) &&
-                    alloc((void**)&ws->coef1, kMaxBasis * sizeof(double2)) &&
-                    alloc((void**)&ws->y1, n * sizeof(double2)) && alloc((void**)&ws->b1, n * sizeof(double2)) &&
-                    alloc((void**)&ws->x1, n * sizeof(double2)) && alloc((void**)&ws->d1, n * sizeof(double2)) &&
-                    alloc((void**)&ws->r1, n * sizeof(double2)) && alloc((void**)&ws->x32_1, n * sizeof(float2));
-    if (!ok) {
-      ws->free_single();
-      return smh_fail(ctx, SMH_ERR_HIP, "solver allocation failed (%lld unknowns, restart %d)", (long long)n, restart);
-    }
-    ws->n1 = n;
-    ws->restart1 = restart;
-    return SMH_OK;
-  }
-
-  // out = M v (padded), precision of the coupling matvec as requested
-  int master(const double2* v, double2* out, int precision) {
-    int rc;
-    if (precision == SMH_FP64) {
-      if ((rc = smh::op_apply(op, SMH_FP64, v, ws->y1, false))) return rc;
-      hipLaunchKernelGGL(master_fp64_kernel, dim3(blocks_for(n)), dim3(256), 0, s, v, ws->t1, ws->y1, out, n);
-      ++mv64;
-    } else {
-      hipLaunchKernelGGL(to_fp32_kernel, dim3(blocks_for(n)), dim3(256), 0, s, v, ws->x32_1, n);
-      if ((rc = smh::op_apply(op, SMH_FP32, ws->x32_1, op->d_y32, false))) return rc;
-      hipLaunchKernelGGL(master_fp32_kernel, dim3(blocks_for(n)), dim3(256), 0, s, v, ws->t1, op->d_y32, out, n);
-      ++mv32;
-    }
-    SMH_HIP(ctx, hipGetLastError());
-    return SMH_OK;
-  }
-
-  // h[0..nv) = V[0..nv)^H w (device -> host)
-  int dots(const double2* Vb, int nv, const double2* wv, zd* h) {
-    if (nv < 1 || nv > kMaxBasis) return smh_fail(ctx, SMH_ERR_ARG, "basis size out of range");
-    hipLaunchKernelGGL(multi_dot_kernel, dim3(kDotBlocks), dim3(kDotThreads), 0, s, Vb, n, nv, wv, n, ws->partial1);
-    hipLaunchKernelGGL(reduce_partials_kernel, dim3(1), dim3(kMaxBasis), 0, s, ws->partial1, kDotBlocks, nv,
-                       ws->coef1);
-    SMH_HIP(ctx, hipMemcpyAsync(h, ws->coef1, nv * sizeof(double2), hipMemcpyDeviceToHost, s));
-    SMH_HIP(ctx, hipStreamSynchronize(s));
-    return SMH_OK;
-  }
-  int norm(const double2* v, double& out) {
-    zd h;
-    int rc = dots(v, 1, v, &h);
-    out = std::sqrt(std::max(0.0, h.real()));
-    return rc;
-  }
-
-  // Restarted GMRES on M x = b from x (in/out), stops at ||b - M x|| <= atol.
-  // x_zero: x is zero on entry, so the first residual is b itself.
-  // trust_estimate (inner solves of the refinement): one restart cycle at
-  // most, returning as soon as the Arnoldi residual estimate reaches atol or
-  // the cycle ends, without recomputing the true residual (the caller takes
-  // it in FP64 and starts the next sweep: a reduced-precision operator whose
-  // error sits above atol would otherwise stall the restarts).
-  // On return res_out is the true residual of x (or the estimate, see above)
-  // and steps the number of Arnoldi steps taken.
-  int gmres(double2* x, const double2* b, double atol, int maxiter, int precision, double& res_out, int& steps,
-            bool x_zero = false, bool trust_estimate = false) {
-    std::vector<zd> H((size_t)(restart + 1) * restart), cs(restart), sn(restart), g(restart + 1), hcol(restart + 1),
-        hcol2(restart + 1), yv(restart);
-    double2* V = ws->V1;
-    double2* w = ws->w1;
-    int rc;
-    steps = 0;
-    double beta = 0;
-    for (int outer = 0;; ++outer) {
-      // r = b - M x -> V_0
-      if (outer == 0 && x_zero) {
-        SMH_HIP(ctx, hipMemcpyAsync(w, b, n * sizeof(double2), hipMemcpyDeviceToDevice, s));
-      } else {
-        if ((rc = master(x, w, precision))) return rc;
-        hipLaunchKernelGGL(sub_kernel, dim3(blocks_for(n)), dim3(256), 0, s, b, w, w, n);
-      }
-      if ((rc = norm(w, beta))) return rc;
-      res_out = beta;
-      if (beta <= atol || steps >= maxiter || beta == 0.0) return SMH_OK;
-      hipLaunchKernelGGL(scale_copy_kernel, dim3(blocks_for(n)), dim3(256), 0, s, w, 1.0 / beta, V, n);
-      std::fill(g.begin(), g.end(), zd(0));
-      g[0] = beta;
-      int k = 0;
-      for (; k < restart && steps < maxiter; ++k, ++steps) {
-        double2* vk = V + (size_t)k * n;
-        if ((rc = master(vk, w, precision))) return rc;
-        // CGS2 against V_0..V_k
-        if ((rc = dots(V, k + 1, w, hcol.data()))) return rc;
-        SMH_HIP(ctx, hipMemcpyAsync(ws->coef1, hcol.data(), (k + 1) * sizeof(double2), hipMemcpyHostToDevice, s));
-        hipLaunchKernelGGL(multi_axpy_kernel, dim3(blocks_for(n)), dim3(256), 0, s, V, n, k + 1, ws->coef1, w, n);
-        if ((rc = dots(V, k + 1, w, hcol2.data()))) return rc;
-        SMH_HIP(ctx, hipMemcpyAsync(ws->coef1, hcol2.data(), (k + 1) * sizeof(double2), hipMemcpyHostToDevice, s));
-        hipLaunchKernelGGL(multi_axpy_kernel, dim3(blocks_for(n)), dim3(256), 0, s, V, n, k + 1, ws->coef1, w, n);
-        for (int j = 0; j <= k; ++j) hcol[j] += hcol2[j];
-        double hn;
-        if ((rc = norm(w, hn))) return rc;
-        hcol[k + 1] = hn;
-        if (hn > 0)
-          hipLaunchKernelGGL(scale_copy_kernel, dim3(blocks_for(n)), dim3(256), 0, s, w, 1.0 / hn,
-                             V + (size_t)(k + 1) * n, n);
-        // Givens rotations on the new column
-        for (int j = 0; j < k; ++j) {
-          const zd a = hcol[j], bb = hcol[j + 1];
-          hcol[j] = std::conj(cs[j]) * a + std::conj(sn[j]) * bb;
-          hcol[j + 1] = -sn[j] * a + cs[j] * bb;
-        }
-        const zd a = hcol[k], bb = hcol[k + 1];
-        const double den = std::sqrt(std::norm(a) + std::norm(bb));
-        cs[k] = den > 0 ? a / den : zd(1);
-        sn[k] = den > 0 ? bb / den : zd(0);
-        hcol[k] = std::conj(cs[k]) * a + std::conj(sn[k]) * bb;
-        hcol[k + 1] = 0;
-        g[k + 1] = -sn[k] * g[k];
-        g[k] = std::conj(cs[k]) * g[k];
-        for (int j = 0; j <= k; ++j) H[(size_t)j * restart + k] = hcol[j];
-        ++iters;
-        if (std::abs(g[k + 1]) <= atol || hn == 0.0) {
-          ++k;
-          ++steps;
-          break;
-        }
-      }
-      // back substitution and update x += V y
-      for (int i = k - 1; i >= 0; --i) {
-        zd sum = g[i];
-        for (int j = i + 1; j < k; ++j) sum -= H[(size_t)i * restart + j] * yv[j];
-        yv[i] = sum / H[(size_t)i * restart + i];
-      }
-      if (k > 0) {
-        SMH_HIP(ctx, hipMemcpyAsync(ws->coef1, yv.data(), k * sizeof(double2), hipMemcpyHostToDevice, s));
-        hipLaunchKernelGGL(multi_update_kernel, dim3(blocks_for(n)), dim3(256), 0, s, V, n, k, ws->coef1, x, n);
-      }
-      if (trust_estimate) {
-        res_out = std::abs(g[k]);
-        return SMH_OK;
-      }
-    }
-  }
-};
-
-// kBatch right-hand sides x n_seg segments in lockstep, device-side Givens.
-struct BatchSolver {
-  smh_op* op;
-  smh_ctx* ctx;
-  hipStream_t s;
-  Ws* ws;
-  int64_t n, n8, per_part;  // padded length, times kB, elements per particle
+  SolveWs* ws;
+  int64_t n, n8, per_part;  // padded length, times KB, elements per particle
   int restart, nsys, nblk;
-  bool use_P;
+  bool use_P, small;
   int64_t mv64 = 0, mv32 = 0, mv16 = 0, iters = 0;
 
   int init() {
-    nsys = op->n_seg * kB;
-    nblk = std::max(8, std::min(kDotBlocks, kDotBlocks / op->n_seg));
+    nsys = op->n_seg * KB;
+    // dot partials: about 1024 entries of the largest segment per block, the chip filled at most twice
+    int64_t most = 0;
+    for (int q = 0; q < op->n_seg; ++q) most = std::max(most, (op->seg_off[q + 1] - op->seg_off[q]) * per_part);
+    nblk = (int)std::max<int64_t>(1, std::min<int64_t>((most + 1023) / 1024, std::max(8, kDotBlocks / op->n_seg)));
     use_P = op->d_P != nullptr;
-    if (!ws->h_pin) SMH_HIP(ctx, hipHostMalloc((void**)&ws->h_pin, 4 * sizeof(int), hipHostMallocDefault));
+    small = KB == 1 && op->n_seg == 1 && n8 <= kSmallVector;
     if (ws->n8 == n8 && ws->restart == restart && ws->nsys == nsys && ws->nblk == nblk) return SMH_OK;
-    ws->free_batch();
-    const size_t n32 = (size_t)op->n_part * op->b32_S * kB;
-    const bool half = smh::op_has_batch(op, SMH_FP16);
+    ws->release();
+    const size_t n32 = KB == 1 ? (size_t)n : (size_t)op->n_part * op->b32_S * KB;
+    const bool half = KB > 1 && smh::op_has_batch(op, SMH_FP16);
     const int ldh = restart + 1;
     auto alloc = [&](void** p, size_t bytes) { return hipMalloc(p, std::max<size_t>(bytes, 16)) == hipSuccess; };
     const bool ok =
         alloc((void**)&ws->V, (size_t)(restart + 1) * n8 * sizeof(double2)) &&
         alloc((void**)&ws->w, n8 * sizeof(double2)) && alloc((void**)&ws->t, n * sizeof(double2)) &&
-        alloc((void**)&ws->partial, (size_t)op->n_seg * nblk * kMaxBasis * kB * sizeof(double2)) &&
+        alloc((void**)&ws->partial, (size_t)op->n_seg * nblk * kMaxBasis * KB * sizeof(double2)) &&
         alloc((void**)&ws->h1, (size_t)nsys * ldh * sizeof(double2)) &&
         alloc((void**)&ws->h2, (size_t)nsys * ldh * sizeof(double2)) &&
         alloc((void**)&ws->hn, (size_t)nsys * sizeof(double2)) &&
@@ -705,17 +578,19 @@ struct BatchSolver {
         alloc((void**)&ws->yv, (size_t)nsys * ldh * sizeof(double2)) &&
         alloc((void**)&ws->y64, n8 * sizeof(double2)) && alloc((void**)&ws->b, n8 * sizeof(double2)) &&
         alloc((void**)&ws->x, n8 * sizeof(double2)) && alloc((void**)&ws->d, n8 * sizeof(double2)) &&
-        alloc((void**)&ws->r, n8 * sizeof(double2)) && alloc((void**)&ws->pv, n8 * sizeof(double2)) &&
-        alloc((void**)&ws->tmp, n8 * sizeof(double2)) && alloc((void**)&ws->atol, nsys * sizeof(double)) &&
+        alloc((void**)&ws->r, n8 * sizeof(double2)) &&
+        (KB == 1 || (alloc((void**)&ws->pv, n8 * sizeof(double2)) && alloc((void**)&ws->tmp, n8 * sizeof(double2)))) &&
+        alloc((void**)&ws->atol, nsys * sizeof(double)) &&
         alloc((void**)&ws->scale, nsys * sizeof(double)) && alloc((void**)&ws->res, nsys * sizeof(double)) &&
         alloc((void**)&ws->live, nsys * sizeof(int)) && alloc((void**)&ws->kr, nsys * sizeof(int)) &&
         alloc((void**)&ws->nlive, (restart + 1) * sizeof(int)) && alloc((void**)&ws->active, nsys * sizeof(int)) &&
         alloc((void**)&ws->x32, n32 * sizeof(float2)) && alloc((void**)&ws->y32, n8 * sizeof(float2)) &&
-        (!half || alloc(&ws->x16, n32 * 2 * sizeof(_Float16)));
+        (!half || alloc(&ws->x16, n32 * 2 * sizeof(_Float16))) &&
+        hipHostMalloc((void**)&ws->h_live, 4 * sizeof(int), hipHostMallocDefault) == hipSuccess &&
+        hipHostMalloc((void**)&ws->h_val, (size_t)nsys * sizeof(double2), hipHostMallocDefault) == hipSuccess;
     if (!ok) {
-      ws->free_batch();
-      return smh_fail(ctx, SMH_ERR_HIP, "batched solver allocation failed (%lld entries, restart %d)", (long long)n8,
-                      restart);
+      ws->release();
+      return smh_fail(ctx, SMH_ERR_HIP, "solver allocation failed (%lld entries, restart %d)", (long long)n8, restart);
     }
     // the FP32 input's padding slots stay zero
     hipLaunchKernelGGL(zero_f2_kernel, dim3(1024), dim3(256), 0, s, ws->x32, (int64_t)n32);
@@ -727,6 +602,10 @@ struct BatchSolver {
     return SMH_OK;
   }
 
+  int apply(int precision, const void* x, void* y) {
+    return KB == 1 ? smh::op_apply(op, precision, x, y, false) : smh::op_apply_batch(op, precision, x, y, false);
+  }
+
   // out = M v, or M P v with the preconditioner (with_P)
   int master(const double2* v, double2* out, int precision, bool with_P) {
     int rc;
@@ -736,19 +615,22 @@ struct BatchSolver {
       src = ws->pv;
     }
     if (precision == SMH_FP64) {
-      if ((rc = smh::op_apply_batch(op, SMH_FP64, src, ws->y64, false))) return rc;
-      hipLaunchKernelGGL(bmaster_fp64_kernel, dim3(blocks_for(n8)), dim3(256), 0, s, src, ws->t, ws->y64, out, n8);
+      if ((rc = apply(SMH_FP64, src, ws->y64))) return rc;
+      hipLaunchKernelGGL(bmaster_fp64_kernel<KB>, dim3(blocks_for(n8)), dim3(256), 0, s, src, ws->t, ws->y64, out, n8);
       ++mv64;
     } else if (precision == SMH_FP16) {
       if ((rc = smh::op_to_half_batch(op, src, ws->x16))) return rc;
-      if ((rc = smh::op_apply_batch(op, SMH_FP16, ws->x16, ws->y32, false))) return rc;
-      hipLaunchKernelGGL(bmaster_fp32_kernel, dim3(blocks_for(n8)), dim3(256), 0, s, src, ws->t, ws->y32, out, n8);
+      if ((rc = apply(SMH_FP16, ws->x16, ws->y32))) return rc;
+      hipLaunchKernelGGL(bmaster_fp32_kernel<KB>, dim3(blocks_for(n8)), dim3(256), 0, s, src, ws->t, ws->y32, out, n8);
       ++mv16;
     } else {
-      hipLaunchKernelGGL(to_fp32_b32_kernel, dim3(blocks_for(n8)), dim3(256), 0, s, src, ws->x32, n8, op->B,
-                         op->b32_S, (const int*)op->d_b32_tab);
-      if ((rc = smh::op_apply_batch(op, SMH_FP32, ws->x32, ws->y32, false))) return rc;
-      hipLaunchKernelGGL(bmaster_fp32_kernel, dim3(blocks_for(n8)), dim3(256), 0, s, src, ws->t, ws->y32, out, n8);
+      if (KB == 1)
+        hipLaunchKernelGGL(to_fp32_kernel, dim3(blocks_for(n8)), dim3(256), 0, s, src, ws->x32, n8);
+      else
+        hipLaunchKernelGGL(to_fp32_b32_kernel, dim3(blocks_for(n8)), dim3(256), 0, s, src, ws->x32, n8, op->B,
+                           op->b32_S, (const int*)op->d_b32_tab);
+      if ((rc = apply(SMH_FP32, ws->x32, ws->y32))) return rc;
+      hipLaunchKernelGGL(bmaster_fp32_kernel<KB>, dim3(blocks_for(n8)), dim3(256), 0, s, src, ws->t, ws->y32, out, n8);
       ++mv32;
     }
     SMH_HIP(ctx, hipGetLastError());
@@ -758,9 +640,9 @@ struct BatchSolver {
   // out[sys * ldo + j] = V_j[., sys]^H w[., sys], j < nv (device, no sync)
   int dots(const double2* Vb, int nv, const double2* wv, double2* out, int ldo) {
     if (nv < 1 || nv > kMaxBasis) return smh_fail(ctx, SMH_ERR_ARG, "basis size out of range");
-    hipLaunchKernelGGL(sdot_kernel, dim3(nblk, op->n_seg), dim3(kDotThreads), 0, s, Vb, n8, nv, wv, per_part,
+    hipLaunchKernelGGL(sdot_kernel<KB>, dim3(nblk, op->n_seg), dim3(kDotThreads), 0, s, Vb, n8, nv, wv, per_part,
                        (const int64_t*)op->d_seg_off, ws->partial);
-    hipLaunchKernelGGL(sreduce_kernel, dim3(nv * kB, op->n_seg), dim3(256), 0, s, ws->partial, nblk, out, ldo);
+    hipLaunchKernelGGL(sreduce_kernel<KB>, dim3(nv * KB, op->n_seg), dim3(256), 0, s, ws->partial, nblk, out, ldo);
     SMH_HIP(ctx, hipGetLastError());
     return SMH_OK;
   }
@@ -768,47 +650,58 @@ struct BatchSolver {
   int norms(const double2* v, double* out) {
     int rc = dots(v, 1, v, ws->hn, 1);
     if (rc) return rc;
-    std::vector<double2> h(nsys);
-    SMH_HIP(ctx, hipMemcpyAsync(h.data(), ws->hn, nsys * sizeof(double2), hipMemcpyDeviceToHost, s));
+    SMH_HIP(ctx, hipMemcpyAsync(ws->h_val, ws->hn, nsys * sizeof(double2), hipMemcpyDeviceToHost, s));
     SMH_HIP(ctx, hipStreamSynchronize(s));
-    for (int k = 0; k < nsys; ++k) out[k] = std::sqrt(std::max(0.0, h[k].x));
+    for (int k = 0; k < nsys; ++k) out[k] = std::sqrt(std::max(0.0, ws->h_val[k].x));
     return SMH_OK;
   }
 
+  void saxpy(int nv, const double2* c, double sgn, double2* w) {
+    hipLaunchKernelGGL(saxpy_kernel<KB>, dim3(blocks_for(n8)), dim3(256), 0, s, ws->V, n8, nv, c, restart + 1, sgn, w,
+                       n8, per_part, (const int*)op->d_seg_of);
+  }
+
   // Arnoldi step k of every system: w = M (P) V_k, CGS2, ||w||, rotation,
-  // V_{k+1} = w / ||w||. Device only (captured in a graph).
+  // V_{k+1} = w / ||w||, the live count to the host. Device only (captured in
+  // a graph).
   int arnoldi_step(int k, int precision) {
     int rc;
     const int ldh = restart + 1;
     const double2* vk = ws->V + (size_t)k * n8;
     if ((rc = master(vk, ws->w, precision, use_P))) return rc;
+    if (small) {
+      hipLaunchKernelGGL(arnoldi_small_kernel, dim3(1), dim3(kSmallThreads), 0, s, k, ws->V, (const double2*)ws->w,
+                         (int)n8, ws->atol, restart, ws->live, ws->H, ws->cs, ws->sn, ws->g, ws->kr, ws->nlive,
+                         ws->h_live);
+      SMH_HIP(ctx, hipGetLastError());
+      return SMH_OK;
+    }
     if ((rc = dots(ws->V, k + 1, ws->w, ws->h1, ldh))) return rc;
-    hipLaunchKernelGGL(saxpy_kernel, dim3(blocks_for(n8)), dim3(256), 0, s, ws->V, n8, k + 1, ws->h1, ldh, -1.0, ws->w,
-                       n8, per_part, (const int*)op->d_seg_of);
+    saxpy(k + 1, ws->h1, -1.0, ws->w);
     if ((rc = dots(ws->V, k + 1, ws->w, ws->h2, ldh))) return rc;
-    hipLaunchKernelGGL(saxpy_kernel, dim3(blocks_for(n8)), dim3(256), 0, s, ws->V, n8, k + 1, ws->h2, ldh, -1.0, ws->w,
-                       n8, per_part, (const int*)op->d_seg_of);
+    saxpy(k + 1, ws->h2, -1.0, ws->w);
     if ((rc = dots(ws->w, 1, ws->w, ws->hn, 1))) return rc;
     hipLaunchKernelGGL(givens_kernel, dim3(blocks_for(nsys, 64)), dim3(64), 0, s, k, ws->h1, ws->h2, ldh, ws->hn,
                        ws->atol, nsys, restart, ws->live, ws->H, ws->cs, ws->sn, ws->g, ws->kr, ws->scale, ws->nlive);
-    hipLaunchKernelGGL(sscale_kernel, dim3(blocks_for(n8)), dim3(256), 0, s, ws->w, ws->scale,
-                       ws->V + (size_t)(k + 1) * n8, n8, per_part, (const int*)op->d_seg_of);
+    hipLaunchKernelGGL(sscale_kernel<KB>, dim3(blocks_for(n8)), dim3(256), 0, s, ws->w, ws->scale,
+                       ws->V + (size_t)(k + 1) * n8, n8, per_part, (const int*)op->d_seg_of,
+                       (const int*)(ws->nlive + k), ws->h_live);
     SMH_HIP(ctx, hipGetLastError());
     return SMH_OK;
   }
 
-  // Step k through its graph: the first step of a configuration runs eagerly
-  // (lazy allocations and kernel attributes happen outside any capture),
-  // later ones are captured once and replayed.
+  // Step k: its first run is eager (lazy allocations and kernel attributes
+  // happen outside any capture, and a solver used once pays for no graph), the
+  // second is captured and replayed from then on.
   int run_step(int k, int precision) {
     const int pi = precision == SMH_FP64 ? 0 : (precision == SMH_FP32 ? 1 : 2);
     const int ui = use_P ? 1 : 0;
-    if (!graphs_enabled() || !ws->warmed[pi][ui]) {
+    const int key = ((pi * 2 + ui) << 8) | k;
+    if (!graphs_enabled() || !ws->ran.count(key)) {
       const int rc = arnoldi_step(k, precision);
-      if (!rc) ws->warmed[pi][ui] = true;
+      if (!rc) ws->ran.insert(key);
       return rc;
     }
-    const int key = ((pi * 2 + ui) << 8) | k;
     auto it = ws->graphs.find(key);
     if (it == ws->graphs.end()) {
       // the matvec counters count launches: the replay below counts this step's one matvec
@@ -840,9 +733,24 @@ struct BatchSolver {
     return SMH_OK;
   }
 
-  // GMRES on M x = b for the systems with active[sys] (others left untouched),
-  // each to ||b - M x|| <= atol[sys]; x_zero / trust_estimate as for the
-  // single right-hand side solver. res_out[sys]: residual (or estimate) of x.
+  // the systems' residuals (or estimates) to the host
+  int residuals(double* res_out) {
+    SMH_HIP(ctx, hipMemcpyAsync(ws->h_val, ws->res, nsys * sizeof(double), hipMemcpyDeviceToHost, s));
+    SMH_HIP(ctx, hipStreamSynchronize(s));
+    const double* v = reinterpret_cast<const double*>(ws->h_val);
+    std::copy(v, v + nsys, res_out);
+    return SMH_OK;
+  }
+
+  // GMRES on M x = b for the systems with active[sys] (others left untouched)
+  // from x (in/out), each to ||b - M x|| <= atol[sys]. x_zero: x is zero on
+  // entry, so the first residual is b itself. trust_estimate (inner solves of
+  // the refinement): one restart cycle at most, returning as soon as the
+  // Arnoldi residual estimates reach atol or the cycle ends, without
+  // recomputing the true residual (the caller takes it in FP64 and starts the
+  // next sweep: a reduced-precision operator whose error sits above atol would
+  // otherwise stall the restarts). res_out[sys]: residual of x (or the
+  // estimate); steps: Arnoldi steps taken.
   int gmres(double2* x, const double2* b, const double* atol, const int* active, int maxiter, int precision,
             double* res_out, int& steps, bool x_zero, bool trust_estimate) {
     int rc;
@@ -861,20 +769,18 @@ struct BatchSolver {
       hipLaunchKernelGGL(zero_int_kernel, dim3(1), dim3(256), 0, s, ws->nlive, R + 1);
       hipLaunchKernelGGL(cycle_init_kernel, dim3(blocks_for(nsys, 64)), dim3(64), 0, s, ws->hn, ws->atol, ws->active,
                          nsys, R, ws->g, ws->live, ws->scale, ws->res, ws->kr, ws->nlive);
+      // V_0 (zero for systems that do not run) and the live count
+      hipLaunchKernelGGL(sscale_kernel<KB>, dim3(blocks_for(n8)), dim3(256), 0, s, ws->w, ws->scale, ws->V, n8,
+                         per_part, (const int*)op->d_seg_of, (const int*)(ws->nlive + R), ws->h_live);
       SMH_HIP(ctx, hipGetLastError());
-      SMH_HIP(ctx, hipMemcpyAsync(res_out, ws->res, nsys * sizeof(double), hipMemcpyDeviceToHost, s));
-      SMH_HIP(ctx, hipMemcpyAsync(ws->h_pin, ws->nlive + R, sizeof(int), hipMemcpyDeviceToHost, s));
-      SMH_HIP(ctx, hipStreamSynchronize(s));
-      if (ws->h_pin[0] == 0 || steps >= maxiter) return SMH_OK;
-      hipLaunchKernelGGL(sscale_kernel, dim3(blocks_for(n8)), dim3(256), 0, s, ws->w, ws->scale, ws->V, n8, per_part,
-                         (const int*)op->d_seg_of);
+      if ((rc = residuals(res_out))) return rc;
+      if (ws->h_live[0] == 0 || steps >= maxiter) return SMH_OK;
       int k = 0;
       for (; k < R && steps < maxiter; ++k, ++steps) {
         if ((rc = run_step(k, precision))) return rc;
         ++iters;
-        SMH_HIP(ctx, hipMemcpyAsync(ws->h_pin, ws->nlive + k, sizeof(int), hipMemcpyDeviceToHost, s));
         SMH_HIP(ctx, hipStreamSynchronize(s));
-        if (ws->h_pin[0] == 0) {
+        if (*(volatile int*)ws->h_live == 0) {
           ++k;
           ++steps;
           break;
@@ -886,20 +792,14 @@ struct BatchSolver {
       if (k > 0) {
         if (use_P) {
           hipLaunchKernelGGL(zero2_kernel, dim3(1024), dim3(256), 0, s, ws->tmp, n8);
-          hipLaunchKernelGGL(saxpy_kernel, dim3(blocks_for(n8)), dim3(256), 0, s, ws->V, n8, k, ws->yv, R + 1, 1.0,
-                             ws->tmp, n8, per_part, (const int*)op->d_seg_of);
+          saxpy(k, ws->yv, 1.0, ws->tmp);
           if ((rc = smh::op_apply_precond_batch(op, ws->tmp, x, true))) return rc;
         } else {
-          hipLaunchKernelGGL(saxpy_kernel, dim3(blocks_for(n8)), dim3(256), 0, s, ws->V, n8, k, ws->yv, R + 1, 1.0, x,
-                             n8, per_part, (const int*)op->d_seg_of);
+          saxpy(k, ws->yv, 1.0, x);
         }
       }
       SMH_HIP(ctx, hipGetLastError());
-      if (trust_estimate) {
-        SMH_HIP(ctx, hipMemcpyAsync(res_out, ws->res, nsys * sizeof(double), hipMemcpyDeviceToHost, s));
-        SMH_HIP(ctx, hipStreamSynchronize(s));
-        return SMH_OK;
-      }
+      if (trust_estimate) return residuals(res_out);
     }
   }
 };
@@ -914,7 +814,9 @@ void solver_release(smh_op* op) {
 }
 
 void solver_drop_graphs(smh_op* op) {
-  if (op->solver_ws) static_cast<Ws*>(op->solver_ws)->drop_graphs();
+  if (!op->solver_ws) return;
+  static_cast<Ws*>(op->solver_ws)->one.drop_graphs();
+  static_cast<Ws*>(op->solver_ws)->batch.drop_graphs();
 }
 
 int op_apply_precond_batch(smh_op* op, const double2* x, double2* y, bool accumulate) {
@@ -946,29 +848,30 @@ int op_reserve_precond(smh_op* op, int k1) {
 
 }  // namespace smh
 
-// Blocks of kB right-hand sides over every segment, solved together (every
-// coupling matvec is one batched launch for all systems); same modes and
-// stopping rule as the single right-hand side path.
-static int solve_batched(smh_op* op, const double* t_diag, const double* rhs, double* x, int64_t nrhs, double tol,
-                         int restart, int maxiter, int mode, double* stats,
-                         std::chrono::steady_clock::time_point t0) {
+// Blocks of KB right-hand sides over every segment, solved together (every
+// coupling matvec is one launch for all systems).
+template <int KB>
+static int solve_blocks(smh_op* op, const double* t_diag, const double* rhs, double* x, int64_t nrhs, double tol,
+                        int restart, int maxiter, int mode, double* stats,
+                        std::chrono::steady_clock::time_point t0) {
   smh_ctx* ctx = op->ctx;
   hipStream_t s = ctx->stream;
-  BatchSolver S;
+  Ws* all = ws_of(op);
+  Solver<KB> S;
   S.op = op;
   S.ctx = ctx;
   S.s = s;
-  S.ws = ws_of(op);
+  S.ws = KB == 1 ? &all->one : &all->batch;
   S.n = op->n_part * op->B;
-  S.n8 = S.n * kB;
-  S.per_part = (int64_t)op->B * kB;
+  S.n8 = S.n * KB;
+  S.per_part = (int64_t)op->B * KB;
   S.restart = restart;
   int rc = S.init();
   if (rc) return rc;
-  Ws* ws = S.ws;
+  SolveWs* ws = S.ws;
   const int nsys = S.nsys;
-  if ((rc = smh::op_reserve_packed(op, kB))) return rc;
-  if ((rc = smh::op_reserve_batch(op))) return rc;
+  if ((rc = smh::op_reserve_packed(op, KB))) return rc;
+  if (KB > 1 && (rc = smh::op_reserve_batch(op))) return rc;
   SMH_HIP(ctx, hipMemcpyAsync(op->d_pk_in, t_diag, op->n_unk * sizeof(double2), hipMemcpyDefault, s));
   if ((rc = smh::op_unpack(op, SMH_FP64, op->d_pk_in, ws->t))) return rc;
   double worst = 0, sweeps_total = 0;
@@ -976,15 +879,17 @@ static int solve_batched(smh_op* op, const double* t_diag, const double* rhs, do
   bool converged_all = true;
   std::vector<double> bnorm(nsys), atol(nsys), res(nsys), prev_res(nsys), inner_atol(nsys), inner_res(nsys);
   std::vector<int> active(nsys), act(nsys);
-  for (int64_t r0 = 0; r0 < nrhs; r0 += kB) {
-    const int nb = (int)std::min<int64_t>(kB, nrhs - r0);
+  for (int64_t r0 = 0; r0 < nrhs; r0 += KB) {
+    const int nb = (int)std::min<int64_t>(KB, nrhs - r0);
     SMH_HIP(ctx, hipMemcpyAsync(op->d_pk_in, rhs + 2 * r0 * op->n_unk, (size_t)nb * op->n_unk * sizeof(double2),
                                 hipMemcpyDefault, s));
-    if ((rc = smh::op_unpack_batch(op, SMH_FP64, op->d_pk_in, nb, ws->b))) return rc;
+    if ((rc = KB == 1 ? smh::op_unpack(op, SMH_FP64, op->d_pk_in, ws->b)
+                      : smh::op_unpack_batch(op, SMH_FP64, op->d_pk_in, nb, ws->b)))
+      return rc;
     if ((rc = S.norms(ws->b, bnorm.data()))) return rc;
     for (int q = 0; q < nsys; ++q) {
       atol[q] = tol * bnorm[q];
-      active[q] = (q % kB) < nb && bnorm[q] > 0.0;
+      active[q] = (q % KB) < nb && bnorm[q] > 0.0;
     }
     int steps = 0;
     if (mode == SMH_SOLVE_FP64) {
@@ -1060,12 +965,14 @@ static int solve_batched(smh_op* op, const double* t_diag, const double* rhs, do
       }
     }
     for (int q = 0; q < nsys; ++q) {
-      if ((q % kB) >= nb) continue;
+      if ((q % KB) >= nb) continue;
       const double rel = bnorm[q] > 0 ? res[q] / bnorm[q] : 0.0;
       worst = std::max(worst, rel);
       if (rel > tol) converged_all = false;
     }
-    if ((rc = smh::op_pack_batch(op, SMH_FP64, ws->x, nb, op->d_pk_out))) return rc;
+    if ((rc = KB == 1 ? smh::op_pack(op, SMH_FP64, ws->x, op->d_pk_out)
+                      : smh::op_pack_batch(op, SMH_FP64, ws->x, nb, op->d_pk_out)))
+      return rc;
     SMH_HIP(ctx, hipMemcpyAsync(x + 2 * r0 * op->n_unk, op->d_pk_out, (size_t)nb * op->n_unk * sizeof(double2),
                                 hipMemcpyDefault, s));
   }
@@ -1078,101 +985,8 @@ static int solve_batched(smh_op* op, const double* t_diag, const double* rhs, do
     stats[3] = worst;
     stats[4] = secs;
     stats[5] = sweeps_total;
-    stats[6] = (double)kB;  // right-hand sides per batched matvec
+    stats[6] = KB == 1 ? 0.0 : (double)KB;  // right-hand sides per batched matvec
     stats[7] = (double)S.mv16;
-  }
-  if (!converged_all)
-    return smh_fail(ctx, SMH_ERR_NOCONV, "GMRES stopped at relative residual %.3e (tol %.1e)", worst, tol);
-  return SMH_OK;
-}
-
-static int solve_single(smh_op* op, const double* t_diag, const double* rhs, double* x, int64_t nrhs, double tol,
-                        int restart, int maxiter, int mode, double* stats,
-                        std::chrono::steady_clock::time_point t0) {
-  smh_ctx* ctx = op->ctx;
-  hipStream_t s = ctx->stream;
-  Solver S;
-  S.op = op;
-  S.ctx = ctx;
-  S.s = s;
-  S.ws = ws_of(op);
-  S.n = op->n_part * op->B;
-  S.restart = restart;
-  int rc = S.init();
-  if (rc) return rc;
-  Ws* ws = S.ws;
-  if ((rc = smh::op_reserve_packed(op, 1))) return rc;
-  // T diagonal in padded layout
-  SMH_HIP(ctx, hipMemcpyAsync(op->d_pk_in, t_diag, op->n_unk * sizeof(double2), hipMemcpyDefault, s));
-  if ((rc = smh::op_unpack(op, SMH_FP64, op->d_pk_in, ws->t1))) return rc;
-  double worst = 0, sweeps_total = 0;
-  int64_t steps_total = 0;
-  bool converged_all = true;
-  for (int64_t r = 0; r < nrhs; ++r) {
-    SMH_HIP(ctx, hipMemcpyAsync(op->d_pk_in, rhs + 2 * r * op->n_unk, op->n_unk * sizeof(double2),
-                                hipMemcpyDefault, s));
-    if ((rc = smh::op_unpack(op, SMH_FP64, op->d_pk_in, ws->b1))) return rc;
-    double bnorm;
-    if ((rc = S.norm(ws->b1, bnorm))) return rc;
-    const double atol = tol * bnorm;
-    double res = 0;
-    int steps = 0;
-    if (mode == SMH_SOLVE_FP64) {
-      // x0 = rhs, as smuthi passes rhs as initial guess; GMRES returns the true residual of x
-      SMH_HIP(ctx, hipMemcpyAsync(ws->x1, ws->b1, S.n * sizeof(double2), hipMemcpyDeviceToDevice, s));
-      if ((rc = S.gmres(ws->x1, ws->b1, atol, maxiter, SMH_FP64, res, steps))) return rc;
-      steps_total += steps;
-      sweeps_total += 1;
-    } else {
-      // iterative refinement from x0 = 0: FP64 residual, FP32-matvec inner GMRES
-      hipLaunchKernelGGL(zero2_kernel, dim3(1024), dim3(256), 0, s, ws->x1, S.n);
-      SMH_HIP(ctx, hipMemcpyAsync(ws->r1, ws->b1, S.n * sizeof(double2), hipMemcpyDeviceToDevice, s));
-      res = bnorm;
-      bool fresh = true;  // res is the FP64 residual of the current x
-      int budget = maxiter;
-      for (int sweep = 0; sweep < 50; ++sweep) {
-        if (sweep > 0) {
-          if ((rc = S.master(ws->x1, ws->r1, SMH_FP64))) return rc;
-          hipLaunchKernelGGL(sub_kernel, dim3(blocks_for(S.n)), dim3(256), 0, s, ws->b1, ws->r1, ws->r1, S.n);
-          if ((rc = S.norm(ws->r1, res))) return rc;
-          fresh = true;
-        }
-        if (res <= atol || budget <= 0) break;
-        hipLaunchKernelGGL(zero2_kernel, dim3(1024), dim3(256), 0, s, ws->d1, S.n);
-        double inner_res = 0;
-        int inner_steps = 0;
-        const double inner_atol = std::max(atol * 0.5, kInnerRel * res);
-        if ((rc = S.gmres(ws->d1, ws->r1, inner_atol, budget, SMH_FP32, inner_res, inner_steps, true, true))) return rc;
-        budget -= inner_steps;
-        steps_total += inner_steps;
-        hipLaunchKernelGGL(add_kernel, dim3(blocks_for(S.n)), dim3(256), 0, s, ws->x1, ws->d1, S.n);
-        sweeps_total += 1;
-        fresh = false;
-      }
-      if (!fresh) {
-        if ((rc = S.master(ws->x1, ws->r1, SMH_FP64))) return rc;
-        hipLaunchKernelGGL(sub_kernel, dim3(blocks_for(S.n)), dim3(256), 0, s, ws->b1, ws->r1, ws->r1, S.n);
-        if ((rc = S.norm(ws->r1, res))) return rc;
-      }
-    }
-    const double rel = bnorm > 0 ? res / bnorm : 0.0;
-    worst = std::max(worst, rel);
-    if (rel > tol) converged_all = false;
-    if ((rc = smh::op_pack(op, SMH_FP64, ws->x1, op->d_pk_out))) return rc;
-    SMH_HIP(ctx, hipMemcpyAsync(x + 2 * r * op->n_unk, op->d_pk_out, op->n_unk * sizeof(double2),
-                                hipMemcpyDefault, s));
-  }
-  SMH_HIP(ctx, hipStreamSynchronize(s));
-  const double secs = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-  if (stats) {
-    stats[0] = (double)steps_total;
-    stats[1] = (double)S.mv64;
-    stats[2] = (double)S.mv32;
-    stats[3] = worst;
-    stats[4] = secs;
-    stats[5] = sweeps_total;
-    stats[6] = 0;
-    stats[7] = 0;
   }
   if (!converged_all)
     return smh_fail(ctx, SMH_ERR_NOCONV, "GMRES stopped at relative residual %.3e (tol %.1e)", worst, tol);
@@ -1202,8 +1016,8 @@ extern "C" int smh_solve(smh_op* op, const double* t_diag, const double* rhs, do
   SMH_CHECK(ctx, batch_ok || !need_batch, SMH_ERR_UNSUPPORTED,
             "ensembles and preconditioned solves need an operator with the batched kernels");
   if (batch_ok && (nrhs > 1 || need_batch))
-    return solve_batched(op, t_diag, rhs, x, nrhs, tol, restart, maxiter, mode, stats, t0);
-  return solve_single(op, t_diag, rhs, x, nrhs, tol, restart, maxiter, mode, stats, t0);
+    return solve_blocks<kB>(op, t_diag, rhs, x, nrhs, tol, restart, maxiter, mode, stats, t0);
+  return solve_blocks<1>(op, t_diag, rhs, x, nrhs, tol, restart, maxiter, mode, stats, t0);
 }
 
 extern "C" int smh_op_set_preconditioner(smh_op* op, int k1, const int* nbr, const double* blocks) {

@@ -1,0 +1,44 @@
+"""Solves of one right-hand side on the device: systems whose Arnoldi step runs
+in one workgroup (up to 4096 unknowns, edge at 682 / 683 particles of 6), the
+several-launch step above, restart lengths from one step to the largest basis,
+and repeated solves (the first runs eagerly, the second captures its graphs,
+the third replays them, with eager matvecs between). The residual is taken
+with the plain numpy operator of the partial-sum tests; an FP64 solve to tol
+leaves tol plus the FP64 operators' own difference (1e-13)."""
+import numpy as np
+import pytest
+
+from smuthi_amd.particles import Sphere
+from test_gpu_partials import H, _reference, _system
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope='module')
+def gpu():
+    from smuthi_amd import cuda
+    assert cuda.enable_gpu(), 'MI355X not available'
+    return cuda
+
+
+@pytest.mark.parametrize('n,restart', [(2, 1), (17, 127), (682, 6), (682, 40), (683, 6), (683, 40)])
+def test_single_solves_meet_the_tolerance(gpu, n, restart):
+    from smuthi_amd.linear_system import CouplingMatrixRadialLookupCUDA
+    xy, rho, table = _system(n, n)
+    op = CouplingMatrixRadialLookupCUDA.from_table(table, rho, [Sphere([a, b, 200.0], 1.5, 50.0, 1, 1)
+                                                                for a, b in xy], H, 'linear')
+    rng = np.random.default_rng(n + restart)
+    d = np.hypot(xy[:, None, 0] - xy[None, :, 0], xy[:, None, 1] - xy[None, :, 1])
+    t = (0.25 / (6 * (1 / (1 + d / 500)).sum(1).max()) * np.exp(2j * np.pi * rng.uniform(size=(n, 6)))).ravel()
+    b = rng.standard_normal(n * 6) + 1j * rng.standard_normal(n * 6)
+    print('single solve: %d particles, restart %d' % (n, restart), flush=True)
+    first = None
+    for repeat in range(3):
+        for precision in ('double', 'mixed'):
+            x, stats, ok = op.solve_master(t, b, 1e-9, precision=precision, restart=restart, with_stats=True)
+            assert ok and stats['relative_residual'] <= 1e-9
+            r = b - x + t * _reference(xy, rho, table, x.reshape(1, n, 6)).ravel()
+            assert np.linalg.norm(r) <= (1e-9 + 1e-12) * np.linalg.norm(b), (precision, repeat)
+            first = x if first is None else first
+            assert np.linalg.norm(x - first) <= 1e-8 * np.linalg.norm(first)
+        op.matvec(b, 'single')
