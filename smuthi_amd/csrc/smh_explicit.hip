@@ -26,13 +26,15 @@
 // A last pass writes the complex64 copy used by FP32 matvecs.
 //
 // Matvec: y = W x, a dense complex GEMV over the padded vectors, one
-// wavefront per row (HBM-bound on W).
+// wavefront per row, or a product with kBatch vectors at a time on the MFMA
+// (both HBM-bound on W, which a batch reads once).
 #include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <vector>
 
 #include "smh_op.h"
+#include "smh_radial_kernel.h"
 #include "smh_special.h"
 
 namespace {
@@ -345,9 +347,118 @@ __global__ void __launch_bounds__(256) explicit_gemv_kernel(const void* __restri
   }
 }
 
+// Y = W X for kBatch vectors, X and Y [n][kBatch] complex, W [n][n]. A workgroup
+// takes 16 rows, its waves the columns in turns of kCols; a lane (q = lane / 16)
+// reads 64 contiguous bytes of its row, which are its K values of the turn's
+// MFMA 16x16x4 steps (the column order inside a turn is the lanes' own, the same
+// for W and X). The 16 result columns are (vector, re | im): Re W meets (Re x,
+// Im x), Im W meets (-Im x, Re x), the other half of the lane pair. Even and odd
+// steps and the two products keep sums of their own, the waves' sums are added
+// at the end. Bound by HBM on W, read once for all vectors: the next turn's
+// loads are in flight during the products, and eight waves of four such
+// workgroups keep about 130 KB per CU outstanding.
+constexpr int kGemmWaves = 8;
+template <typename Real>
+__global__ void __launch_bounds__(64 * kGemmWaves)
+    explicit_gemm_kernel(const void* __restrict__ Wv, const void* __restrict__ xv, void* __restrict__ yv, int64_t n) {
+  using M = smh::Mfma<Real>;
+  using R2 = typename smh::Vec2<Real>::t;
+  constexpr int J = 64 / (int)sizeof(R2), kCols = 4 * J;  // columns per lane and per turn
+  __shared__ Real part[kGemmWaves][16][16];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, q = lane >> 4, c = lane & 15;
+  const int64_t row0 = (int64_t)blockIdx.x * 16;
+  const int64_t row = min(row0 + c, n - 1);  // rows beyond n repeat the last one (not stored)
+  const R2* W = (const R2*)Wv + row * n;
+  const Real* x = (const Real*)xv + c;  // this lane's column (vector, re | im) of X
+  const Real sgn = (c & 1) ? Real(1) : Real(-1);
+  typename M::v4 acc[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = typename M::v4{0, 0, 0, 0};
+  auto load = [&](int64_t c0, R2 (&w)[J], Real (&b)[J]) {
+    const int64_t k0 = c0 + q * J;
+    if constexpr (sizeof(Real) == 4) {
+      // 16-byte loads: rows of W start at multiples of 16 bytes (n is even: blocksizes are)
+      const float4* w4 = reinterpret_cast<const float4*>(W + k0);
+#pragma unroll
+      for (int j = 0; j < J / 2; ++j) {
+        const float4 v = w4[j];
+        w[2 * j] = R2{v.x, v.y};
+        w[2 * j + 1] = R2{v.z, v.w};
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < J; ++j) w[j] = W[k0 + j];
+    }
+#pragma unroll
+    for (int j = 0; j < J; ++j) b[j] = x[(k0 + j) * 16];
+  };
+  auto multiply = [&](const R2 (&w)[J], const Real (&b)[J]) {
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      acc[j & 1] = M::op(w[j].x, b[j], acc[j & 1]);
+      acc[2 + (j & 1)] = M::op(w[j].y, sgn * smh::lane_xor1(b[j]), acc[2 + (j & 1)]);
+    }
+  };
+  const int64_t turns = n / kCols;
+  if (wave < turns) {
+    R2 w[J];
+    Real b[J];
+    load((int64_t)wave * kCols, w, b);
+    for (int64_t t = wave; t < turns; t += kGemmWaves) {
+      R2 w1[J];
+      Real b1[J];
+      load((t + kGemmWaves < turns ? t + kGemmWaves : t) * kCols, w1, b1);
+      multiply(w, b);
+#pragma unroll
+      for (int j = 0; j < J; ++j) {
+        w[j] = w1[j];
+        b[j] = b1[j];
+      }
+    }
+  }
+  if (turns * kCols < n && wave == (int)(turns % kGemmWaves)) {  // the columns left over
+    R2 w[J];
+    Real b[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const int64_t k = turns * kCols + q * J + j;
+      w[j] = k < n ? W[k] : R2{0, 0};
+      b[j] = k < n ? x[k * 16] : Real(0);
+    }
+    multiply(w, b);
+  }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const int r = M::kRowIs4q ? 4 * q + v : 4 * v + q;
+    part[wave][r][c] = (acc[0][v] + acc[1][v]) + (acc[2][v] + acc[3][v]);
+  }
+  __syncthreads();
+  if (threadIdx.x < 256) {
+    const int r = threadIdx.x >> 4, k = threadIdx.x & 15;
+    Real s = part[0][r][k];
+#pragma unroll
+    for (int w = 1; w < kGemmWaves; ++w) s += part[w][r][k];
+    if (row0 + r < n) ((Real*)yv)[(row0 + r) * 16 + k] = s;
+  }
+}
+
 }  // namespace
 
 namespace smh {
+
+int explicit_apply_batch(smh_op* op, int precision, const void* x_pad, void* y_pad) {
+  smh_ctx* ctx = op->ctx;
+  const int64_t n = op->n_part * op->B;
+  const dim3 grid((unsigned)((n + 15) / 16)), block(64 * kGemmWaves);
+  if (precision == SMH_FP32)
+    hipLaunchKernelGGL(explicit_gemm_kernel<float>, grid, block, 0, ctx->stream, (const void*)op->d_W32, x_pad, y_pad,
+                       n);
+  else
+    hipLaunchKernelGGL(explicit_gemm_kernel<double>, grid, block, 0, ctx->stream, (const void*)op->d_W64, x_pad,
+                       y_pad, n);
+  SMH_HIP(ctx, hipGetLastError());
+  return SMH_OK;
+}
 
 int explicit_apply(smh_op* op, int precision, const void* x_pad, void* y_pad, bool time_kernel) {
   smh_ctx* ctx = op->ctx;
@@ -541,6 +652,7 @@ extern "C" int smh_explicit_create(smh_ctx* ctx, int64_t n_part, const double* x
   op->B = smh_blocksize(l_max, m_max);
   op->Bh = (op->B + 15) / 16 * 16;
   op->MP = 2 * op->Bh;
+  op->b32_S = op->B;  // batches in the plain layout [n][kBatch]
   auto fail = [&](int code) {
     smh_op_free(op);
     delete op;

@@ -183,6 +183,7 @@ int vol_upload(smh_op* op, const double* plus, const double* minus);
 int vol_download(smh_op* op, double* plus, double* minus);
 // explicit operator: dense matvec and the padded matrix (smh_explicit.hip)
 int explicit_apply(smh_op* op, int precision, const void* x_pad, void* y_pad, bool time_kernel);
+int explicit_apply_batch(smh_op* op, int precision, const void* x_pad, void* y_pad);
 int explicit_download(smh_op* op, double* W);
 // solver workspace release, and the drop of its captured graphs when the
 // operator's buffers change (smh_solver.hip)
@@ -200,6 +201,11 @@ void lu_release(smh_op* op);
 // kBatch-RHS matvec (radial operators): FP64 input and every output on padded
 // [n_part][B][kBatch] vectors; the FP32 input in the layout of b32_index()
 bool op_has_batch(const smh_op* op, int precision);
+// whether blocks of right-hand sides share a launch: the lookup operators above
+// and the explicit matrix (which has no preconditioner and no launch shapes)
+inline bool op_takes_blocks(const smh_op* op, int precision) {
+  return (op->kind == 2 && precision != SMH_FP16) || op_has_batch(op, precision);
+}
 int op_apply_batch(smh_op* op, int precision, const void* x_pad, void* y_pad, bool time_kernel);
 int op_unpack_batch(smh_op* op, int precision, const double2* pk, int nrhs, void* pad);
 int op_pack_batch(smh_op* op, int precision, const void* pad, int nrhs, double2* pk);

@@ -798,6 +798,10 @@ int op_apply_batch(smh_op* op, int precision, const void* x_pad, void* y_pad, bo
               "no FP16 matvec for this volume operator");
     return vol_apply_batch(op, precision, x_pad, y_pad, time_kernel);
   }
+  if (op->kind == 2) {
+    SMH_CHECK(ctx, precision != SMH_FP16, SMH_ERR_UNSUPPORTED, "no FP16 matvec for the explicit matrix");
+    return explicit_apply_batch(op, precision, x_pad, y_pad);
+  }
   const bool half = precision == SMH_FP16;
   const int pi = (precision == SMH_FP32 || half) ? 0 : 1;
   SMH_CHECK(ctx, op_has_batch(op, precision), SMH_ERR_UNSUPPORTED, "no batched matvec for this operator");
@@ -1226,7 +1230,7 @@ extern "C" int smh_op_matvec(smh_op* op, const double* x, double* y, int64_t nrh
   if (rc) return rc;
   hipStream_t s = ctx->stream;
   SMH_HIP(ctx, hipMemcpyAsync(op->d_pk_in, x, op->n_unk * nrhs * sizeof(double2), hipMemcpyHostToDevice, s));
-  if ((nrhs > 1 || precision == SMH_FP16) && op_has_batch(op, precision)) {
+  if ((nrhs > 1 || precision == SMH_FP16) && op_takes_blocks(op, precision)) {
     // blocks of kBatch right-hand sides through the batched kernel
     if ((rc = op_reserve_batch(op))) return rc;
     for (int64_t r0 = 0; r0 < nrhs; r0 += kBatch) {

@@ -1012,10 +1012,11 @@ extern "C" int smh_solve(smh_op* op, const double* t_diag, const double* rhs, do
   SMH_HIP(ctx, hipSetDevice(ctx->device));
   const auto t0 = std::chrono::steady_clock::now();
   const bool batch_ok = smh::op_has_batch(op, SMH_FP32) && smh::op_has_batch(op, SMH_FP64);
+  const bool blocks_ok = smh::op_takes_blocks(op, SMH_FP32) && smh::op_takes_blocks(op, SMH_FP64);
   const bool need_batch = mode == SMH_SOLVE_MIXED16 || op->d_P != nullptr || op->n_seg > 1;
   SMH_CHECK(ctx, batch_ok || !need_batch, SMH_ERR_UNSUPPORTED,
             "ensembles and preconditioned solves need an operator with the batched kernels");
-  if (batch_ok && (nrhs > 1 || need_batch))
+  if (blocks_ok && (nrhs > 1 || need_batch))
     return solve_blocks<kB>(op, t_diag, rhs, x, nrhs, tol, restart, maxiter, mode, stats, t0);
   return solve_blocks<1>(op, t_diag, rhs, x, nrhs, tol, restart, maxiter, mode, stats, t0);
 }
