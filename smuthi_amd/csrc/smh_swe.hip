@@ -11,12 +11,16 @@
 // Layout. One thread per point, 256 points per workgroup; the particles are
 // staged through LDS in chunks (centre, squared radius, z range, the B
 // coefficients), every thread reading the same particle at the same time (LDS
-// broadcast). Per (point, particle) the distance runs in FP64 and, in the FP32
+// broadcast). Where the points alone leave the chip idle, the particles are
+// split over workgroups too, whose sums a second kernel adds in FP64. Per (point, particle) the distance runs in FP64 and, in the FP32
 // kernel, the phase Re(k) r is reduced to [-pi, pi] in FP64 (large k r stays
 // accurate); the Hankel recurrence, the normalized Legendre functions and the
-// multipole sum run in Real (FP32 or FP64). The sum is
-// formed in spherical components per m, rotated by e^{i m phi} once per m and
-// added in Cartesian components.
+// multipole sum run in Real (FP32 or FP64). The
+// sum runs per l over m >= 0 in spherical components: the waves m and -m share
+// their Legendre functions, so their coefficients are staged as sum and
+// difference (b_m + b_-m and b_m - b_-m), which cos / sin(m phi) combine; the
+// radial factors multiply each l's sums once and the unit vectors the total
+// once.
 #include <algorithm>
 #include <cmath>
 #include <complex>
@@ -31,10 +35,11 @@ constexpr int kSweChunk = 32;
 
 struct SweArgs {
   const double* part;   // [n_part][6]: x, y, z, radius^2, z lower, z upper
-  const double2* coef;  // [n_part][B] in (tau, l, m) order; H: b_(1-tau) staged at tau
+  const double2* coef;  // [n_part][B], H: b_(1-tau) staged at tau; unrolled kernels in swe_pair_offset order, else (tau, l, m)
   const double* pts;    // [n_pts][3]
-  double2* out;         // [3][n_pts]
+  void* out;            // [splits][3][n_pts] complex of Real
   int64_t n_part, n_pts;
+  int64_t per_split;    // particles per blockIdx.y
   double k_re, k_im;
 };
 
@@ -46,6 +51,15 @@ __host__ __device__ constexpr int swe_index(int tau, int l, int m, int l_max, in
   return n + m + (l < m_max ? l : m_max);
 }
 
+// Position of (l, m >= 0)'s coefficients in the unrolled kernels' order: by l,
+// then m; m = 0: b_0 (tau 0), b_0 (tau 1); m > 0: sum and difference of b_m and
+// b_-m for tau 0, then for tau 1.
+__host__ __device__ constexpr int swe_pair_offset(int l, int m, int m_max) {
+  int n = 0;
+  for (int q = 1; q < l; ++q) n += 2 + 4 * (q < m_max ? q : m_max);
+  return n + (m > 0 ? 2 + 4 * (m - 1) : 0);
+}
+
 // Prefactor of the normalized P_m^m = pref st^m (legendre_normalized, utility/math.py:38-104):
 // res_m = prod_{t = 2, 4, .., 2m} (1 + 1/t), pref = sqrt(res_m / 2)
 __host__ __device__ inline double legendre_mm_prefactor(int m) {
@@ -54,12 +68,15 @@ __host__ __device__ inline double legendre_mm_prefactor(int m) {
   return sqrt(res / 2.0);
 }
 
+// Bound by VALU issue: per pair about 100 instructions of FP64 geometry and
+// phase, 100 of Hankel and Legendre recurrences and 250 of the sum at l_max =
+// m_max = 3.
 template <typename Real, int LMAX, int MMAX>
 __global__ void __launch_bounds__(kSwePoints) swe_field_kernel(SweArgs a) {
   constexpr int B = 2 * (MMAX * (MMAX + 2) + (LMAX - MMAX) * (2 * MMAX + 1));
   using C = cplx<Real>;
   __shared__ double sp[kSweChunk][6];
-  __shared__ C sc[kSweChunk][B];
+  __shared__ __align__(16) C sc[kSweChunk][B];
 
   const int64_t ip = (int64_t)blockIdx.x * kSwePoints + threadIdx.x;
   const bool live = ip < a.n_pts;
@@ -70,9 +87,13 @@ __global__ void __launch_bounds__(kSwePoints) swe_field_kernel(SweArgs a) {
     pz = a.pts[3 * ip + 2];
   }
   C ex{0, 0}, ey{0, 0}, ez{0, 0};
+  const double k2 = a.k_re * a.k_re + a.k_im * a.k_im;
+  const double ikr = a.k_re / k2, iki = -a.k_im / k2;  // 1 / k
+  const int64_t first = (int64_t)blockIdx.y * a.per_split;
+  const int64_t last = first + a.per_split < a.n_part ? first + a.per_split : a.n_part;
 
-  for (int64_t p0 = 0; p0 < a.n_part; p0 += kSweChunk) {
-    const int np = (int)(a.n_part - p0 < kSweChunk ? a.n_part - p0 : kSweChunk);
+  for (int64_t p0 = first; p0 < last; p0 += kSweChunk) {
+    const int np = (int)(last - p0 < kSweChunk ? last - p0 : kSweChunk);
     __syncthreads();
     for (int j = threadIdx.x; j < np * 6; j += kSwePoints) sp[j / 6][j % 6] = a.part[(p0 + j / 6) * 6 + j % 6];
     for (int j = threadIdx.x; j < np * B; j += kSwePoints) {
@@ -83,9 +104,9 @@ __global__ void __launch_bounds__(kSwePoints) swe_field_kernel(SweArgs a) {
     if (!live) continue;
     for (int q = 0; q < np; ++q) {
       const double dx = px - sp[q][0], dy = py - sp[q][1], dz = pz - sp[q][2];
-      const double r2 = dx * dx + dy * dy + dz * dz;
+      const double rho2 = dx * dx + dy * dy, r2 = rho2 + dz * dz;
       if (!(r2 > sp[q][3]) || pz < sp[q][4] || pz >= sp[q][5]) continue;
-      const double r = sqrt(r2), rho = sqrt(dx * dx + dy * dy);
+      const double r = sqrt(r2), rho = sqrt(rho2);
       const double ir = 1.0 / r;
       const Real ct = (Real)(dz * ir), st = (Real)(rho * ir);
       Real cp = 1, sn = 0;
@@ -94,38 +115,25 @@ __global__ void __launch_bounds__(kSwePoints) swe_field_kernel(SweArgs a) {
         cp = (Real)(dx * irho);
         sn = (Real)(dy * irho);
       }
-      // spherical Hankel h_l(x), x = k r, and d/dx(x h_l) / x. FP64 kernel: all in FP64. FP32
-      // kernel: the phase Re(k) r is reduced to [-pi, pi] in FP64, the rest runs in FP32.
+      // spherical Hankel h_l(x), x = k r. FP64 kernel: all in FP64. FP32 kernel: the phase Re(k) r is
+      // reduced to [-pi, pi] in FP64, the rest runs in FP32.
       using Z = cplx<Real>;
-      const Z x{(Real)(a.k_re * r), (Real)(a.k_im * r)};
-      const Z ix = cdiv(Z{Real(1), Real(0)}, x);
+      const Z ix{(Real)(ikr * ir), (Real)(iki * ir)};
       Z eix;
       if constexpr (sizeof(Real) == 8) {
-        const double dmp = exp(-x.im);
-        eix = Z{dmp * cos(x.re), dmp * sin(x.re)};
+        sincos(a.k_re * r, &eix.im, &eix.re);
+        if (a.k_im != 0.0) eix = cscale(eix, exp(-a.k_im * r));
       } else {
         const double ph = a.k_re * r;
         const float red = (float)(ph - 6.283185307179586477 * rint(ph * 0.15915494309189533577));
-        const float dmp = expf((float)(-a.k_im * r));
-        float sr, cr;
-        sincosf(red, &sr, &cr);
-        eix = Z{dmp * cr, dmp * sr};
+        sincosf(red, &eix.im, &eix.re);
+        if (a.k_im != 0.0) eix = cscale(eix, expf((float)(-a.k_im * r)));
       }
       Z h[LMAX + 1];
-      h[0] = cmul(Z{eix.im, -eix.re}, ix);  // -i e^{ix} / x
-      h[1] = cscale(cmul(cmul(eix, Z{x.re, x.im + Real(1)}), cmul(ix, ix)), Real(-1));
+      h[0] = cmul(Z{eix.im, -eix.re}, ix);            // -i e^{ix} / x
+      h[1] = cmul(h[0], Z{ix.re, ix.im - Real(1)});  // -e^{ix} (x + i) / x^2
 #pragma unroll
       for (int l = 1; l < LMAX; ++l) h[l + 1] = csub(cscale(cmul(ix, h[l]), Real(2 * l + 1)), h[l - 1]);
-      // radial factors per l: A = h / sqrt(2l(l+1)), Bv = l(l+1) h / x / sqrt(..), Cv = (x h_(l-1) - l h_l) / x / sqrt(..)
-      C A[LMAX + 1], Bv[LMAX + 1], Cv[LMAX + 1];
-#pragma unroll
-      for (int l = 1; l <= LMAX; ++l) {
-        const Real pf = (Real)(1.0 / sqrt(2.0 * l * (l + 1)));
-        const Z hx = cmul(h[l], ix);
-        A[l] = cscale(h[l], pf);
-        Bv[l] = cscale(hx, pf * Real(l * (l + 1)));
-        Cv[l] = cscale(csub(h[l - 1], cscale(hx, Real(l))), pf);
-      }
       // normalized associated Legendre P, pi, tau of cos(theta) (utility/math.py:38-104, real argument)
       Real P[LMAX + 1][MMAX + 1], PI[LMAX + 1][MMAX + 1], TA[LMAX + 1][MMAX + 1];
       {
@@ -135,7 +143,6 @@ __global__ void __launch_bounds__(kSwePoints) swe_field_kernel(SweArgs a) {
         pp[0] = 0;
         pp[1] = (Real)sqrt(3.0) * P[0][0];
         TA[1][0] = -st * pp[1];
-        PI[1][0] = 0;
 #pragma unroll
         for (int l = 1; l < LMAX; ++l) {
           P[l + 1][0] = (Real)(sqrt((2.0 * l + 1) * (2.0 * l + 3)) / (l + 1)) * ct * P[l][0] -
@@ -143,7 +150,6 @@ __global__ void __launch_bounds__(kSwePoints) swe_field_kernel(SweArgs a) {
           pp[l + 1] = (Real)((l + 1) * sqrt((2.0 * l + 3) / (2.0 * l + 1))) * P[l][0] +
                       (Real)sqrt((2.0 * l + 3) / (2.0 * l + 1)) * ct * pp[l];
           TA[l + 1][0] = -st * pp[l + 1];
-          PI[l + 1][0] = 0;
         }
 #pragma unroll
         for (int m = 1; m <= MMAX; ++m) {
@@ -166,52 +172,90 @@ __global__ void __launch_bounds__(kSwePoints) swe_field_kernel(SweArgs a) {
           }
         }
       }
-      // unit vectors
-      const Real erx = st * cp, ery = st * sn, erz = ct;
-      const Real etx = ct * cp, ety = ct * sn, etz = -st;
-      const Real epx = -sn, epy = cp;
-      const C* b = sc[q];
-      // e^{i m phi} for m >= 0
-      C eim[MMAX + 1];
-      eim[0] = C{1, 0};
+      // cos, sin(m phi)
+      Real cm[MMAX + 1], sm[MMAX + 1];
+      cm[0] = 1;
+      sm[0] = 0;
 #pragma unroll
-      for (int m = 1; m <= MMAX; ++m) eim[m] = cmul(eim[m - 1], C{cp, sn});
-#pragma unroll
-      for (int m = -MMAX; m <= MMAX; ++m) {
-        const int am = m < 0 ? -m : m;
-        // spherical components of sum_l at this m (before e^{i m phi})
-        C cr{0, 0}, cth{0, 0}, cph{0, 0};
-#pragma unroll
-        for (int l = (am > 1 ? am : 1); l <= LMAX; ++l) {
-          const C b0 = b[swe_index(0, l, m, LMAX, MMAX)], b1 = b[swe_index(1, l, m, LMAX, MMAX)];
-          const C u = cmul(b0, A[l]);   // tau = 0
-          const C wb = cmul(b1, Bv[l]);  // tau = 1, radial part
-          const C wc = cmul(b1, Cv[l]);  // tau = 1, transverse part
-          const Real mpi = Real(m) * PI[l][am], ta = TA[l][am];
-          // tau 0: u (i m pi e_theta - tau e_phi); tau 1: wb P e_r + wc (tau e_theta + i m pi e_phi)
-          cr.re += wb.re * P[l][am];
-          cr.im += wb.im * P[l][am];
-          cth.re += -mpi * u.im + ta * wc.re;
-          cth.im += mpi * u.re + ta * wc.im;
-          cph.re += -ta * u.re - mpi * wc.im;
-          cph.im += -ta * u.im + mpi * wc.re;
-        }
-        const C e = m >= 0 ? eim[am] : C{eim[am].re, -eim[am].im};
-        const C r_ = cmul(cr, e), t_ = cmul(cth, e), f_ = cmul(cph, e);
-        ex.re += r_.re * erx + t_.re * etx + f_.re * epx;
-        ex.im += r_.im * erx + t_.im * etx + f_.im * epx;
-        ey.re += r_.re * ery + t_.re * ety + f_.re * epy;
-        ey.im += r_.im * ery + t_.im * ety + f_.im * epy;
-        ez.re += r_.re * erz + t_.re * etz;
-        ez.im += r_.im * erz + t_.im * etz;
+      for (int m = 1; m <= MMAX; ++m) {
+        cm[m] = cm[m - 1] * cp - sm[m - 1] * sn;
+        sm[m] = cm[m - 1] * sn + sm[m - 1] * cp;
       }
+      const C* b = sc[q];
+      C er{0, 0}, et{0, 0}, ep{0, 0};  // spherical components of the particle's field
+#pragma unroll
+      for (int l = 1; l <= LMAX; ++l) {
+        // tau 0: h_l (i m pi e_theta - tau e_phi) / sqrt(2 l (l + 1)); tau 1: (l (l + 1) h_l / x P e_r +
+        // (x h_l)' / x (tau e_theta + i m pi e_phi)) / sqrt(2 l (l + 1)): sums over m of
+        // P b1, tau b1, m pi b1, m pi b0, tau b0 (times e^{i m phi})
+        const C* bl = b + swe_pair_offset(l, 0, MMAX);
+        const C b00 = bl[0], b10 = bl[1];
+        C rp{b10.re * P[l][0], b10.im * P[l][0]};
+        C t1{b10.re * TA[l][0], b10.im * TA[l][0]}, t0{b00.re * TA[l][0], b00.im * TA[l][0]};
+        C q1{0, 0}, q0{0, 0};
+#pragma unroll
+        for (int m = 1; m <= (l < MMAX ? l : MMAX); ++m) {
+          const C* bm = bl + 2 + 4 * (m - 1);
+          const C s0 = bm[0], d0 = bm[1], s1 = bm[2], d1 = bm[3];
+          // b_m e^{i m phi} +- b_-m e^{-i m phi}
+          const C u0{s0.re * cm[m] - d0.im * sm[m], s0.im * cm[m] + d0.re * sm[m]};
+          const C v0{d0.re * cm[m] - s0.im * sm[m], d0.im * cm[m] + s0.re * sm[m]};
+          const C u1{s1.re * cm[m] - d1.im * sm[m], s1.im * cm[m] + d1.re * sm[m]};
+          const C v1{d1.re * cm[m] - s1.im * sm[m], d1.im * cm[m] + s1.re * sm[m]};
+          const Real p_ = P[l][m], ta = TA[l][m], mpi = Real(m) * PI[l][m];
+          rp.re += p_ * u1.re;
+          rp.im += p_ * u1.im;
+          t1.re += ta * u1.re;
+          t1.im += ta * u1.im;
+          t0.re += ta * u0.re;
+          t0.im += ta * u0.im;
+          q1.re += mpi * v1.re;
+          q1.im += mpi * v1.im;
+          q0.re += mpi * v0.re;
+          q0.im += mpi * v0.im;
+        }
+        const Real pf = (Real)(1.0 / sqrt(2.0 * l * (l + 1)));
+        const Z hx = cmul(h[l], ix);
+        const C A = cscale(h[l], pf), Bv = cscale(hx, pf * Real(l * (l + 1)));
+        const C Cv = cscale(csub(h[l - 1], cscale(hx, Real(l))), pf);
+        er.re += Bv.re * rp.re - Bv.im * rp.im;
+        er.im += Bv.re * rp.im + Bv.im * rp.re;
+        // e_theta: A i q0 + Cv t1; e_phi: -A t0 + Cv i q1
+        et.re += Cv.re * t1.re - Cv.im * t1.im - A.re * q0.im - A.im * q0.re;
+        et.im += Cv.re * t1.im + Cv.im * t1.re + A.re * q0.re - A.im * q0.im;
+        ep.re -= Cv.re * q1.im + Cv.im * q1.re + A.re * t0.re - A.im * t0.im;
+        ep.im += Cv.re * q1.re - Cv.im * q1.im - A.re * t0.im - A.im * t0.re;
+      }
+      const Real stc = st * cp, sts = st * sn, ctc = ct * cp, cts = ct * sn;
+      ex.re += er.re * stc + et.re * ctc - ep.re * sn;
+      ex.im += er.im * stc + et.im * ctc - ep.im * sn;
+      ey.re += er.re * sts + et.re * cts + ep.re * cp;
+      ey.im += er.im * sts + et.im * cts + ep.im * cp;
+      ez.re += er.re * ct - et.re * st;
+      ez.im += er.im * ct - et.im * st;
     }
   }
   if (live) {
-    a.out[ip] = make_double2((double)ex.re, (double)ex.im);
-    a.out[a.n_pts + ip] = make_double2((double)ey.re, (double)ey.im);
-    a.out[2 * a.n_pts + ip] = make_double2((double)ez.re, (double)ez.im);
+    C* out = reinterpret_cast<C*>(a.out) + 3 * (int64_t)blockIdx.y * a.n_pts + ip;
+    out[0] = ex;
+    out[a.n_pts] = ey;
+    out[2 * a.n_pts] = ez;
   }
+}
+
+// out[j] = sum over the splits' partial fields, in FP64 and in their order
+template <typename Real>
+__global__ void swe_sum_kernel(const cplx<Real>* __restrict__ part, int splits, int64_t count, double2* out) {
+  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= count) return;
+  double re = 0, im = 0;
+#pragma unroll 4
+  for (int q = 0; q < splits; ++q) {
+    const cplx<Real> v = part[q * count + j];
+    re += (double)v.re;
+    im += (double)v.im;
+  }
+  out[j] = make_double2(re, im);
 }
 
 // Any (l_max, m_max): the same sum with runtime orders. Per (point,
@@ -239,8 +283,10 @@ __global__ void __launch_bounds__(kSwePoints) swe_field_any_kernel(SweArgs a, in
     pz = a.pts[3 * ip + 2];
   }
   C ex{0, 0}, ey{0, 0}, ez{0, 0};
-  for (int64_t p0 = 0; p0 < a.n_part; p0 += chunk) {
-    const int np = (int)(a.n_part - p0 < chunk ? a.n_part - p0 : chunk);
+  const int64_t first = (int64_t)blockIdx.y * a.per_split;
+  const int64_t last = first + a.per_split < a.n_part ? first + a.per_split : a.n_part;
+  for (int64_t p0 = first; p0 < last; p0 += chunk) {
+    const int np = (int)(last - p0 < chunk ? last - p0 : chunk);
     __syncthreads();
     for (int j = threadIdx.x; j < np * 6; j += kSwePoints) sp[j] = a.part[p0 * 6 + j];
     for (int j = threadIdx.x; j < np * B; j += kSwePoints) {
@@ -374,9 +420,10 @@ __global__ void __launch_bounds__(kSwePoints) swe_field_any_kernel(SweArgs a, in
     }
   }
   if (live) {
-    a.out[ip] = make_double2((double)ex.re, (double)ex.im);
-    a.out[a.n_pts + ip] = make_double2((double)ey.re, (double)ey.im);
-    a.out[2 * a.n_pts + ip] = make_double2((double)ez.re, (double)ez.im);
+    C* out = reinterpret_cast<C*>(a.out) + 3 * (int64_t)blockIdx.y * a.n_pts + ip;
+    out[0] = ex;
+    out[a.n_pts] = ey;
+    out[2 * a.n_pts] = ez;
   }
 }
 
@@ -439,19 +486,42 @@ extern "C" int smh_swe_field(smh_ctx* ctx, int64_t n_part, const double* pos, co
     part[6 * p + 3] = radius[p] * radius[p];
     part[6 * p + 4] = zlim[2 * p];
     part[6 * p + 5] = zlim[2 * p + 1];
-    for (int n = 0; n < B; ++n) {
-      const int src = field == 0 ? n : (n < half ? n + half : n - half);
-      cf[2 * ((size_t)p * B + n)] = coef[2 * ((size_t)p * B + src)];
-      cf[2 * ((size_t)p * B + n) + 1] = coef[2 * ((size_t)p * B + src) + 1];
+    const std::complex<double>* b = reinterpret_cast<const std::complex<double>*>(coef) + (size_t)p * B;
+    std::complex<double>* c = reinterpret_cast<std::complex<double>*>(cf.data()) + (size_t)p * B;
+    auto src = [&](int n) { return b[field == 0 ? n : (n < half ? n + half : n - half)]; };
+    if (!fn) {
+      for (int n = 0; n < B; ++n) c[n] = src(n);
+      continue;
     }
+    for (int tau = 0; tau < 2; ++tau)
+      for (int l = 1; l <= l_max; ++l)
+        for (int m = 0; m <= std::min(l, m_max); ++m) {
+          const int o = swe_pair_offset(l, m, m_max);
+          const std::complex<double> bp = src(swe_index(tau, l, m, l_max, m_max));
+          if (m == 0) {
+            c[o + tau] = bp;
+          } else {
+            const std::complex<double> bn = src(swe_index(tau, l, -m, l_max, m_max));
+            c[o + 2 * tau] = bp + bn;
+            c[o + 2 * tau + 1] = bp - bn;
+          }
+        }
   }
-  void* buf[4] = {nullptr, nullptr, nullptr, nullptr};
-  const size_t sizes[4] = {part.size() * 8, cf.size() * 8, (size_t)3 * n_pts * 8, (size_t)3 * n_pts * 16};
+  // particles split so that about eight workgroups a CU run (256 x 8; a split sums at least kSweChunk particles)
+  const unsigned nb = (unsigned)((n_pts + kSwePoints - 1) / kSwePoints);
+  const int64_t want = std::max<int64_t>(1, std::min<int64_t>((8 * (int64_t)ctx->num_cu + nb - 1) / nb,
+                                                              (n_part + kSweChunk - 1) / kSweChunk));
+  const int64_t per_split = (n_part + want - 1) / want;
+  const int splits = (int)((n_part + per_split - 1) / per_split);
+  const size_t csize = precision == SMH_FP32 ? sizeof(float2) : sizeof(double2);
+  void* buf[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+  const size_t sizes[5] = {part.size() * 8, cf.size() * 8, (size_t)3 * n_pts * 8, (size_t)3 * n_pts * 16,
+                           (size_t)splits * 3 * n_pts * csize};
   auto release = [&]() {
     for (void* q : buf)
       if (q) hipFree(q);
   };
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 5; ++i)
     if (hipMalloc(&buf[i], sizes[i]) != hipSuccess) {
       release();
       return smh_fail(ctx, SMH_ERR_HIP, "SWE field device allocation failed");
@@ -467,13 +537,12 @@ extern "C" int smh_swe_field(smh_ctx* ctx, int64_t n_part, const double* pos, co
   a.part = (const double*)buf[0];
   a.coef = (const double2*)buf[1];
   a.pts = (const double*)buf[2];
-  a.out = (double2*)buf[3];
+  a.out = buf[4];
   a.n_part = n_part;
   a.n_pts = n_pts;
+  a.per_split = per_split;
   a.k_re = k_re;
   a.k_im = k_im;
-  const unsigned nb = (unsigned)((n_pts + kSwePoints - 1) / kSwePoints);
-  const size_t csize = precision == SMH_FP32 ? sizeof(float2) : sizeof(double2);
   int lmax_ = l_max, mmax_ = m_max, B_ = B;
   int chunk = (int)std::min<size_t>(32, 65536 / (6 * sizeof(double) + (size_t)B * csize));
   const size_t lds = fn ? 0 : (size_t)chunk * (6 * sizeof(double) + (size_t)B * csize);
@@ -484,7 +553,17 @@ extern "C" int smh_swe_field(smh_ctx* ctx, int64_t n_part, const double* pos, co
   void* args_fixed[] = {&a};
   void* args_any[] = {&a, &lmax_, &mmax_, &B_, &chunk};
   if (e == hipSuccess)
-    e = hipLaunchKernel(fn, dim3(nb), dim3(kSwePoints), lds ? args_any : args_fixed, lds, s);
+    e = hipLaunchKernel(fn, dim3(nb, (unsigned)splits), dim3(kSwePoints), lds ? args_any : args_fixed, lds, s);
+  if (e == hipSuccess) {
+    const unsigned sb = (unsigned)((3 * n_pts + 255) / 256);
+    if (precision == SMH_FP32)
+      hipLaunchKernelGGL(swe_sum_kernel<float>, dim3(sb), dim3(256), 0, s, (const cplx<float>*)buf[4], splits,
+                         3 * n_pts, (double2*)buf[3]);
+    else
+      hipLaunchKernelGGL(swe_sum_kernel<double>, dim3(sb), dim3(256), 0, s, (const cplx<double>*)buf[4], splits,
+                         3 * n_pts, (double2*)buf[3]);
+    e = hipGetLastError();
+  }
   if (e == hipSuccess) e = hipEventRecord(ctx->ev1, s);
   if (e == hipSuccess) e = hipMemcpyAsync(out, buf[3], sizes[3], hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
