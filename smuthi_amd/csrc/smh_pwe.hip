@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "smh_common.h"
+#include "smh_radial_kernel.h"
 
 namespace {
 
@@ -148,7 +149,8 @@ __global__ void __launch_bounds__(kLeaf) pwe_field_kernel(PweArgs a) {
 
 // Recursive median split of idx[b, e) along the widest extent into leaves of
 // at most `leaf` points.
-void split_leaves(const double* xyz, std::vector<int>& idx, int b, int e, std::vector<int>& bounds, int leaf = kLeaf) {
+void split_leaves(const double* xyz, std::vector<int>& idx, int b, int e, std::vector<int>& bounds) {
+  constexpr int leaf = kLeaf;
   if (e - b <= leaf) {
     bounds.push_back(e);
     return;
@@ -167,8 +169,8 @@ void split_leaves(const double* xyz, std::vector<int>& idx, int b, int e, std::v
   const int mid = std::min(e - 1, b + half);
   std::nth_element(idx.begin() + b, idx.begin() + mid, idx.begin() + e,
                    [&](int u, int v) { return xyz[3 * u + dim] < xyz[3 * v + dim]; });
-  split_leaves(xyz, idx, b, mid, bounds, leaf);
-  split_leaves(xyz, idx, mid, e, bounds, leaf);
+  split_leaves(xyz, idx, b, mid, bounds);
+  split_leaves(xyz, idx, mid, e, bounds);
 }
 
 }  // namespace
@@ -327,157 +329,189 @@ extern "C" int smh_pwe_field(smh_ctx* ctx, int kind, int64_t n_k, const double* 
 // c_{p,m,pol,dir} = sum_{tau,l} b_{p,tau l m} B_{tau l m,pol}(+-kz/k, kappa/k) / (2 pi kz k)
 // (swe_to_pwe_conversion, fields/transformations.py:133-226, summed over the
 // particles of one layer as scattered_field_pwe, postprocessing/scattered_field.py:80-150).
-// One workgroup per kappa, one thread per alpha; particles are taken leaf by
-// leaf, their c staged in LDS; the leaf centre's phase is applied in FP64.
-// A launch covers NM consecutive orders m (its accumulators live in
-// registers); more than kAsmOrders orders run as several launches, each adding
-// its orders' share into g.
+// Per kappa this is a complex matrix product over the particles, phases
+// [alpha][particle] times coefficients [particle][(m, pol, dir)], on the MFMA
+// 16x16x4 (FP32 or FP64): a wave holds kAsmTiles tiles of 16 alpha, its lanes
+// compute one phase each per four particles (no phase twice), and the
+// coefficients of a chunk of particles, e^{+-i kz (z_ref - z)} included, are
+// staged in LDS by the workgroup. The phase's argument is formed and reduced to
+// a revolution in FP64 (FP32: then native sine and cosine). The particles are
+// split over workgroups until the chip is filled (a far field of 90 polar
+// angles, or the one direction of an extinction cross section, has too few
+// kappa for that); a second kernel adds the splits' sums in FP64. Bound by the
+// FP64 sincos of the phases (about 60 instructions per particle and alpha)
+// beside as much time in the MFMA: 90 x 361 waves, 1000 particles, l_max 3, FP64:
+// 1.34 ms when a thread summed all orders of one alpha in registers.
+// A launch covers kAsmOrders orders m at most; more run as several launches,
+// each adding its orders' share into g.
 namespace {
 
-constexpr int kAsmLeaf = 128;
-constexpr int kAsmOrders = 9;  // orders per launch (m_max <= 4 in one launch)
+constexpr int kAsmChunk = 32;   // particles staged at a time
+constexpr int kAsmTiles = 2;    // alpha tiles per wave
+constexpr int kAsmWaves = 4;
+constexpr int kAsmOrders = 12;  // orders per launch: 4 (dir, pol) each in 3 column tiles
 
 struct AsmArgs {
-  const double* pts;    // [n_part][3], leaf order
-  const double2* coef;  // [n_part][B], leaf order
-  const int* leaf;      // [n_leaves + 1]
-  const double* ctr;    // [n_leaves][2] leaf centres (x, y)
+  const double* pts;    // [n_part][3]
+  const double2* coef;  // [n_part][B]
   const double2* kp;    // [n_k]
   const double2* kz;    // [n_k] upgoing kz
   const double2* btab;  // [n_k][2 dir][2 pol][B], 1 / (2 pi kz k) included
   const int* nlist;     // [NM][LM] multipole indices n of order m = j + m_first (-1: none)
   const double* alpha;  // [n_a]
-  double2* g;           // [2 dir][2 pol][n_k][n_a]
+  double2* part;        // [splits][2 dir][2 pol][n_k][n_a]
   double z_ref;
-  int B, LM, n_leaves, n_k, n_a;
-  int m_first;     // order of the launch's first row of nlist
-  int accumulate;  // add into g (later launches of a chunked order range)
+  int64_t n_part;
+  int B, LM, NM, n_k, n_a;
+  int per_split;        // particles per blockIdx.y
+  unsigned a_blocks;    // alpha blocks per kappa (blockIdx.x = kappa * a_blocks + block)
+  int m_first;          // order of the launch's first row of nlist
 };
 
-template <typename Real, int NM>
-__global__ void __launch_bounds__(256) pwe_assemble_kernel(AsmArgs a) {
-  using M = PweMath<Real>;
-  constexpr int Q = 4;  // (dir, pol)
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  Real* cl = reinterpret_cast<Real*>(smem_raw);  // [kAsmLeaf][NM][Q][2]
-  Real* dxy = cl + (size_t)kAsmLeaf * NM * Q * 2;  // [kAsmLeaf][2]
-  const int k = blockIdx.x, tid = threadIdx.x;
-  const int ia = blockIdx.y * blockDim.x + tid;
-  const bool active = ia < a.n_a;
-  const double al = active ? a.alpha[ia] : 0.0;
-  const double cad = cos(al), sad = sin(al);
-  const Real ca = (Real)cad, sa = (Real)sad;
-  const double2 kp = a.kp[k], kzu = a.kz[k];
-  const Real kr = (Real)(-kp.x / kTwoPi);   // e^{-i kappa s}: revolutions per nm
-  const Real ki = (Real)(kp.y * kLog2e);    // |e^{-i kappa s}| = 2^(ki s)
+// e^{i 2 pi t} for any t
+__device__ inline void cis_turns(double t, double& c, double& s) { sincospi(2.0 * (t - rint(t)), &s, &c); }
+__device__ inline void cis_turns(double t, float& c, float& s) { PweMath<float>::cis_rev((float)(t - rint(t)), c, s); }
+
+// CT: tiles of 16 columns (m, q), q = (dir, pol), of the real and of the imaginary parts
+template <typename Real, int CT>
+__global__ void __launch_bounds__(64 * kAsmWaves) pwe_assemble_kernel(AsmArgs a) {
+  using M = smh::Mfma<Real>;
+  constexpr int Q = 4, SC = CT * 16 + 16;  // (the row stride puts neighbouring particles in other banks)
+  __shared__ Real cr[kAsmChunk][SC], ci[kAsmChunk][SC];
+  __shared__ double px[kAsmChunk], py[kAsmChunk];
+  __shared__ double2 ez[kAsmChunk][2];
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, h = lane >> 4;
+  const int k = (int)(blockIdx.x / a.a_blocks), ab = (int)(blockIdx.x - k * a.a_blocks);
+  const int tile0 = (ab * (int)(blockDim.x >> 6) + (tid >> 6)) * kAsmTiles;
+  const double2 kp = a.kp[k], kz = a.kz[k];
+  const double kturn = -kp.x / kTwoPi;        // e^{-i kappa s}: turns per nm
+  const Real klog = (Real)(kp.y * kLog2e);    // |e^{-i kappa s}| = 2^(klog s)
   const bool lossy = kp.y != 0.0;
-  Real U[NM][Q][2];
+  // this lane's alpha of each tile
+  double ca[kAsmTiles], sa[kAsmTiles];
 #pragma unroll
-  for (int m = 0; m < NM; ++m)
+  for (int t = 0; t < kAsmTiles; ++t) {
+    const int ia = (tile0 + t) * 16 + c;
+    sincos(ia < a.n_a ? a.alpha[ia] : 0.0, &sa[t], &ca[t]);
+  }
+  typename M::v4 ar[kAsmTiles][CT], ai[kAsmTiles][CT];
 #pragma unroll
-    for (int q = 0; q < Q; ++q) U[m][q][0] = U[m][q][1] = Real(0);
-  for (int l = 0; l < a.n_leaves; ++l) {
-    const int p0 = a.leaf[l], np = a.leaf[l + 1] - p0;
-    const double X = a.ctr[2 * l], Y = a.ctr[2 * l + 1];
+  for (int t = 0; t < kAsmTiles; ++t)
+#pragma unroll
+    for (int j = 0; j < CT; ++j) ar[t][j] = ai[t][j] = typename M::v4{0, 0, 0, 0};
+  const int64_t first = (int64_t)blockIdx.y * a.per_split;
+  const int64_t last = first + a.per_split < a.n_part ? first + a.per_split : a.n_part;
+  for (int64_t p0 = first; p0 < last; p0 += kAsmChunk) {
+    const int np = (int)(last - p0 < kAsmChunk ? last - p0 : kAsmChunk);
     __syncthreads();
-    for (int w = tid; w < np * NM; w += blockDim.x) {
-      const int pl = w / NM, m = w - pl * NM, p = p0 + pl;
-      const double zp = a.pts[3 * p + 2];
+    for (int p = tid; p < kAsmChunk; p += blockDim.x) {
+      const bool on = p < np;
+      px[p] = on ? a.pts[3 * (p0 + p)] : 0.0;
+      py[p] = on ? a.pts[3 * (p0 + p) + 1] : 0.0;
       // e^{i kz (z_ref - z_p)} (up) and e^{-i kz (z_ref - z_p)} (down)
-      const double dz = a.z_ref - zp;
+      const double dz = on ? a.z_ref - a.pts[3 * (p0 + p) + 2] : 0.0;
       double su, cu;
-      sincos(kzu.x * dz, &su, &cu);
-      const double mu = exp(-kzu.y * dz), md = exp(kzu.y * dz);
-      const double2 ph[2] = {make_double2(mu * cu, mu * su), make_double2(md * cu, -md * su)};
-      double cr[Q] = {0, 0, 0, 0}, ci[Q] = {0, 0, 0, 0};
-      for (int j = 0; j < a.LM; ++j) {
-        const int n = a.nlist[m * a.LM + j];
-        if (n < 0) break;
-        const double2 b = a.coef[(size_t)p * a.B + n];
-        for (int q = 0; q < Q; ++q) {
-          const double2 t = a.btab[((size_t)k * Q + q) * a.B + n];
-          cr[q] += b.x * t.x - b.y * t.y;
-          ci[q] += b.x * t.y + b.y * t.x;
-        }
-      }
-      Real* dst = cl + ((size_t)pl * NM + m) * Q * 2;
-      for (int q = 0; q < Q; ++q) {
-        const double2 e = ph[q >> 1];
-        dst[2 * q] = (Real)(cr[q] * e.x - ci[q] * e.y);
-        dst[2 * q + 1] = (Real)(cr[q] * e.y + ci[q] * e.x);
-      }
-      if (m == 0) {
-        dxy[2 * pl] = (Real)(a.pts[3 * p] - X);
-        dxy[2 * pl + 1] = (Real)(a.pts[3 * p + 1] - Y);
-      }
+      sincos(kz.x * dz, &su, &cu);
+      const double mu = exp(-kz.y * dz), md = exp(kz.y * dz);
+      ez[p][0] = make_double2(mu * cu, mu * su);
+      ez[p][1] = make_double2(md * cu, -md * su);
     }
     __syncthreads();
-    Real S[NM][Q][2];
-#pragma unroll
-    for (int m = 0; m < NM; ++m)
-#pragma unroll
-      for (int q = 0; q < Q; ++q) S[m][q][0] = S[m][q][1] = Real(0);
-    for (int pl = 0; pl < np; ++pl) {
-      const Real s = dxy[2 * pl] * ca + dxy[2 * pl + 1] * sa;
-      Real pc, ps;
-      M::cis_rev(kr * s, pc, ps);
-      if (lossy) {
-        const Real mg = M::exp2_(ki * s);
-        pc *= mg;
-        ps *= mg;
-      }
-      const Real* c = cl + (size_t)pl * NM * Q * 2;
-#pragma unroll
-      for (int m = 0; m < NM; ++m)
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-          const Real xr = c[(m * Q + q) * 2], xi = c[(m * Q + q) * 2 + 1];
-          S[m][q][0] += xr * pc - xi * ps;
-          S[m][q][1] += xr * ps + xi * pc;
+    for (int w = tid; w < kAsmChunk * CT * 16; w += blockDim.x) {
+      const int p = w / (CT * 16), col = w - p * (CT * 16), m = col >> 2, q = col & 3;
+      double re = 0, im = 0;
+      if (p < np && m < a.NM) {
+        for (int j = 0; j < a.LM; ++j) {
+          const int n = a.nlist[m * a.LM + j];
+          if (n < 0) break;
+          const double2 b = a.coef[(p0 + p) * a.B + n], t = a.btab[((size_t)k * Q + q) * a.B + n];
+          re += b.x * t.x - b.y * t.y;
+          im += b.x * t.y + b.y * t.x;
         }
-    }
-    // leaf centre phase e^{-i kappa (X cos a + Y sin a)} in FP64
-    const double sc = X * cad + Y * sad;
-    double sn, cn;
-    sincos(-kp.x * sc, &sn, &cn);
-    const double mg = exp(kp.y * sc);
-    const Real lr = (Real)(mg * cn), li = (Real)(mg * sn);
-#pragma unroll
-    for (int m = 0; m < NM; ++m)
-#pragma unroll
-      for (int q = 0; q < Q; ++q) {
-        U[m][q][0] += S[m][q][0] * lr - S[m][q][1] * li;
-        U[m][q][1] += S[m][q][0] * li + S[m][q][1] * lr;
+        const double2 e = ez[p][q >> 1];
+        const double r = re * e.x - im * e.y;
+        im = re * e.y + im * e.x;
+        re = r;
       }
-  }
-  if (!active) return;
-  for (int q = 0; q < Q; ++q) {
-    double gr = 0, gi = 0;
+      cr[p][col] = (Real)re;
+      ci[p][col] = (Real)im;
+    }
+    __syncthreads();
+    if (tile0 * 16 >= a.n_a) continue;
+    for (int s = 0; s < (np + 3) / 4; ++s) {
+      const int p = 4 * s + h;  // (particles beyond np have zero coefficients)
+      Real br[CT], bi[CT];
 #pragma unroll
-    for (int m = 0; m < NM; ++m) {
-      double em_s, em_c;
-      sincos((double)(m + a.m_first) * al, &em_s, &em_c);
-      gr += (double)U[m][q][0] * em_c - (double)U[m][q][1] * em_s;
-      gi += (double)U[m][q][0] * em_s + (double)U[m][q][1] * em_c;
+      for (int j = 0; j < CT; ++j) {
+        br[j] = cr[p][16 * j + c];
+        bi[j] = ci[p][16 * j + c];
+      }
+#pragma unroll
+      for (int t = 0; t < kAsmTiles; ++t) {
+        const double sd = px[p] * ca[t] + py[p] * sa[t];
+        Real pr, pi;
+        cis_turns(kturn * sd, pr, pi);
+        if (lossy) {
+          const Real mg = PweMath<Real>::exp2_(klog * (Real)sd);
+          pr *= mg;
+          pi *= mg;
+        }
+#pragma unroll
+        for (int j = 0; j < CT; ++j) {
+          ar[t][j] = M::op(pr, br[j], ar[t][j]);
+          ai[t][j] = M::op(pr, bi[j], ai[t][j]);
+          ar[t][j] = M::op(pi, -bi[j], ar[t][j]);
+          ai[t][j] = M::op(pi, br[j], ai[t][j]);
+        }
+      }
     }
-    double2* dst = a.g + ((size_t)q * a.n_k + k) * a.n_a + ia;
-    if (a.accumulate) {
-      const double2 o = *dst;
-      gr += o.x;
-      gi += o.y;
-    }
-    *dst = make_double2(gr, gi);
   }
+  // sum over m of e^{i m alpha}: the lane's columns of each alpha, then the lanes of the same q
+#pragma unroll
+  for (int t = 0; t < kAsmTiles; ++t)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int ia = (tile0 + t) * 16 + (M::kRowIs4q ? 4 * h + v : 4 * v + h);
+      const double al = ia < a.n_a ? a.alpha[ia] : 0.0;
+      double gr = 0, gi = 0;
+#pragma unroll
+      for (int j = 0; j < CT; ++j) {
+        double es, ec;
+        sincos((double)(4 * j + (c >> 2) + a.m_first) * al, &es, &ec);
+        gr += (double)ar[t][j][v] * ec - (double)ai[t][j][v] * es;
+        gi += (double)ar[t][j][v] * es + (double)ai[t][j][v] * ec;
+      }
+#pragma unroll
+      for (int off = 4; off < 16; off <<= 1) {
+        gr += __shfl_xor(gr, off);
+        gi += __shfl_xor(gi, off);
+      }
+      if (c < Q && ia < a.n_a)
+        a.part[(((size_t)blockIdx.y * Q + c) * a.n_k + k) * a.n_a + ia] = make_double2(gr, gi);
+    }
+}
+
+// g = sum of the splits in order (g += it for the later launches of a chunked order range)
+__global__ void pwe_sum_kernel(const double2* __restrict__ part, int splits, int64_t count, int accumulate,
+                               double2* g) {
+  const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (j >= count) return;
+  double2 s = accumulate ? g[j] : make_double2(0.0, 0.0);
+#pragma unroll 4
+  for (int q = 0; q < splits; ++q) {
+    const double2 v = part[q * count + j];
+    s.x += v.x;
+    s.y += v.y;
+  }
+  g[j] = s;
 }
 
 template <typename Real>
 void* assemble_kernel_for(int nm) {
-  switch (nm) {
-    case 3: return reinterpret_cast<void*>(&pwe_assemble_kernel<Real, 3>);
-    case 5: return reinterpret_cast<void*>(&pwe_assemble_kernel<Real, 5>);
-    case 7: return reinterpret_cast<void*>(&pwe_assemble_kernel<Real, 7>);
-    case 9: return reinterpret_cast<void*>(&pwe_assemble_kernel<Real, 9>);
-    default: return nullptr;
+  switch ((4 * nm + 15) / 16) {
+    case 1: return reinterpret_cast<void*>(&pwe_assemble_kernel<Real, 1>);
+    case 2: return reinterpret_cast<void*>(&pwe_assemble_kernel<Real, 2>);
+    default: return reinterpret_cast<void*>(&pwe_assemble_kernel<Real, 3>);
   }
 }
 
@@ -512,46 +546,34 @@ extern "C" int smh_pwe_assemble(smh_ctx* ctx, int64_t n_part, const double* xyz,
         nlist[(size_t)j * LM + fill[j]++] = smh_multi_to_single(tau, l, m, l_max, m_max);
       }
     }
-  // particle leaves
-  std::vector<int> idx(n_part);
-  std::iota(idx.begin(), idx.end(), 0);
-  std::vector<int> bounds{0};
-  split_leaves(xyz, idx, 0, (int)n_part, bounds, kAsmLeaf);
-  const int n_leaves = (int)bounds.size() - 1;
-  std::vector<double> pts((size_t)3 * n_part), ctr((size_t)2 * n_leaves);
-  std::vector<double> cf((size_t)2 * n_part * B);
-  for (int64_t j = 0; j < n_part; ++j) {
-    for (int d = 0; d < 3; ++d) pts[3 * j + d] = xyz[3 * (size_t)idx[j] + d];
-    std::memcpy(&cf[(size_t)2 * j * B], &coef[(size_t)2 * idx[j] * B], sizeof(double) * 2 * B);
-  }
-  for (int l = 0; l < n_leaves; ++l) {
-    double lo[2] = {1e300, 1e300}, hi[2] = {-1e300, -1e300};
-    for (int j = bounds[l]; j < bounds[l + 1]; ++j)
-      for (int d = 0; d < 2; ++d) {
-        lo[d] = std::min(lo[d], pts[3 * j + d]);
-        hi[d] = std::max(hi[d], pts[3 * j + d]);
-      }
-    ctr[2 * l] = 0.5 * (lo[0] + hi[0]);
-    ctr[2 * l + 1] = 0.5 * (lo[1] + hi[1]);
-  }
-  const size_t rs = precision == SMH_FP32 ? sizeof(float) : sizeof(double);
-  const size_t lds = (size_t)kAsmLeaf * NM * 4 * 2 * rs + (size_t)kAsmLeaf * 2 * rs;
-  void* buf[10] = {nullptr};
-  const size_t sizes[10] = {pts.size() * 8, cf.size() * 8, bounds.size() * 4, ctr.size() * 8,
-                            (size_t)n_k * 16, (size_t)n_k * 16, (size_t)n_k * 4 * B * 16, nlist.size() * 4,
-                            (size_t)n_a * 8, (size_t)4 * n_k * n_a * 16};
+  // waves of a workgroup: no more than the alpha tiles ask for
+  const int64_t tiles = (n_a + 15) / 16;
+  const int waves = (int)std::min<int64_t>(kAsmWaves, (tiles + kAsmTiles - 1) / kAsmTiles);
+  const int threads = 64 * waves;
+  const unsigned a_blocks = (unsigned)((tiles + waves * kAsmTiles - 1) / (waves * kAsmTiles));
+  // splits of the particles: about eight workgroups per CU, whole chunks each
+  const int64_t blocks = n_k * a_blocks, chunks = (n_part + kAsmChunk - 1) / kAsmChunk;
+  const int64_t want = std::max<int64_t>(1, std::min<int64_t>((8 * (int64_t)ctx->num_cu + blocks - 1) / blocks, chunks));
+  const int per_split = (int)((chunks + want - 1) / want) * kAsmChunk;
+  const int splits = (int)((n_part + per_split - 1) / per_split);
+  const int64_t count = 4 * n_k * n_a;
+  SMH_CHECK(ctx, blocks < ((int64_t)1 << 31), SMH_ERR_ARG, "invalid sizes");
+  void* buf[9] = {nullptr};
+  const size_t sizes[9] = {(size_t)n_part * 24, (size_t)n_part * B * 16, (size_t)n_k * 16, (size_t)n_k * 16,
+                           (size_t)n_k * 4 * B * 16, nlist.size() * 4, (size_t)n_a * 8, (size_t)count * 16,
+                           (size_t)splits * count * 16};
   auto release = [&]() {
     for (void* b : buf)
       if (b) hipFree(b);
   };
-  for (int i = 0; i < 10; ++i)
+  for (int i = 0; i < 9; ++i)
     if (hipMalloc(&buf[i], sizes[i]) != hipSuccess) {
       release();
       return smh_fail(ctx, SMH_ERR_HIP, "PWE assembly allocation failed");
     }
   hipStream_t s = ctx->stream;
-  const void* src[9] = {pts.data(), cf.data(), bounds.data(), ctr.data(), kp, kz, btab, nlist.data(), alpha};
-  for (int i = 0; i < 9; ++i)
+  const void* src[7] = {xyz, coef, kp, kz, btab, nlist.data(), alpha};
+  for (int i = 0; i < 7; ++i)
     if (hipMemcpyAsync(buf[i], src[i], sizes[i], hipMemcpyHostToDevice, s) != hipSuccess) {
       release();
       return smh_fail(ctx, SMH_ERR_HIP, "PWE assembly upload failed");
@@ -559,35 +581,34 @@ extern "C" int smh_pwe_assemble(smh_ctx* ctx, int64_t n_part, const double* xyz,
   AsmArgs a;
   a.pts = (const double*)buf[0];
   a.coef = (const double2*)buf[1];
-  a.leaf = (const int*)buf[2];
-  a.ctr = (const double*)buf[3];
-  a.kp = (const double2*)buf[4];
-  a.kz = (const double2*)buf[5];
-  a.btab = (const double2*)buf[6];
-  a.nlist = (const int*)buf[7];
-  a.alpha = (const double*)buf[8];
-  a.g = (double2*)buf[9];
+  a.kp = (const double2*)buf[2];
+  a.kz = (const double2*)buf[3];
+  a.btab = (const double2*)buf[4];
+  a.alpha = (const double*)buf[6];
+  a.part = (double2*)buf[8];
+  a.per_split = per_split;
+  a.a_blocks = a_blocks;
   a.z_ref = z_ref;
+  a.n_part = n_part;
   a.B = B;
   a.LM = LM;
-  a.n_leaves = n_leaves;
+  a.NM = NM;
   a.n_k = (int)n_k;
   a.n_a = (int)n_a;
   void* kfn = precision == SMH_FP32 ? assemble_kernel_for<float>(NM) : assemble_kernel_for<double>(NM);
-  const int threads = (int)std::min<int64_t>(256, (n_a + 63) / 64 * 64);
-  const unsigned a_blocks = (unsigned)((n_a + threads - 1) / threads);
-  hipError_t e = hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (e == hipSuccess) e = hipEventRecord(ctx->ev0, s);
+  hipError_t e = hipEventRecord(ctx->ev0, s);
   void* args[] = {&a};
-  const int* nlist_dev = a.nlist;
   for (int c = 0; c < n_chunks && e == hipSuccess; ++c) {
-    a.nlist = nlist_dev + (size_t)c * NM * LM;
+    a.nlist = (const int*)buf[5] + (size_t)c * NM * LM;
     a.m_first = c * NM - m_max;
-    a.accumulate = c > 0;
-    e = hipLaunchKernel(kfn, dim3((unsigned)n_k, a_blocks), dim3(threads), args, lds, s);
+    e = hipLaunchKernel(kfn, dim3((unsigned)blocks, (unsigned)splits), dim3(threads), args, 0, s);
+    if (e != hipSuccess) break;
+    hipLaunchKernelGGL(pwe_sum_kernel, dim3((unsigned)((count + 255) / 256)), dim3(256), 0, s,
+                       (const double2*)buf[8], splits, count, c > 0 ? 1 : 0, (double2*)buf[7]);
+    e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipEventRecord(ctx->ev1, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(g, buf[9], sizes[9], hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipMemcpyAsync(g, buf[7], sizes[7], hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   float ms = 0;
   if (e == hipSuccess) e = hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1);
