@@ -828,12 +828,12 @@ def main_batching(args):
         'speedup_vs_fp64_gmres_batched': value * fp64_s / systems_per_step,
         'matvec_ms': {'fp16_8rhs_all_ensembles': k16, 'fp32_8rhs_all_ensembles': k32, 'fp32_8rhs_total': tot32,
                       'fp64_8rhs_all_ensembles': k64, 'fp64_8rhs_total': tot64},
-        'roofline': {'bound': ('mfma by the algorithmic count; in practice the tap rows: about one pair per '
-                               '(receiver chunk, rho, z) cell, so each pair reads its 16 tap rows per table'),
+        'roofline': {'bound': ('mfma by the algorithmic count; in practice the tap rows: each unit of two pairs '
+                               'reads its 16 tap rows per table from the L2'),
                      'achieved': achieved, 'peak': peak_inner, 'unit': 'TFLOP/s', 'frac': achieved / peak_inner,
                      'traffic': None,
-                     'kernel': ('batch_half_kernel<3,3,4,true>' if half else 'batch_slots_kernel<3,3,4,true>') +
-                               ' (8 launches: 2 tables x 4 z slices)',
+                     'kernel': ('vol_half_kernel<3,3>' if half else 'vol_slots_kernel<3,3>') +
+                               ' (per table and slab of pairs)',
                      'flops_per_matvec': flops},
         'table_seconds': batch.table_seconds, 'setup_seconds': prep, 'autotune': tune,
         'device': dev, 'compute_units': n_cu,

@@ -75,6 +75,13 @@ struct smh_op {
     const float* lsum_rows = nullptr;
     int lsum_T = 0, lsum_vmode = 0, lsum_len_z = 0;
     size_t part_bytes = 0;  // partial-result bytes one work item writes (d_ypart holds n_items of them)
+    // volume kBatch-RHS kernels: slabs of neighbouring bins take the place of
+    // receiver chunks; pairs [slab_pair[s], slab_pair[s+1]) are slab s, and
+    // recv_pair[recv_off[s n_part + i] ..) are receiver i's pairs in it, in
+    // sender order
+    std::vector<int> slab_pair;
+    int *d_recv_off = nullptr, *d_recv_pair = nullptr;
+    int* d_xcd_bounds = nullptr;  // the XCDs' shares of each slab's entries (VolWalk)
   } bin[2];
   Binning bbin[2];  // the same pairs binned for the kBatch-RHS kernel (smaller receiver chunks)
   int64_t n_pairs = 0;
@@ -92,7 +99,8 @@ struct smh_op {
   int vmode = 1, vq = 1;  // interpolation mode (vol_tap_offset) and tap rows per (rho, z) node
   float* d_vrowsum[2] = {nullptr, nullptr};
   Binning vbin[2][2];
-  Binning vbbin[2][2];  // the same pairs binned for the kBatch-RHS kernel
+  Binning vbbin[2][2];  // the same pairs in slabs for the kBatch-RHS kernels
+  double* d_vacc = nullptr;  // their receiver sums over slabs and tables, [n_part][16 S]
 
   // explicit operator: dense W [n_part * B][n_part * B] on padded vectors
   double2* d_W64 = nullptr;

@@ -918,11 +918,12 @@ void smh_op_free(smh_op* op) {
     if (p) hipFree(p);
   void* ptrs[] = {op->d_xy, op->d_xyz, op->d_pk2pad, op->d_table, op->d_table_minus, op->d_tt64, op->d_tt32,
                   op->d_tt32b, op->d_tt64b, op->d_x64s, op->d_b32_tab, op->d_tth, op->d_hscale, op->d_W64, op->d_W32, op->d_ypart, op->d_pk_in, op->d_pk_out, op->d_x32, op->d_y32, op->d_x64, op->d_y64,
-                  op->d_rowsum, op->d_xmax, op->d_xb, op->d_yb};
+                  op->d_rowsum, op->d_xmax, op->d_xb, op->d_yb, op->d_vacc};
   for (void* p : ptrs)
     if (p) hipFree(p);
   auto free_bin = [](smh_op::Binning& b) {
-    void* bp[] = {b.d_rec, b.d_entries, b.d_items, b.d_chunk_items, b.d_item_lsum, b.d_item_en, b.d_order};
+    void* bp[] = {b.d_rec, b.d_entries, b.d_items, b.d_chunk_items, b.d_item_lsum, b.d_item_en, b.d_order,
+                  b.d_recv_off, b.d_recv_pair, b.d_xcd_bounds};
     for (void* p : bp)
       if (p) hipFree(p);
   };

@@ -45,6 +45,7 @@ int regroup(smh_op* op, const std::vector<smh_op::Binning*>& bins, int per_cu, i
   smh_ctx* ctx = op->ctx;
   size_t need = 0;
   for (smh_op::Binning* bn : bins) {
+    if (!bn->slab_pair.empty()) continue;  // (volume, batched: entries are taken from queues, not grouped)
     if (int rc = group_work_items(op, *bn, per_cu, order_mode)) return rc;
     need = std::max(need, (size_t)bn->n_items * bn->part_bytes);
   }
@@ -82,7 +83,7 @@ extern "C" int smh_op_autotune(smh_op* op, int batch, int precision, int iters, 
     SMH_CHECK(ctx, op_has_batch(op, precision), SMH_ERR_UNSUPPORTED, "no batched matvec for this operator");
   const std::vector<smh_op::Binning*> bins = tuned_binnings(op, batch != 0, pi);
   for (smh_op::Binning* bn : bins)
-    SMH_CHECK(ctx, bn->Rc > 0 && bn->count_items, SMH_ERR_UNSUPPORTED, "no %s kernel for this operator",
+    SMH_CHECK(ctx, bn->Rc > 0 && bn->n_entries > 0, SMH_ERR_UNSUPPORTED, "no %s kernel for this operator",
               pi ? "FP64" : "FP32");
   SMH_HIP(ctx, hipSetDevice(ctx->device));
   // captured solver graphs hold the item arrays' addresses and grid sizes

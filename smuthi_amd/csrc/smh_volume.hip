@@ -17,9 +17,7 @@
 // rows. The FP64 kernel reads the same FP32 tap table (complex64 data, exact).
 #include <cmath>
 
-#include "smh_batch_slots.h"
-#include "smh_batch_slots64.h"
-#include "smh_batch_half.h"
+#include "smh_batch_volume.h"
 #include "smh_lookup.h"
 #include "smh_special.h"
 
@@ -250,7 +248,7 @@ __global__ void vol_taps4_kernel(const float2* __restrict__ table, const double2
   }
 }
 
-// The tap rows in the slot fragment order of batch_slots_kernel<..., VOL>:
+// The tap rows in the slot fragment order of vol_slots_kernel:
 // [rows][MT][NS/4][64 lanes][4] FP32, lane (q, rr) of tile i holding
 // A(slot 16 (i mod MH) + rr, slot 4 (4 s4 + e) + q) of the row (tiles i < MH
 // from Re, the others from Im); row = node * vq + kind, kind 0 the table
@@ -289,7 +287,7 @@ __global__ void vol_slot_taps_kernel(const float2* __restrict__ table, const dou
   }
 }
 
-// The same rows in FP64 in the fragment order of batch_slots64_kernel<..., VOL>:
+// The same rows in FP64 in the fragment order of vol_slots64_kernel:
 // [rows][MT][NS/2][64 lanes][2], lane (q, rr) of tile i holding
 // A(slot 16 (i mod MH) + rr, slot 4 (2 s2 + e) + q).
 __global__ void vol_slot_taps64_kernel(const float2* __restrict__ table, const double2* __restrict__ mr,
@@ -326,7 +324,7 @@ __global__ void vol_slot_taps64_kernel(const float2* __restrict__ table, const d
   }
 }
 
-// The same rows in FP16 in the fragment order of batch_half_kernel<..., VOL>:
+// The same rows in FP16 in the fragment order of vol_half_kernel:
 // [rows][MT][64 lanes][NC][4], lane (q, rr) of tile i holding
 // A(slot 16 (i mod MH) + rr, slot 16 c + 4 q + j) / hs[row], hs[row] the
 // smallest power of two with max |A| / hs <= 2^12 over the row; one block
@@ -508,94 +506,61 @@ KernelInfo volume_kernel(int precision, int l, int m, bool tap64 = false) {
   return KernelInfo{};
 }
 
-// FP16 operands: where the FP32 slot-order kernel is used (same binning and
-// input slot order)
+// kBatch-RHS kernels: FP32, FP64 over FP64 tap rows, FP64 over the FP32 rows
+// (tables of plain values, vq = 1: those hold the table values exactly) and
+// FP16 operands (binning and input slot order of the FP32 kernel). Cubic
+// lookups (four z slices, 16 rows per pair) take the slab kernels of
+// smh_batch_volume.h; the bilinear lookup, whose pairs have four rows (32 KB
+// in FP32 at l_max 3, where writing and reading back a product costs 4 KB),
+// the receiver-chunk kernels: 3000 spheres, 9 M pairs per table, FP32 24.6 ms
+// against 30.9 with the slab kernels, FP16 operands 12.0 against 24.4 (with
+// cubic splines and 1500 spheres at two heights 46.5 against 13.3 and 28.3
+// against 9.1).
+enum VolBatch { kVolFp32, kVolFp64, kVolFp64Rows32, kVolHalf };
+bool vol_in_slabs(int vmode) { return vol_slices(vmode) > 1; }
 template <int L, int Mx>
-void* vol_half_fn() {
-  if constexpr (SlotShape<L, Mx, 4>::P32 > 0 && Mx <= 4 && half_tile_parts(4, SvwfIdx<L, Mx>::B) > 0)
-    return reinterpret_cast<void*>(&batch_half_kernel<L, Mx, 4, true>);
-  else
-    return nullptr;
-}
-void* vol_half_kernel(int l, int m) {
-#define SMH_V(L, Mx) \
-  if (l == L && m == Mx) return vol_half_fn<L, Mx>();
-  SMH_V(1, 1)
-  SMH_V(2, 1)
-  SMH_V(2, 2)
-  SMH_V(3, 1)
-  SMH_V(3, 2)
-  SMH_V(3, 3)
-  SMH_V(4, 1)
-  SMH_V(4, 2)
-  SMH_V(4, 3)
-  SMH_V(4, 4)
-#undef SMH_V
-  return nullptr;
-}
-
-// FP32 kBatch-RHS kernel: slot order, its tap fragments in whole parts of the
-// K-steps (every cut-off up to l_max = m_max = 4)
-template <int L, int Mx>
-KernelInfo vol_batch32_kernel_info() {
-  if constexpr (SlotShape<L, Mx, 4>::P32 > 0 && Mx <= 4) {
-    KernelInfo k;
-    k.fn = reinterpret_cast<void*>(&batch_slots_kernel<L, Mx, 4, true>);
-    k.threads = 512;
-    k.sy = SlotShape<L, Mx, 4>::SY;
-    k.slots = SlotShape<L, Mx, 4>::S;
-    k.slot_tables = &slot_tables<L, Mx>;
-    return k;
-  } else {
-    return KernelInfo{};
+KernelInfo vol_chunk_kernel_info(VolBatch form) {
+  using Sh = SlotShape<L, Mx, 4>;
+  KernelInfo k;
+  k.threads = 512;
+  k.slots = Sh::S;
+  k.slot_tables = &slot_tables<L, Mx>;
+  switch (form) {
+    case kVolFp32:
+      k.fn = reinterpret_cast<void*>(&batch_slots_kernel<L, Mx, 4, true>);
+      k.sy = Sh::SY;
+      break;
+    case kVolFp64Rows32:
+      k.fn = reinterpret_cast<void*>(&batch_slots64_kernel<L, Mx, 4, true, true>);
+      k.threads = kSlots64Threads;
+      k.sy = Sh::LO;  // doubles
+      break;
+    case kVolHalf:
+      k.fn = reinterpret_cast<void*>(&batch_half_kernel<L, Mx, 4, true>);
+      k.threads = kHalfThreads;
+      k.sy = Sh::SY;
+      break;
+    default: break;  // (bilinear tables have no FP64 rows)
   }
+  return k;
 }
-// FP64 kBatch-RHS kernel: slot order, its coefficients in parts of the
-// K-steps (the tap rows in FP64 whatever the single-vector kernel's taps)
 template <int L, int Mx>
-KernelInfo vol_batch64_kernel_info() {
-  if constexpr (SlotShape<L, Mx, 4>::P64 > 0 && Mx <= 4) {
-    KernelInfo k;
-    k.fn = reinterpret_cast<void*>(&batch_slots64_kernel<L, Mx, 4, true>);
-    k.threads = kSlots64Threads;
-    k.sy = SlotShape<L, Mx, 4>::LO;  // doubles
-    k.slots = SlotShape<L, Mx, 4>::S;
-    k.slot_tables = &slot_tables<L, Mx>;
-    return k;
-  } else {
-    return KernelInfo{};
+KernelInfo vol_slab_kernel_info(VolBatch form) {
+  KernelInfo k;
+  k.threads = kVolThreads;
+  k.slots = SlotShape<L, Mx, 4>::S;
+  k.slot_tables = &slot_tables<L, Mx>;
+  switch (form) {
+    case kVolFp32: k.fn = reinterpret_cast<void*>(&vol_slots_kernel<L, Mx>); break;
+    case kVolFp64: k.fn = reinterpret_cast<void*>(&vol_slots64_kernel<L, Mx, false>); break;
+    case kVolFp64Rows32: k.fn = reinterpret_cast<void*>(&vol_slots64_kernel<L, Mx, true>); break;
+    case kVolHalf: k.fn = reinterpret_cast<void*>(&vol_half_kernel<L, Mx>); break;
   }
+  return k;
 }
-// FP64 kBatch-RHS kernel over the FP32 slot-order tap rows (tables of plain
-// values, vq = 1: the rows hold the FP32 table values exactly)
-template <int L, int Mx>
-void* vol_batch64_tap32_fn() {
-  if constexpr (SlotShape<L, Mx, 4>::P64 > 0 && SlotShape<L, Mx, 4>::P32 > 0 && Mx <= 4)
-    return reinterpret_cast<void*>(&batch_slots64_kernel<L, Mx, 4, true, true>);
-  else
-    return nullptr;
-}
-void* vol_batch64_tap32_kernel(int l, int m) {
-#define SMH_V(L, Mx) \
-  if (l == L && m == Mx) return vol_batch64_tap32_fn<L, Mx>();
-  SMH_V(1, 1)
-  SMH_V(2, 1)
-  SMH_V(2, 2)
-  SMH_V(3, 1)
-  SMH_V(3, 2)
-  SMH_V(3, 3)
-  SMH_V(4, 1)
-  SMH_V(4, 2)
-  SMH_V(4, 3)
-  SMH_V(4, 4)
-#undef SMH_V
-  return nullptr;
-}
-
-KernelInfo volume_batch_kernel(int precision, int l, int m) {
-#define SMH_V(L, Mx)                                                                                    \
-  if (l == L && m == Mx)                                                                                \
-    return precision == SMH_FP32 ? vol_batch32_kernel_info<L, Mx>() : vol_batch64_kernel_info<L, Mx>();
+KernelInfo vol_batch_kernel(VolBatch form, int l, int m, int vmode) {
+#define SMH_V(L, Mx)     \
+  if (l == L && m == Mx) return vol_in_slabs(vmode) ? vol_slab_kernel_info<L, Mx>(form) : vol_chunk_kernel_info<L, Mx>(form);
   SMH_V(1, 1)
   SMH_V(2, 1)
   SMH_V(2, 2)
@@ -609,9 +574,209 @@ KernelInfo volume_batch_kernel(int precision, int l, int m) {
 #undef SMH_V
   return KernelInfo{};
 }
+// FP64 form of an operator: its FP64 rows hold spline moments
+VolBatch vol_fp64_form(const smh_op* op) { return op->vq == 1 ? kVolFp64Rows32 : kVolFp64; }
+
+// Position of every ordered pair of a segment by (receiver, sender): row i of
+// the dense list begins at row_off[i].
+__global__ void vol_pair_position_kernel(const uint2* __restrict__ pairs, int64_t n_pairs,
+                                         const int* __restrict__ row_off, const int* __restrict__ seg_of,
+                                         const int64_t* __restrict__ seg_off, int* pos) {
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n_pairs) return;
+  const uint2 pr = pairs[p];
+  const int sg = seg_of ? seg_of[pr.x] : 0;
+  pos[row_off[pr.x] + (int)((int64_t)pr.y - seg_off[sg])] = (int)p;
+}
+
+__device__ inline int slab_of(const int* __restrict__ slab_pair, int n_slabs, int p) {
+  int lo = 0, hi = n_slabs;  // slab_pair[lo] <= p < slab_pair[hi]
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (slab_pair[mid] <= p)
+      lo = mid;
+    else
+      hi = mid;
+  }
+  return lo;
+}
+
+__global__ void vol_recv_count_kernel(const uint2* __restrict__ pairs, int64_t n_pairs,
+                                      const int* __restrict__ slab_pair, int n_slabs, int n_part, int* cnt) {
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n_pairs) return;
+  atomicAdd(&cnt[(int64_t)slab_of(slab_pair, n_slabs, (int)p) * n_part + pairs[p].x], 1);
+}
+
+// Each receiver's pairs per slab, in sender order: one wave per receiver goes
+// through its row of positions and appends to the slabs' lists, whose ends it
+// keeps in LDS (one int per slab).
+__global__ void __launch_bounds__(64) vol_recv_fill_kernel(const int* __restrict__ pos, const int* __restrict__ row_off,
+                                                           const int* __restrict__ slab_pair, int n_slabs, int n_part,
+                                                           const int* __restrict__ recv_off, int* recv_pair) {
+  extern __shared__ int list_end[];
+  const int i = blockIdx.x, lane = threadIdx.x;
+  for (int s = lane; s < n_slabs; s += 64) list_end[s] = recv_off[(int64_t)s * n_part + i];
+  __syncthreads();
+  const int j1 = row_off[i + 1];
+  for (int j0 = row_off[i]; j0 < j1; j0 += 64) {
+    const bool live = j0 + lane < j1;
+    const int p = live ? pos[j0 + lane] : 0;
+    const int s = live ? slab_of(slab_pair, n_slabs, p) : -1;
+    unsigned long long left = __ballot(live);
+    while (left) {
+      const int leader = __ffsll((long long)left) - 1;
+      const int sl = __shfl(s, leader);
+      const unsigned long long same = __ballot(s == sl);
+      int at = 0;
+      if (lane == leader) at = atomicAdd(&list_end[sl], __popcll(same));
+      at = __shfl(at, leader);
+      if (s == sl) recv_pair[at + __popcll(same & ((1ull << lane) - 1))] = p;
+      left &= ~same;
+    }
+  }
+}
+
+// Slabs of the kBatch-RHS kernels: kVolSlabBytes of products, which the
+// receiver sums then read back from the last-level cache (256 MB; 700 spheres,
+// l_max 3, FP32: 4.6 ms with 128 MB, 4.9 with 256, of 30 us per slab for the
+// sums), and no more than kVolSlabs of them.
+constexpr size_t kVolSlabBytes = (size_t)128 << 20;
+constexpr int kVolSlabs = 2048;
+
+// Entries, slabs and receiver lists of the kBatch-RHS kernels: cnt / off: pair
+// count and first pair of each bin, pairs: (receiver, sender) in that order.
+template <typename Real>
+int vol_build_slabs(smh_op* op, smh_op::Binning& bn, const std::vector<int>& cnt, const std::vector<int>& off,
+                    const uint2* d_pairs, int64_t n_pairs) {
+  smh_ctx* ctx = op->ctx;
+  hipStream_t s = ctx->stream;
+  const int64_t n_part = op->n_part;
+  constexpr int kUnit = sizeof(Real) == 4 ? kVolPairs32 : kVolPairs64;
+  const int64_t pair_bytes = (int64_t)2 * kBatchRhs * op->b32_S * sizeof(Real);
+  const int64_t slab_pairs = std::max<int64_t>((int64_t)kVolSlabBytes / pair_bytes, (n_pairs + kVolSlabs - 1) / kVolSlabs);
+  bn.Rc = (int)n_part;
+  std::vector<int4> units;
+  bn.slab_pair.assign(1, 0);
+  std::vector<int> slab_unit(1, 0);
+  for (size_t k = 0; k < cnt.size(); ++k)
+    for (int p0 = 0; p0 < cnt[k]; p0 += kUnit) {
+      const int np = std::min(kUnit, cnt[k] - p0), first = off[k] + p0;
+      if (first + np - bn.slab_pair.back() > slab_pairs && first > bn.slab_pair.back()) {
+        bn.slab_pair.push_back(first);
+        slab_unit.push_back((int)units.size());
+      }
+      units.push_back(make_int4((int)k * op->vq, first, np, 0));
+    }
+  bn.slab_pair.push_back((int)n_pairs);
+  const int n_slabs = (int)bn.slab_pair.size() - 1;
+  bn.n_chunks = n_slabs;
+  bn.n_entries = (int)units.size();
+  slab_unit.push_back(bn.n_entries);
+  // the XCDs' equal shares of a slab's units
+  std::vector<int> bounds;
+  for (int sl = 0; sl < n_slabs; ++sl) {
+    const int64_t n = slab_unit[sl + 1] - slab_unit[sl];
+    for (int x = 0; x <= kVolXcds; ++x) bounds.push_back(slab_unit[sl] + (int)(n * x / kVolXcds));
+  }
+  // receiver lists
+  std::vector<int> row_off(n_part + 1, 0), recv_off((size_t)n_slabs * n_part + 1, 0);
+  for (int sg = 0; sg < op->n_seg; ++sg)
+    for (int64_t i = op->seg_off[sg]; i < op->seg_off[sg + 1]; ++i)
+      row_off[i + 1] = row_off[i] + (int)(op->seg_off[sg + 1] - op->seg_off[sg]);
+  int *d_row = nullptr, *d_pos = nullptr, *d_slab = nullptr;
+  auto run = [&]() {
+    const size_t nr = recv_off.size() * sizeof(int), ns = bn.slab_pair.size() * sizeof(int);
+    if (hipMalloc(&d_row, row_off.size() * sizeof(int)) != hipSuccess || hipMalloc(&d_pos, n_pairs * sizeof(int)) != hipSuccess ||
+        hipMalloc(&d_slab, ns) != hipSuccess || hipMalloc(&bn.d_recv_off, nr) != hipSuccess ||
+        hipMalloc(&bn.d_recv_pair, n_pairs * sizeof(int)) != hipSuccess ||
+        hipMalloc(&bn.d_xcd_bounds, bounds.size() * sizeof(int)) != hipSuccess ||
+        hipMemcpyAsync(bn.d_xcd_bounds, bounds.data(), bounds.size() * sizeof(int), hipMemcpyHostToDevice, s) != hipSuccess ||
+        hipMalloc(&bn.d_entries, units.size() * sizeof(int4)) != hipSuccess ||
+        hipMemcpyAsync(bn.d_entries, units.data(), units.size() * sizeof(int4), hipMemcpyHostToDevice, s) != hipSuccess ||
+        hipMemcpyAsync(d_row, row_off.data(), row_off.size() * sizeof(int), hipMemcpyHostToDevice, s) != hipSuccess ||
+        hipMemcpyAsync(d_slab, bn.slab_pair.data(), ns, hipMemcpyHostToDevice, s) != hipSuccess ||
+        hipMemsetAsync(bn.d_recv_off, 0, nr, s) != hipSuccess)
+      return smh_fail(ctx, SMH_ERR_HIP, "device allocation failed (volume slabs)");
+    const dim3 grid((unsigned)((n_pairs + 255) / 256));
+    hipLaunchKernelGGL(vol_pair_position_kernel, grid, dim3(256), 0, s, d_pairs, n_pairs, d_row,
+                       (const int*)op->d_seg_of, (const int64_t*)op->d_seg_off, d_pos);
+    hipLaunchKernelGGL(vol_recv_count_kernel, grid, dim3(256), 0, s, d_pairs, n_pairs, d_slab, n_slabs, (int)n_part,
+                       bn.d_recv_off);
+    if (hipMemcpyAsync(recv_off.data(), bn.d_recv_off, nr, hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipStreamSynchronize(s) != hipSuccess)
+      return smh_fail(ctx, SMH_ERR_HIP, "volume receiver lists failed");
+    int acc = 0;
+    for (int& v : recv_off) {
+      const int c = v;
+      v = acc;
+      acc += c;
+    }
+    if (hipMemcpyAsync(bn.d_recv_off, recv_off.data(), nr, hipMemcpyHostToDevice, s) != hipSuccess)
+      return smh_fail(ctx, SMH_ERR_HIP, "volume receiver lists failed");
+    hipLaunchKernelGGL(vol_recv_fill_kernel, dim3((unsigned)n_part), dim3(64), n_slabs * sizeof(int), s, d_pos, d_row,
+                       d_slab, n_slabs, (int)n_part, bn.d_recv_off, bn.d_recv_pair);
+    if (hipStreamSynchronize(s) != hipSuccess) return smh_fail(ctx, SMH_ERR_HIP, "volume receiver lists failed");
+    return (int)SMH_OK;
+  };
+  const int rc = run();
+  for (int* p : {d_row, d_pos, d_slab})
+    if (p) hipFree(p);
+  return rc;
+}
+
+// Receiver sums of a slab's products (smh_batch_volume.h): y of receiver i is
+// the sum over its pairs, added in FP64 in sender order by four strands of 4 S
+// threads, the strands then in order. sums keeps the receivers' totals between
+// the slabs and tables (first: none yet); the last slab writes y, in the plain
+// layout [n_part][B][kBatch]. Bound by reading the products once: 2 KB per
+// pair in FP32 at l_max 3.
+constexpr int kVolStrands = 4;
+template <typename Real>
+__global__ void vol_sum_kernel(const Real* __restrict__ products, const int* __restrict__ recv_off,
+                               const int* __restrict__ recv_pair, int pair0, int S, int B,
+                               const int* __restrict__ n_of, int first, int last, double* sums,
+                               typename Vec2<Real>::t* y) {
+  typedef Real v4_t __attribute__((ext_vector_type(4)));
+  extern __shared__ __align__(16) double part[];  // [kVolStrands - 1][16 S]
+  const int i1 = blockIdx.x, t = threadIdx.x, E = 2 * kBatchRhs * S;
+  const int k0 = recv_off[i1], k1 = recv_off[i1 + 1];
+  const int per = (k1 - k0 + kVolStrands - 1) / kVolStrands;
+  const int a0 = min(k1, k0 + (int)threadIdx.y * per), a1 = min(k1, a0 + per);
+  double v[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 8
+  for (int k = a0; k < a1; ++k) {
+    const v4_t p = *reinterpret_cast<const v4_t*>(products + (size_t)(recv_pair[k] - pair0) * E + 4 * t);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] += (double)p[j];
+  }
+  if (threadIdx.y > 0) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) part[(threadIdx.y - 1) * E + 4 * t + j] = v[j];
+  }
+  __syncthreads();
+  if (threadIdx.y > 0) return;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int e = 4 * t + j;
+    double w = v[j];
+    for (int d = 0; d < kVolStrands - 1; ++d) w += part[d * E + e];
+    if (!first) w += sums[(size_t)i1 * E + e];
+    if (!last) {
+      sums[(size_t)i1 * E + e] = w;
+      continue;
+    }
+    // element e of a product: tile e / 256, see smh_batch_volume.h
+    const int i = e >> 8, lane = sizeof(Real) == 4 ? (e & 255) >> 2 : e & 63;
+    const int slot = sizeof(Real) == 4 ? 16 * i + 4 * (lane >> 4) + (e & 3) : 16 * i + 4 * ((e >> 6) & 3) + (lane >> 4);
+    const int n1 = n_of[slot], col = lane & 15;
+    if (n1 >= 0) reinterpret_cast<Real*>(y)[(((size_t)i1 * B + n1) * kBatchRhs + (col >> 1)) * 2 + (col & 1)] = (Real)w;
+  }
+}
 
 // Bin the pairs of table tab (0: z1 + z2, 1: z1 - z2) for precision pi, for
-// the single-vector kernel or (batch) the kBatch-RHS kernel.
+// the single-vector kernel or (batch) the kBatch-RHS kernels, in receiver
+// chunks of Rc, or in slabs (batch, cubic lookups; Rc = n_part: one chunk).
 template <typename Real>
 int vol_bin_pairs(smh_op* op, int tab, int pi, int Rc, bool batch) {
   smh_ctx* ctx = op->ctx;
@@ -620,6 +785,7 @@ int vol_bin_pairs(smh_op* op, int tab, int pi, int Rc, bool batch) {
   const int64_t n_part = op->n_part, len_rho = op->len_rho, len_z = op->len_z;
   const double zmin = tab == 0 ? op->sz_min : op->dz_min, zsgn = tab == 0 ? 1.0 : -1.0;
   const int lo = op->vmode == 2 ? 1 : 0, hi = op->vmode == 2 ? 3 : 2;
+  const bool slabs = batch && vol_in_slabs(op->vmode);
   bn.Rc = Rc;
   bn.n_chunks = (int)((n_part + Rc - 1) / Rc);
   const int64_t nkeys = (int64_t)bn.n_chunks * len_rho * len_z;
@@ -682,13 +848,18 @@ int vol_bin_pairs(smh_op* op, int tab, int pi, int Rc, bool batch) {
                      (const int64_t*)op->d_seg_off, d_cnt, (const int*)d_off, d_cur, d_pairs, d_err);
   if (acc > 0)
     hipLaunchKernelGGL(vol_pair_record_kernel<Real>, dim3((unsigned)((acc + 255) / 256)), dim3(256), 0, s, d_pairs,
-                       acc, op->d_xyz, op->rho_min, op->h, zmin, zsgn, Rc, (PairRec2<Real>*)bn.d_rec);
+                       acc, op->d_xyz, op->rho_min, op->h, zmin, zsgn, slabs ? 1 : Rc, (PairRec2<Real>*)bn.d_rec);
   if (hipStreamSynchronize(s) != hipSuccess) {
     cleanup();
     return smh_fail(ctx, SMH_ERR_HIP, "volume pair records failed");
   }
-  cleanup();
   op->n_pairs = acc;
+  if (slabs) {
+    const int rc = vol_build_slabs<Real>(op, bn, cnt, off, d_pairs, acc);
+    cleanup();
+    return rc;
+  }
+  cleanup();
   // a (chunk, r, j) key is a bin; its entry starts at the node's first tap row (r * len_z + j) * vq
   const int vq = op->vq;
   return build_work_items<PairRec2<Real>>(op, bn, cnt, off, len_rho * len_z,
@@ -761,7 +932,7 @@ int vol_make_taps(smh_op* op) {
       }
       hipLaunchKernelGGL(vol_slot_taps_kernel, dim3(4096), dim3(256), 0, s, op->d_vtab[t], mr, mz, mrz, rows, op->vq,
                          op->B, S, (const int*)op->d_b32_tab + op->B, op->d_vtts[t]);
-      if (vol_half_kernel(op->l_max, op->m_max)) {
+      if (vol_batch_kernel(kVolHalf, op->l_max, op->m_max, op->vmode).fn) {
         if (!op->d_vtth[t] && (hipMalloc(&op->d_vtth[t], (size_t)rows * 2 * S * S * sizeof(_Float16)) != hipSuccess ||
                                hipMalloc(&op->d_vhs[t], (size_t)rows * sizeof(float)) != hipSuccess)) {
           cleanup();
@@ -772,7 +943,7 @@ int vol_make_taps(smh_op* op) {
       }
       // FP64 slot rows only for tables with spline moments (vq = 4); plain
       // values (vq = 1) reach the FP64 kernel through the FP32 rows above
-      if (op->vq == 4 && volume_batch_kernel(SMH_FP64, op->l_max, op->m_max).slots == S) {
+      if (op->vq == 4) {
         if (!op->d_vtts64[t] &&
             hipMalloc(&op->d_vtts64[t], (size_t)rows * 2 * S * S * sizeof(double)) != hipSuccess) {
           cleanup();
@@ -784,8 +955,8 @@ int vol_make_taps(smh_op* op) {
     }
     hipLaunchKernelGGL(frag_rowsum_kernel, dim3((unsigned)std::min<int64_t>(rows, 65536)), dim3(256), 0, s,
                        op->d_vtt[t], rows, op->B, op->Bh, g.NG, g.FR, op->d_vrowsum[t]);
-    for (smh_op::Binning* bn : {&op->vbin[t][0], &op->vbbin[t][0]})
-      set_item_lsum(*bn, op->d_vrowsum[t], 4, op->vmode, (int)op->len_z, s);
+    set_item_lsum(op->vbin[t][0], op->d_vrowsum[t], 4, op->vmode, (int)op->len_z, s);
+    if (!vol_in_slabs(op->vmode)) set_item_lsum(op->vbbin[t][0], op->d_vrowsum[t], 4, op->vmode, (int)op->len_z, s);
     // the moments of this table must be consumed before the next one overwrites them
     if (hipStreamSynchronize(s) != hipSuccess) {
       cleanup();
@@ -860,37 +1031,34 @@ int vol_apply(smh_op* op, int precision, const void* x_pad, void* y_pad, bool ti
   return SMH_OK;
 }
 
-// kBatch right-hand sides on the plain layout [n_part][B][kBatch] (FP32 input
-// float2, FP64 double2): one batched launch per table and z slice, their
-// partials summed into y in launch order.
+// kBatch right-hand sides (FP32 and FP16 input in the slot layout, FP64
+// [n_part][B][kBatch] double2). Cubic lookups: per table and slab the products
+// of its pairs, then their receiver sums; bilinear: one launch per table, its
+// partials summed into y in table order.
 int vol_apply_batch(smh_op* op, int precision, const void* x_pad, void* y_pad, bool time_kernel) {
   smh_ctx* ctx = op->ctx;
   // the FP16-operand kernel shares the FP32 kernel's binning, slot order and partial-sum layout
   const bool half = precision == SMH_FP16;
   const int pi = (precision == SMH_FP32 || half) ? 0 : 1;
-  const bool tap64 = pi == 1 && op->vq == 4;
-  const KernelInfo k = volume_batch_kernel(half ? SMH_FP32 : precision, op->l_max, op->m_max);
   // FP64 over tables of plain values: the FP32 slot rows, widened in the kernel
-  const bool rows32 = pi == 1 && op->vq == 1 && k.slots > 0;
-  void* fn = half ? vol_half_kernel(op->l_max, op->m_max)
-                  : (rows32 ? vol_batch64_tap32_kernel(op->l_max, op->m_max) : k.fn);
-  SMH_CHECK(ctx, fn != nullptr && op->vbbin[0][pi].Rc > 0, SMH_ERR_UNSUPPORTED,
+  const bool rows32 = pi == 1 && op->vq == 1;
+  const bool slabs = vol_in_slabs(op->vmode);
+  const KernelInfo k = vol_batch_kernel(half ? kVolHalf : (pi == 0 ? kVolFp32 : vol_fp64_form(op)), op->l_max,
+                                        op->m_max, op->vmode);
+  SMH_CHECK(ctx, k.fn != nullptr && op->vbbin[0][pi].Rc > 0, SMH_ERR_UNSUPPORTED,
             "no batched volume matvec kernel for l_max %d m_max %d", op->l_max, op->m_max);
   hipStream_t s = ctx->stream;
-  const bool slots = k.slots > 0;
   SMH_CHECK(ctx,
-            !slots || (op->d_b32_tab && op->b32_S == k.slots &&
-                       (half ? op->d_vtth[0] && op->d_vtth[1]
-                             : (pi == 0 || rows32 ? op->d_vtts[0] && op->d_vtts[1]
-                                                  : op->d_vtts64[0] && op->d_vtts64[1]))),
+            op->d_b32_tab && op->b32_S == k.slots &&
+                (half ? op->d_vtth[0] && op->d_vtth[1]
+                      : (pi == 0 || rows32 ? op->d_vtts[0] && op->d_vtts[1] : op->d_vtts64[0] && op->d_vtts64[1])),
             SMH_ERR_STATE, "slot-order tap rows missing");
-  SMH_CHECK(ctx, !half || slots, SMH_ERR_STATE, "the FP16 kernel needs the slot order");
-  const int S = slots ? k.slots : op->B;
-  const int* slot = slots ? (const int*)op->d_b32_tab : nullptr;
+  const int S = k.slots;
+  const int* slot = (const int*)op->d_b32_tab;
   // (the FP16 input was scaled by the xmax its conversion wrote)
-  if (pi == 0 && !half) launch_xmax((const float2*)x_pad, op->n_part * S * kBatchRhs, op->d_xmax, s);
+  if (pi == 0 && !half && !slabs) launch_xmax((const float2*)x_pad, op->n_part * S * kBatchRhs, op->d_xmax, s);
   const void* xin = x_pad;
-  if (pi == 1 && slots) {
+  if (pi == 1) {
     // FP64 padded [n_part][B][kBatch] -> the slot layout (padding slots stay zero)
     const int64_t n8 = op->n_part * op->B * kBatchRhs;
     if (!op->d_x64s) {
@@ -903,18 +1071,30 @@ int vol_apply_batch(smh_op* op, int precision, const void* x_pad, void* y_pad, b
     xin = op->d_x64s;
   }
   double ms_total = 0;
-  const int n_slices = op->vmode >= 2 ? 4 : 1;
+  auto launch = [&](const void* fn, int blocks, void** args, size_t lds) -> int {
+    if (time_kernel) SMH_HIP(ctx, hipEventRecord(ctx->ev0, s));
+    SMH_HIP(ctx, hipLaunchKernel(fn, dim3(blocks), dim3(k.threads), args, lds, s));
+    if (time_kernel) {
+      SMH_HIP(ctx, hipEventRecord(ctx->ev1, s));
+      SMH_HIP(ctx, hipEventSynchronize(ctx->ev1));
+      float ms = 0;
+      SMH_HIP(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
+      ms_total += ms;
+    }
+    return SMH_OK;
+  };
   for (int t = 0; t < 2; ++t) {
     const smh_op::Binning& bn = op->vbbin[t][pi];
-    for (int sl = 0; sl < n_slices; ++sl) {
+    const void* rows = half ? (const void*)op->d_vtth[t]
+                            : (pi == 0 || rows32 ? (const void*)op->d_vtts[t] : (const void*)op->d_vtts64[t]);
+    const float* hs = op->d_vhs[t];
+    if (!slabs) {
       RadialKArgs a;
       a.recs = bn.d_rec;
       a.entries = bn.d_entries;
       a.items = bn.d_items;
       a.order = bn.d_order;
-      a.tt = half ? (const void*)op->d_vtth[t]
-                  : (slots ? (pi == 0 || rows32 ? (const void*)op->d_vtts[t] : (const void*)op->d_vtts64[t])
-                           : (tap64 ? (const void*)op->d_vtt64[t] : (const void*)op->d_vtt[t]));
+      a.tt = rows;
       a.x = xin;
       a.ypart = op->d_ypart;
       a.xmax = op->d_xmax;
@@ -926,31 +1106,50 @@ int vol_apply_batch(smh_op* op, int precision, const void* x_pad, void* y_pad, b
       a.Rc = bn.Rc;
       a.len_z = (int)op->len_z;
       a.vmode = op->vmode;
-      a.vslice = sl;
       a.row_s = 1;
       a.row_o = 0;
-      if (int rc_ = op_set_lds(op, fn, bn.lds)) return rc_;
-      if (bn.n_items > 0) {
-        if (time_kernel) SMH_HIP(ctx, hipEventRecord(ctx->ev0, s));
-        const float* hs = op->d_vhs[t];
-        void* args1[] = {&a};
-        void* args2[] = {&a, &hs};
-        const int threads = half ? kHalfThreads : k.threads;
-        SMH_HIP(ctx, hipLaunchKernel(fn, dim3(bn.n_items), dim3(threads), half ? args2 : args1,
-                                     bn.lds, s));
-        if (time_kernel) {
-          SMH_HIP(ctx, hipEventRecord(ctx->ev1, s));
-          SMH_HIP(ctx, hipEventSynchronize(ctx->ev1));
-          float ms = 0;
-          SMH_HIP(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
-          ms_total += ms;
-        }
-      }
-      const int accumulate = (t > 0 || sl > 0) ? 1 : 0;
+      if (int rc_ = op_set_lds(op, k.fn, bn.lds)) return rc_;
+      void* args1[] = {&a};
+      void* args2[] = {&a, &hs};
+      if (bn.n_items > 0)
+        if (int rc = launch(k.fn, bn.n_items, half ? args2 : args1, bn.lds)) return rc;
       if (pi == 0)
-        launch_reduce_batch<float>(op, bn, S, slots ? slot + op->B : nullptr, y_pad, accumulate, s);
+        launch_reduce_batch<float>(op, bn, S, slot + op->B, y_pad, t, s);
       else
-        launch_reduce_batch<double>(op, bn, S, slots ? slot + op->B : nullptr, y_pad, accumulate, s);
+        launch_reduce_batch<double>(op, bn, S, slot + op->B, y_pad, t, s);
+      SMH_HIP(ctx, hipGetLastError());
+      continue;
+    }
+    VolKArgs a;
+    a.recs = bn.d_rec;
+    a.units = bn.d_entries;
+    a.tt = rows;
+    a.x = xin;
+    a.out = op->d_ypart;
+    a.xmax = op->d_xmax;
+    a.hscale = hs;
+    a.len_z = (int)op->len_z;
+    a.vmode = op->vmode;
+    for (int sl = 0; sl < bn.n_chunks; ++sl) {
+      a.bounds = bn.d_xcd_bounds + sl * (kVolXcds + 1);
+      a.pair0 = bn.slab_pair[sl];
+      // two workgroups per CU, which go through the slab's units
+      const int pairs = bn.slab_pair[sl + 1] - bn.slab_pair[sl], waves = k.threads / 64;
+      const int blocks = std::max(kVolXcds, std::min(2 * ctx->num_cu, (pairs + waves - 1) / waves));
+      void* args[] = {&a};
+      if (int rc = launch(k.fn, blocks, args, 0)) return rc;
+      const int first = t == 0 && sl == 0, last = t == 1 && sl == bn.n_chunks - 1;
+      const dim3 block(4 * S, kVolStrands);
+      const size_t lds = (size_t)(kVolStrands - 1) * 2 * kBatchRhs * S * sizeof(double);
+      const int* recv_off = bn.d_recv_off + (size_t)sl * op->n_part;
+      if (pi == 0)
+        hipLaunchKernelGGL(vol_sum_kernel<float>, dim3((unsigned)op->n_part), block, lds, s, (const float*)op->d_ypart,
+                           recv_off, bn.d_recv_pair, a.pair0, S, op->B, slot + op->B, first, last, op->d_vacc,
+                           (float2*)y_pad);
+      else
+        hipLaunchKernelGGL(vol_sum_kernel<double>, dim3((unsigned)op->n_part), block, lds, s,
+                           (const double*)op->d_ypart, recv_off, bn.d_recv_pair, a.pair0, S, op->B, slot + op->B,
+                           first, last, op->d_vacc, (double2*)y_pad);
       SMH_HIP(ctx, hipGetLastError());
     }
   }
@@ -1043,7 +1242,7 @@ static int volume_create(smh_ctx* ctx, int n_ens, const int64_t* ens_off, int64_
   // kernel, else the plain layout [n_part][B][kBatch]
   op->b32_S = op->B;
   {
-    const KernelInfo kb32 = volume_batch_kernel(SMH_FP32, l_max, m_max);
+    const KernelInfo kb32 = vol_batch_kernel(kVolFp32, l_max, m_max, op->vmode);
     if (kb32.fn && kb32.slots > 0) {
       std::vector<int> tab(op->B + kb32.slots);
       kb32.slot_tables(tab.data());
@@ -1076,17 +1275,31 @@ static int volume_create(smh_ctx* ctx, int n_ens, const int64_t* ens_off, int64_
       op->vbin[t][pi].part_bytes = (size_t)Rc * 2 * op->B * rs;
       ypart = std::max(ypart, (size_t)op->vbin[t][pi].n_items * op->vbin[t][pi].part_bytes);
     }
-    // the same pairs for the kBatch-RHS kernel (its accumulator holds kBatch vectors per receiver)
-    const KernelInfo kb = volume_batch_kernel(pi == 0 ? SMH_FP32 : SMH_FP64, l_max, m_max);
+    // the same pairs for the kBatch-RHS kernels
+    const int64_t E = (int64_t)2 * kBatchRhs * op->b32_S;
+    const bool slabs = vol_in_slabs(op->vmode);
     size_t ldsb = 0;
-    const int Rb = kb.fn ? chunk_size(op, rs, kb.sy, ldsb) : 0;
-    if (Rb == 0) continue;
+    int Rb = (int)n_part;
+    if (!slabs) {
+      const KernelInfo kb = vol_batch_kernel(pi == 0 ? kVolFp32 : vol_fp64_form(op), l_max, m_max, op->vmode);
+      Rb = kb.fn ? chunk_size(op, rs, kb.sy, ldsb) : 0;
+      if (Rb == 0) continue;
+    }
     for (int t = 0; t < 2; ++t) {
-      op->vbbin[t][pi].lds = ldsb;
+      smh_op::Binning& bn = op->vbbin[t][pi];
+      bn.lds = ldsb;
       const int code = pi == 0 ? vol_bin_pairs<float>(op, t, 0, Rb, true) : vol_bin_pairs<double>(op, t, 1, Rb, true);
       if (code) return fail(code);
-      op->vbbin[t][pi].part_bytes = (size_t)Rb * 2 * kBatchRhs * (kb.slots > 0 ? kb.slots : op->B) * rs;
-      ypart = std::max(ypart, (size_t)op->vbbin[t][pi].n_items * op->vbbin[t][pi].part_bytes);
+      if (!slabs) {
+        bn.part_bytes = (size_t)Rb * E * rs;
+        ypart = std::max(ypart, (size_t)bn.n_items * bn.part_bytes);
+      }
+      for (size_t k = 0; k + 1 < bn.slab_pair.size(); ++k)
+        ypart = std::max(ypart, (size_t)(bn.slab_pair[k + 1] - bn.slab_pair[k]) * E * rs);
+    }
+    if (slabs && !op->d_vacc && hipMalloc(&op->d_vacc, n_part * E * sizeof(double)) != hipSuccess) {
+      smh_fail(ctx, SMH_ERR_HIP, "device allocation failed (receiver sums)");
+      return fail(SMH_ERR_HIP);
     }
   }
   op->ypart_bytes = std::max<size_t>(ypart, 16);
