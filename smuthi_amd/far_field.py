@@ -9,7 +9,7 @@ vector without touching the particles' stored fields."""
 import numpy as np
 
 from . import fields as flds
-from .scattered_field import scattered_field_pwe
+from .scattered_field import _by_layer, _scattered_field_pwe, scattered_field_pwe
 
 
 class FarField:
@@ -118,7 +118,7 @@ def pwe_to_ff_conversion(vacuum_wavelength, plane_wave_expansion):
         raise ValueError('complex angles are not allowed')
     kz = flds.k_z(k_parallel=kp, k=k)
     ampli = -2 * np.pi * (kz * k)[None, :, None] * pwe.coefficients
-    intens = (2 * np.pi ** 2 / omega * (kz ** 2 * k)[None, :, None] * abs(pwe.coefficients) ** 2).real
+    intens = (2 * np.pi ** 2 / omega * (kz ** 2 * k)).real[None, :, None] * abs(pwe.coefficients) ** 2
     idx = np.argsort(np.real(polar))
     ff = FarField(polar_angles=np.real(polar)[idx], azimuthal_angles=pwe.azimuthal_angles,
                   reference_point=pwe.reference_point)
@@ -144,14 +144,17 @@ def scattered_far_field(vacuum_wavelength, particle_list, layer_system, polar_an
     n_top = np.sort(np.sin(top) * layer_system.refractive_indices[i_top])
     n_bot = np.sort(np.sin(bot) * layer_system.refractive_indices[0])
     ff_top = ff_bot = None
+    by_layer, scatterers = _by_layer(particle_list, layer_system), {}
+
+    def half_space(layer, n_eff, direction):
+        pwe = _scattered_field_pwe(vacuum_wavelength, by_layer, scatterers, layer_system, layer, n_eff * omega,
+                                   azimuthal_angles, True, True, precision, (direction,))[direction]
+        return pwe_to_ff_conversion(vacuum_wavelength, pwe)
+
     if len(top) > 1 and np.imag(layer_system.refractive_indices[i_top]) == 0:
-        up, _ = scattered_field_pwe(vacuum_wavelength, particle_list, layer_system, i_top, n_top * omega,
-                                    azimuthal_angles, precision=precision)
-        ff_top = pwe_to_ff_conversion(vacuum_wavelength, up)
+        ff_top = half_space(i_top, n_top, 0)
     if len(bot) > 1 and np.imag(layer_system.refractive_indices[0]) == 0:
-        _, dn = scattered_field_pwe(vacuum_wavelength, particle_list, layer_system, 0, n_bot * omega,
-                                    azimuthal_angles, precision=precision)
-        ff_bot = pwe_to_ff_conversion(vacuum_wavelength, dn)
+        ff_bot = half_space(0, n_bot, 1)
     if ff_top is not None:
         if ff_bot is not None:
             ff_top.append(ff_bot)

@@ -40,6 +40,11 @@ class LayerSystem:
         bounds = np.cumsum([0] + list(self.thicknesses[1:-1]))
         return int(np.searchsorted(bounds, z, side='right'))
 
+    def layer_numbers(self, z):
+        """layer_number of every height of the array z."""
+        bounds = np.cumsum([0] + list(self.thicknesses[1:-1]))
+        return np.searchsorted(bounds, z, side='right')
+
     def wavenumber(self, layer_number, vacuum_wavelength):
         return self.refractive_indices[layer_number] * flds.angular_frequency(vacuum_wavelength)
 
