@@ -6,9 +6,9 @@ U(1.5,2.0) + 0.01i) at z = 200 nm in a 60 x 60 um square with 20 nm minimum
 gaps, on glass (n = 1.52) in air, lambda = 550 nm, l_max = m_max = 3
 (300,000 unknowns), radial lookup with cubic (not-a-knot spline)
 interpolation at 2 nm, Sommerfeld contour with neff_resolution = neff_imag =
-2e-3. The right-hand sides are 64 distinct plane waves (32 polar angles from
-0 to 60 degrees, TE and TM); a step solves the next 8 of them to relative
-residual 1e-6: GMRES for the whole batch in lockstep whose coupling matvecs
+2e-3. The right-hand sides are distinct plane waves (32 polar angles from
+0 to 60 degrees, TE and TM: 64, then further azimuths); a step solves the next
+8 of them to relative residual 1e-6: GMRES for the whole batch in lockstep whose coupling matvecs
 run with FP16 operands on MFMA (one launch per 8 RHS; --precision mixed:
 FP32), wrapped in FP64 iterative refinement (FP32 residuals between sweeps,
 the FP64 residual certifies the result). Every timed right-hand side is
@@ -29,6 +29,7 @@ Usage: python bench.py [--gpus 1] [--steps K] [--warmup W] [--particles N] [--ba
 import argparse
 import contextlib
 import json
+import math
 import os
 import platform
 import sys
@@ -327,11 +328,14 @@ def rhs_bench(n_particles, n_dipoles=16, seed=13, cpu_particles=3):
     return json.dumps(out)
 
 
-def incidences():
+def incidences(n=64):
     """The 64 right-hand sides of the batching configuration: polar angles pi - theta_j, theta_j = j 60 deg / 31
-    (j = 0..31), azimuth 0, TE and TM."""
+    (j = 0..31), azimuth 0, TE and TM; where more than 64 are asked for, the same polar angles follow at further
+    azimuths (multiples of the golden angle), so that every one is distinct."""
     th = np.deg2rad(np.arange(32) * 60.0 / 31)
-    return [(np.pi - t, 0.0, pol) for t in th for pol in (0, 1)]
+    turns = max(1, -(-n // 64))
+    return [(np.pi - t, math.fmod(a * math.pi * (3 - math.sqrt(5)), 2 * math.pi), pol)
+            for a in range(turns) for t in th for pol in (0, 1)]
 
 
 def _child(args, timeout=600):
@@ -448,7 +452,7 @@ def main_headline(args):
 
     plist, ls, kp, side = build_workload(args.particles)
     log('workload: %d spheres, side %.0f nm, N_kappa %d' % (len(plist), side, len(kp)))
-    inc = incidences()
+    inc = incidences(args.batch * (args.warmup + args.steps))
     t0 = time.time()
     base = LinearSystem(plist, PlaneWave(WL, *inc[0]), ls, kp, solver_type='gmres', solver_tolerance=args.tol,
                         store_coupling_matrix=False, coupling_matrix_lookup_resolution=2.0, interpolator_kind='cubic',
@@ -459,12 +463,10 @@ def main_headline(args):
     t_diag = base.t_matrix.diagonal
     log('prepare %.2f s (table %.2f s), len_rho %d' % (prep_s, op.table_seconds, len(op.radial_distance_array)))
 
-    # right-hand sides (setup, outside the timed region): step j solves incidences nb j .. nb j + nb - 1 of the
-    # 64 distinct ones; T is the same for every incidence, rhs = T a
+    # right-hand sides (setup, outside the timed region): step j solves incidences nb j .. nb j + nb - 1; T is the
+    # same for every incidence, rhs = T a
     nb = args.batch
     n_rhs = nb * (args.warmup + args.steps)
-    if n_rhs > len(inc):
-        raise SystemExit('at most %d distinct right-hand sides (warmup + steps <= %d)' % (len(inc), len(inc) // nb))
     rhs = np.stack([t_diag * PlaneWave(WL, *inc[j]).swe_coefficients(plist, ls) for j in range(n_rhs)])
 
     tune = autotune(op, ((True, 'half'), (True, 'double'), (False, 'single')), not args.no_autotune)
@@ -748,9 +750,9 @@ def main_batching(args):
     prep = time.time() - t0
     log('%d ensembles (%d..%d spheres, %d total), table %.1f s, setup %.1f s'
         % (len(sizes), min(sizes), max(sizes), sum(sizes), batch.table_seconds, prep))
-    inc = incidences()
     nb = 8
     n_fields = nb * (args.warmup + args.steps)
+    inc = incidences(n_fields)
     t0 = time.time()
     rhs = batch.right_hand_sides([PlaneWave(WL, *inc[j]) for j in range(n_fields)])
     log('right-hand sides %.1f s' % (time.time() - t0))
