@@ -356,11 +356,16 @@ __global__ void __launch_bounds__(256) explicit_gemv_kernel(const void* __restri
 // steps and the two products keep sums of their own, the waves' sums are added
 // at the end. Bound by HBM on W, read once for all vectors: the next turn's
 // loads are in flight during the products, and eight waves of four such
-// workgroups keep about 130 KB per CU outstanding.
-constexpr int kGemmWaves = 8;
+// workgroups keep about 130 KB per CU outstanding. The columns are cut into
+// gridDim.y shares, whose sums explicit_gemm_sum_kernel adds: 9000 unknowns
+// are 563 workgroups for the rows alone, two on some CUs and three on others
+// (FP32: 264 us, 2.45 TB/s; with 4 shares 210 us, 3.1 TB/s; FP64 316 -> 252 us,
+// 5.1 TB/s).
+constexpr int kGemmWaves = 8, kGemmShares = 8;
 template <typename Real>
 __global__ void __launch_bounds__(64 * kGemmWaves)
     explicit_gemm_kernel(const void* __restrict__ Wv, const void* __restrict__ xv, void* __restrict__ yv, int64_t n) {
+  // yv: Y with one share of the columns, else the shares' sums [gridDim.y][n][16]
   using M = smh::Mfma<Real>;
   using R2 = typename smh::Vec2<Real>::t;
   constexpr int J = 64 / (int)sizeof(R2), kCols = 4 * J;  // columns per lane and per turn
@@ -400,14 +405,15 @@ __global__ void __launch_bounds__(64 * kGemmWaves)
     }
   };
   const int64_t turns = n / kCols;
-  if (wave < turns) {
+  const int64_t t0 = turns * blockIdx.y / gridDim.y + wave, t1 = turns * (blockIdx.y + 1) / gridDim.y;
+  if (t0 < t1) {
     R2 w[J];
     Real b[J];
-    load((int64_t)wave * kCols, w, b);
-    for (int64_t t = wave; t < turns; t += kGemmWaves) {
+    load(t0 * kCols, w, b);
+    for (int64_t t = t0; t < t1; t += kGemmWaves) {
       R2 w1[J];
       Real b1[J];
-      load((t + kGemmWaves < turns ? t + kGemmWaves : t) * kCols, w1, b1);
+      load((t + kGemmWaves < t1 ? t + kGemmWaves : t) * kCols, w1, b1);
       multiply(w, b);
 #pragma unroll
       for (int j = 0; j < J; ++j) {
@@ -416,7 +422,7 @@ __global__ void __launch_bounds__(64 * kGemmWaves)
       }
     }
   }
-  if (turns * kCols < n && wave == (int)(turns % kGemmWaves)) {  // the columns left over
+  if (turns * kCols < n && blockIdx.y == gridDim.y - 1 && wave == kGemmWaves - 1) {  // the columns left over
     R2 w[J];
     Real b[J];
 #pragma unroll
@@ -438,25 +444,54 @@ __global__ void __launch_bounds__(64 * kGemmWaves)
     Real s = part[0][r][k];
 #pragma unroll
     for (int w = 1; w < kGemmWaves; ++w) s += part[w][r][k];
-    if (row0 + r < n) ((Real*)yv)[(row0 + r) * 16 + k] = s;
+    if (row0 + r < n) ((Real*)yv)[((int64_t)blockIdx.y * n + row0 + r) * 16 + k] = s;
   }
+}
+
+template <typename Real>
+__global__ void explicit_gemm_sum_kernel(const Real* __restrict__ part, int64_t n16, int shares, Real* __restrict__ y) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= n16) return;
+  Real s = part[e];
+  for (int k = 1; k < shares; ++k) s += part[k * n16 + e];
+  y[e] = s;
 }
 
 }  // namespace
 
 namespace smh {
 
+// Column shares of explicit_gemm_kernel: eight workgroups per CU to even them
+// out, each with at least two turns per wave (fewer cost more than the sum's
+// launch saves).
+static int gemm_shares(const smh_op* op, int64_t n, int real_size) {
+  const int64_t groups = (n + 15) / 16, turns = n / (4 * (64 / (2 * real_size)));
+  const int64_t want = (8 * (int64_t)op->ctx->num_cu + groups - 1) / groups;
+  return (int)std::max<int64_t>(1, std::min({want, turns / (2 * kGemmWaves), (int64_t)kGemmShares}));
+}
+
+static size_t explicit_shares_bytes(const smh_op* op, int64_t n) {
+  return (size_t)n * 16 * std::max(gemm_shares(op, n, 4) * sizeof(float), gemm_shares(op, n, 8) * sizeof(double));
+}
+
+template <typename Real>
+static void launch_gemm(smh_op* op, const void* W, const void* x, void* y, int64_t n) {
+  const int shares = gemm_shares(op, n, sizeof(Real));
+  hipStream_t s = op->ctx->stream;
+  hipLaunchKernelGGL(explicit_gemm_kernel<Real>, dim3((unsigned)((n + 15) / 16), shares), dim3(64 * kGemmWaves), 0, s,
+                     W, x, shares > 1 ? (void*)op->d_ypart : y, n);
+  if (shares > 1)
+    hipLaunchKernelGGL(explicit_gemm_sum_kernel<Real>, dim3((unsigned)((n * 16 + 255) / 256)), dim3(256), 0, s,
+                       (const Real*)op->d_ypart, n * 16, shares, (Real*)y);
+}
+
 int explicit_apply_batch(smh_op* op, int precision, const void* x_pad, void* y_pad) {
-  smh_ctx* ctx = op->ctx;
   const int64_t n = op->n_part * op->B;
-  const dim3 grid((unsigned)((n + 15) / 16)), block(64 * kGemmWaves);
   if (precision == SMH_FP32)
-    hipLaunchKernelGGL(explicit_gemm_kernel<float>, grid, block, 0, ctx->stream, (const void*)op->d_W32, x_pad, y_pad,
-                       n);
+    launch_gemm<float>(op, op->d_W32, x_pad, y_pad, n);
   else
-    hipLaunchKernelGGL(explicit_gemm_kernel<double>, grid, block, 0, ctx->stream, (const void*)op->d_W64, x_pad,
-                       y_pad, n);
-  SMH_HIP(ctx, hipGetLastError());
+    launch_gemm<double>(op, op->d_W64, x_pad, y_pad, n);
+  SMH_HIP(op->ctx, hipGetLastError());
   return SMH_OK;
 }
 
@@ -663,7 +698,8 @@ extern "C" int smh_explicit_create(smh_ctx* ctx, int64_t n_part, const double* x
   if (hipMalloc(&op->d_W64, (size_t)n * n * sizeof(double2)) != hipSuccess ||
       hipMalloc(&op->d_W32, (size_t)n * n * sizeof(float2)) != hipSuccess ||
       hipMalloc(&op->d_x32, n * sizeof(float2)) != hipSuccess || hipMalloc(&op->d_y32, n * sizeof(float2)) != hipSuccess ||
-      hipMalloc(&op->d_x64, n * sizeof(double2)) != hipSuccess || hipMalloc(&op->d_y64, n * sizeof(double2)) != hipSuccess) {
+      hipMalloc(&op->d_x64, n * sizeof(double2)) != hipSuccess || hipMalloc(&op->d_y64, n * sizeof(double2)) != hipSuccess ||
+      hipMalloc(&op->d_ypart, smh::explicit_shares_bytes(op, n)) != hipSuccess) {
     smh_fail(ctx, SMH_ERR_HIP, "device allocation failed (dense matrix of %lld x %lld needs %.1f GB)", (long long)n,
              (long long)n, (double)n * n * 24 / 1e9);
     return fail(SMH_ERR_HIP);
