@@ -3,8 +3,9 @@
 // 259-268), which factors the stored master matrix once with LAPACK
 // (scipy lu_factor), keeps the factors and solves every right-hand side with
 // them (lu_solve). Here the master matrix M = 1 - diag(t) W is formed in FP64
-// from the device-resident explicit matrix, factored with partial pivoting by
-// rocSOLVER's getrf and solved by getrs, all on the device; the factors stay
+// from the device-resident explicit matrix, factored with partial pivoting (up
+// to 2048 unknowns by lu_step_kernel, beyond by rocSOLVER's getrf) and solved by
+// getrs, all on the device; the factors stay
 // on the operator for later right-hand sides with the same T. Every solution
 // is certified by its FP64 residual ||b - M x|| / ||b||, computed with the
 // explicit matvec.
@@ -71,6 +72,261 @@ __global__ void residual_parts_kernel(const double2* __restrict__ b, const doubl
   }
 }
 
+// ---- factorisation of matrices up to kLuRows * 2 rows ----------------------
+// Column-major A(i, j) = A[j n + i], in place, partial pivoting by |re| + |im|
+// (first of equals), LAPACK's factors and 1-based pivots. One launch per panel
+// of kLuPanel columns: workgroup 0 brings the next panel up to date and
+// factors it while the others bring the remaining columns up to date, a strip
+// of kLuPanel columns each, and exchange the rows of the columns before.
+// Bound by the chain of pivots: a panel's rows stay in the registers of one
+// workgroup (two per thread), so that a pivot costs two barriers and no memory
+// access. 1800 unknowns (60 spheres, l_max 3): 13.2 ms in some 4000 launches of
+// rocSOLVER's getrf, 5.4 ms in 226 launches here, 28 us with two rows per thread
+// and 19 with one; errors against 64 bits as getrf's (360 to 2016 unknowns). With more than 2048 rows the panel no
+// longer fits the registers, and a pass over the matrix per eight columns no
+// longer the last-level cache: getrf.
+constexpr int kLuPanel = 8, kLuRows = 1024, kLuWaves = kLuRows / 64;
+
+// Row exchanges of a panel, as one permutation of the rows it touches:
+// row[t] takes the value of row[src[t]]; row[j] = first column + j, j < width.
+struct LuPerm {
+  int count;
+  int row[2 * kLuPanel], src[2 * kLuPanel];
+};
+
+__device__ inline double2 cfma(double2 a, double2 l, double2 u) {  // a + l u
+  a.x = fma(l.x, u.x, a.x);
+  a.x = fma(-l.y, u.y, a.x);
+  a.y = fma(l.x, u.y, a.y);
+  a.y = fma(l.y, u.x, a.y);
+  return a;
+}
+
+// Largest key of the row of 16 lanes, in all of them
+template <int kCtrl>
+__device__ __forceinline__ unsigned long long max_dpp(unsigned long long k) {
+  const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(k & 0xffffffffu), kCtrl, 0xF, 0xF, false);
+  const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(k >> 32), kCtrl, 0xF, 0xF, false);
+  const unsigned long long o = ((unsigned long long)hi << 32) | lo;
+  return o > k ? o : k;
+}
+__device__ __forceinline__ unsigned long long max_row(unsigned long long k) {
+  k = max_dpp<0x128>(k);  // row_ror:8, 4, 2, 1
+  k = max_dpp<0x124>(k);
+  k = max_dpp<0x122>(k);
+  return max_dpp<0x121>(k);
+}
+__device__ __forceinline__ unsigned long long max_xor(unsigned long long k, int d) {
+  const unsigned long long o = __shfl_xor(k, d);
+  return o > k ? o : k;
+}
+
+__device__ inline double2 csub(double2 a, double2 l, double2 u) {  // a - l u
+  a.x = fma(-l.x, u.x, a.x);
+  a.x = fma(l.y, u.y, a.x);
+  a.y = fma(-l.x, u.y, a.y);
+  a.y = fma(-l.y, u.x, a.y);
+  return a;
+}
+
+// k: first column of the factored panel (strip k / kLuPanel), or -kLuPanel for
+// the first launch, which only factors strip 0. Rows below the panel number at
+// most R * kLuRows. Block b < gridDim.x takes strip k / kLuPanel + 1 (b = 0,
+// if there is one) or one of the others.
+template <int R>
+__global__ void __launch_bounds__(kLuRows) lu_step_kernel(double2* __restrict__ A, int64_t n, int k, LuPerm* perms,
+                                                          int* ipiv, int* info) {
+  __shared__ double2 sv[kLuPanel][2 * kLuPanel], us[kLuPanel][kLuPanel], l11[kLuPanel][kLuPanel];
+  __shared__ double2 prow[kLuPanel], orow[kLuPanel];
+  __shared__ unsigned long long redk[kLuWaves];
+  __shared__ int pivots[kLuPanel];
+  const int tid = threadIdx.x, N = (int)n, strips = (N + kLuPanel - 1) / kLuPanel;
+  const int sk = k >= 0 ? k / kLuPanel : -1;  // strip of the factored panel
+  int strip = sk + 1 < strips ? ((int)blockIdx.x == 0 ? sk + 1 : (int)blockIdx.x - 1) : (int)blockIdx.x;
+  if (sk + 1 < strips && blockIdx.x > 0 && strip >= sk) strip += sk >= 0 ? 2 : 1;
+  const int c0 = strip * kLuPanel, w = min(kLuPanel, N - c0);
+  const int wk = kLuPanel, row0 = k + wk;  // (a panel with strips after it is full)
+  double2* C = A + (int64_t)c0 * n;
+  if (k >= 0) {
+    // row exchanges of the strip
+    const LuPerm& pm = perms[sk];
+    const int r = tid & (2 * kLuPanel - 1), c = tid / (2 * kLuPanel), count = pm.count;
+    const bool mine = c < w && r < count;
+    if (mine) sv[c][r] = C[c * n + pm.row[r]];
+    if (strip > sk && tid < kLuPanel * kLuPanel) {
+      const int i = tid / kLuPanel, j = tid % kLuPanel;  // L(j, i) of the panel's triangle
+      l11[j][i] = A[(int64_t)(k + i) * n + k + j];
+    }
+    __syncthreads();
+    if (mine && (strip < sk || r >= wk)) C[c * n + pm.row[r]] = sv[c][pm.src[r]];
+    if (strip < sk) return;
+    // the strip's rows of U
+    if (tid < w) {
+      double2 u[kLuPanel];
+#pragma unroll
+      for (int j = 0; j < kLuPanel; ++j) {
+        u[j] = sv[tid][pm.src[j]];
+#pragma unroll
+        for (int i = 0; i < j; ++i) u[j] = csub(u[j], l11[j][i], u[i]);
+        us[j][tid] = u[j];
+        C[tid * n + k + j] = u[j];
+      }
+    }
+    __syncthreads();
+    // the rows below: C -= L U
+    double2 l[R][kLuPanel];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const int i = row0 + tid + q * kLuRows;
+#pragma unroll
+      for (int j = 0; j < kLuPanel; ++j) l[q][j] = i < N ? A[(int64_t)(k + j) * n + i] : make_double2(0.0, 0.0);
+    }
+#pragma unroll
+    for (int cc = 0; cc < kLuPanel; ++cc) {
+      if (cc >= w) break;
+      double2 v[R];
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const int i = row0 + tid + q * kLuRows;
+        v[q] = i < N ? C[cc * n + i] : make_double2(0.0, 0.0);
+      }
+      // (the products are summed first: one rounding of C per panel, not one per column)
+      double2 s[R];
+#pragma unroll
+      for (int q = 0; q < R; ++q) s[q] = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int j = 0; j < kLuPanel; ++j) {
+        const double2 u = us[j][cc];
+#pragma unroll
+        for (int q = 0; q < R; ++q) s[q] = cfma(s[q], l[q][j], u);
+      }
+#pragma unroll
+      for (int q = 0; q < R; ++q) v[q] = make_double2(v[q].x - s[q].x, v[q].y - s[q].y);
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        const int i = row0 + tid + q * kLuRows;
+        if (i < N) C[cc * n + i] = v[q];
+      }
+    }
+    if (strip != sk + 1) return;
+  }
+  // factor the strip: row row0 + tid + q kLuRows in a[q] (row0 = c0; written above by this thread)
+  double2 a[R][kLuPanel];
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int i = row0 + tid + q * kLuRows;
+#pragma unroll
+    for (int cc = 0; cc < kLuPanel; ++cc) a[q][cc] = cc < w && i < N ? C[cc * n + i] : make_double2(0.0, 0.0);
+  }
+#pragma unroll
+  for (int j = 0; j < kLuPanel; ++j) {
+    if (j >= w) break;
+    // pivot: the largest |re| + |im| of the rows from j on, by its upper 32 bits (a row within
+    // 1e-6 of the largest serves as well), the first of equals
+    unsigned long long key = 0xffffffffu - (unsigned)j;
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const int i = tid + q * kLuRows;
+      const double v = fabs(a[q][j].x) + fabs(a[q][j].y);
+      const unsigned long long kq =
+          ((unsigned long long)__double_as_longlong(v) & ~0xffffffffull) | (0xffffffffu - (unsigned)i);
+      if (i >= j && row0 + i < N && v >= 0.0 && kq > key) key = kq;
+    }
+    key = max_xor(max_xor(max_row(key), 16), 32);
+    if ((tid & 63) == 0) redk[tid >> 6] = key;
+    __syncthreads();
+    key = max_row(redk[tid & (kLuWaves - 1)]);
+    const int at = (int)(0xffffffffu - (unsigned)(key & 0xffffffffu));
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+      if (tid + q * kLuRows == at) {
+#pragma unroll
+        for (int cc = 0; cc < kLuPanel; ++cc) prow[cc] = a[q][cc];
+      }
+    if (tid == j) {
+#pragma unroll
+      for (int cc = 0; cc < kLuPanel; ++cc) orow[cc] = a[0][cc];
+      pivots[j] = row0 + at;
+      ipiv[c0 + j] = row0 + at + 1;
+    }
+    __syncthreads();
+    if (at != j) {
+      if (tid == j) {
+#pragma unroll
+        for (int cc = 0; cc < kLuPanel; ++cc) a[0][cc] = prow[cc];
+      }
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+        if (tid + q * kLuRows == at) {
+#pragma unroll
+          for (int cc = 0; cc < kLuPanel; ++cc) a[q][cc] = orow[cc];
+        }
+    }
+    // 1 / pivot, scaled by a power of two (a zero pivot is reported and leaves its column)
+    const double2 p = prow[j];
+    const bool zero = p.x == 0.0 && p.y == 0.0;
+    if (zero && tid == 0 && *info == 0) *info = c0 + j + 1;
+    const int e = zero ? 0 : -ilogb(fmax(fabs(p.x), fabs(p.y)));
+    const double px = ldexp(p.x, e), py = ldexp(p.y, e);
+    const double d = zero ? 0.0 : 1.0 / (px * px + py * py);
+    const double ix = ldexp(px * d, e), iy = -ldexp(py * d, e);
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      if (tid + q * kLuRows <= j) continue;
+      const double2 v = a[q][j];
+      const double2 lv = make_double2(v.x * ix - v.y * iy, v.x * iy + v.y * ix);
+      a[q][j] = lv;
+#pragma unroll
+      for (int cc = j + 1; cc < kLuPanel; ++cc) a[q][cc] = csub(a[q][cc], lv, prow[cc]);
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < R; ++q) {
+    const int i = row0 + tid + q * kLuRows;
+#pragma unroll
+    for (int cc = 0; cc < kLuPanel; ++cc)
+      if (cc < w && i < N) C[cc * n + i] = a[q][cc];
+  }
+  if (tid < 64) {
+    // the exchanges as one permutation: lane t holds row[t] and src[t]
+    int count = w, row = tid < w ? c0 + tid : -1, src = tid;
+    for (int j = 0; j < w; ++j) {
+      const int pj = pivots[j];
+      const unsigned long long there = __ballot(row == pj);
+      int b = count;
+      if (there) {
+        b = __ffsll((long long)there) - 1;
+      } else {
+        if (tid == count) row = pj;
+        ++count;
+      }
+      const int sj = __shfl(src, j), sb = __shfl(src, b);
+      if (tid == j) src = sb;
+      if (tid == b) src = sj;
+    }
+    LuPerm& pm = perms[strip];
+    if (tid < count) {
+      pm.row[tid] = row;
+      pm.src[tid] = src;
+    }
+    if (tid == 0) pm.count = count;
+  }
+}
+
+// ipiv [n], info [1] and perms [strips] on the device; info is the first zero
+// pivot's column (1-based), or 0
+void lu_factor(double2* A, int64_t n, int* ipiv, int* info, LuPerm* perms, hipStream_t s) {
+  const int strips = (int)((n + kLuPanel - 1) / kLuPanel);
+  (void)hipMemsetAsync(info, 0, sizeof(int), s);
+  for (int st = -1; st < strips; ++st) {
+    const int k = st * kLuPanel;
+    const int blocks = st < 0 ? 1 : strips - 1;  // all strips but the factored one
+    if (blocks == 0) break;
+    const auto kern = n - (k + kLuPanel) > kLuRows ? lu_step_kernel<2> : lu_step_kernel<1>;
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(kLuRows), 0, s, A, n, k, perms, ipiv, info);
+  }
+}
+
 }  // namespace
 
 namespace smh {
@@ -105,9 +361,10 @@ int lu_solve(smh_op* op, const double* t_diag, const double* rhs, double* x, int
   double2 *d_t = nullptr, *d_b = nullptr, *d_x = nullptr, *d_y = nullptr;
   double* d_parts = nullptr;
   int* d_info = nullptr;
+  LuPerm* d_perms = nullptr;
   constexpr int kParts = 256;
   auto done = [&](int code) {
-    void* p[] = {d_t, d_b, d_x, d_y, d_parts, d_info};
+    void* p[] = {d_t, d_b, d_x, d_y, d_parts, d_info, d_perms};
     for (void* q : p)
       if (q) (void)hipFree(q);
     return code;
@@ -144,10 +401,17 @@ int lu_solve(smh_op* op, const double* t_diag, const double* rhs, double* x, int
     hipLaunchKernelGGL(master_dense_kernel, dim3(blocks_of(n * n)), dim3(256), 0, s, (const double2*)op->d_W64,
                        (const double2*)d_t, n, op->d_lu);
     LU_HIP(hipGetLastError());
-    const rocblas_status st = rocsolver_zgetrf(h, (rocblas_int)n, (rocblas_int)n,
-                                               reinterpret_cast<rocblas_double_complex*>(op->d_lu), (rocblas_int)n,
-                                               op->d_piv, d_info);
-    if (st != rocblas_status_success) return done(smh_fail(ctx, SMH_ERR_HIP, "rocsolver_zgetrf failed (%d)", (int)st));
+    if (n <= 2 * kLuRows) {
+      LU_HIP(hipMalloc(&d_perms, (size_t)((n + kLuPanel - 1) / kLuPanel) * sizeof(LuPerm)));
+      lu_factor(op->d_lu, n, op->d_piv, d_info, d_perms, s);
+      LU_HIP(hipGetLastError());
+    } else {
+      const rocblas_status st = rocsolver_zgetrf(h, (rocblas_int)n, (rocblas_int)n,
+                                                 reinterpret_cast<rocblas_double_complex*>(op->d_lu), (rocblas_int)n,
+                                                 op->d_piv, d_info);
+      if (st != rocblas_status_success)
+        return done(smh_fail(ctx, SMH_ERR_HIP, "rocsolver_zgetrf failed (%d)", (int)st));
+    }
     int info = 0;
     LU_HIP(hipMemcpyAsync(&info, d_info, sizeof(int), hipMemcpyDeviceToHost, s));
     LU_HIP(hipStreamSynchronize(s));
