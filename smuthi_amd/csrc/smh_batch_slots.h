@@ -105,8 +105,8 @@ void slot_tables(int* out) {
 // of the result tiles (a tile's Re and Im rows together) within 128 registers,
 // each rotating and adding its own rows (2501 spheres, l_max 4, 3 parts: a
 // block product takes 17.0 ms, 18.4 with parts of the K-steps, which repeat the
-// rotation and the LDS additions of all rows). FP64: P64 parts of an even number of K-steps within
-// 64 values (10000 spheres, l_max 3, 2 parts: 184 ms, 199 with parts of the
+// rotation and the LDS additions of all rows). FP64: P64 parts of an even
+// number of K-steps within 64 values (10000 spheres, l_max 3, 2 parts: 184 ms, 199 with parts of the
 // tiles, which repeat the input's loads and rotation).
 template <int L, int M, int T>
 struct SlotShape {

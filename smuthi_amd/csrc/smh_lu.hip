@@ -82,8 +82,8 @@ __global__ void residual_parts_kernel(const double2* __restrict__ b, const doubl
 // workgroup (two per thread), so that a pivot costs two barriers and no memory
 // access. 1800 unknowns (60 spheres, l_max 3): 13.2 ms in some 4000 launches of
 // rocSOLVER's getrf, 5.4 ms in 226 launches here, 28 us with two rows per thread
-// and 19 with one; errors against 64 bits as getrf's (360 to 2016 unknowns). With more than 2048 rows the panel no
-// longer fits the registers, and a pass over the matrix per eight columns no
+// and 19 with one; errors against 64 bits as getrf's (80 to 2016 unknowns). With
+// more than 2048 rows the panel no longer fits the registers, and a pass over the matrix per eight columns no
 // longer the last-level cache: getrf.
 constexpr int kLuPanel = 8, kLuRows = 1024, kLuWaves = kLuRows / 64;
 
