@@ -142,6 +142,14 @@ __host__ __device__ inline int order_for(const double* limit, double z) {
   return m;  // kMaxM where z is beyond the table
 }
 
+// 2^e; FP32: the whole part of e goes into the exponent field, so that e may be large (rounded to FP32 as a
+// whole it would cost 6e-8 |e| of the result)
+__device__ inline double exp2_split(double e, double) { return exp2(e); }
+__device__ inline float exp2_split(double e, float) {
+  const double w = rint(fmax(-1e4, fmin(1e4, e)));
+  return ldexpf(PweMath<float>::exp2_((float)(e - w)), (int)w);
+}
+
 // Host: the order a leaf with largest |kappa| R = z needs, -1 beyond kMaxM.
 int max_order(int precision, double z) {
   static const double limit32[kMaxM + 1] = {SMH_ORDER_LIMIT_32}, limit64[kMaxM + 1] = {SMH_ORDER_LIMIT_64};
@@ -938,11 +946,16 @@ extern "C" int smh_pwe_field(smh_ctx* ctx, int kind, int64_t n_k, const double* 
 // FP64 sincos of the phases (about 60 instructions per particle and alpha)
 // beside as much time in the MFMA: 90 x 361 waves, 1000 particles, l_max 3, FP64:
 // 1.34 ms when a thread summed all orders of one alpha in registers.
+// FP32 sums go through the sum over m into FP64 ones every kAsmFlush particles:
+// where the waves alone fill the chip, one workgroup sums all particles, and one
+// running FP32 sum of 10000 of them is off by 2.5e-6 (1000 x 361 waves over 60 um,
+// 15.3 ms), in this form by 3.0e-7 (16.7 ms).
 // A launch covers kAsmOrders orders m at most; more run as several launches,
 // each adding its orders' share into g.
 namespace {
 
 constexpr int kAsmChunk = 32;   // particles staged at a time
+constexpr int kAsmFlush = 4 * kAsmChunk;  // particles of one FP32 sum
 constexpr int kAsmTiles = 2;    // alpha tiles per wave
 constexpr int kAsmWaves = 4;
 constexpr int kAsmOrders = 12;  // orders per launch: 4 (dir, pol) each in 3 column tiles
@@ -966,18 +979,19 @@ struct AsmArgs {
 
 // CT: tiles of 16 columns (m, q), q = (dir, pol), of the real and of the imaginary parts
 template <typename Real, int CT>
-__global__ void __launch_bounds__(64 * kAsmWaves) pwe_assemble_kernel(AsmArgs a) {
+__global__ void __launch_bounds__(64 * kAsmWaves, sizeof(Real) == 4 ? 3 : 2) pwe_assemble_kernel(AsmArgs a) {
   using M = smh::Mfma<Real>;
   constexpr int Q = 4, SC = CT * 16 + 16;  // (the row stride puts neighbouring particles in other banks)
   __shared__ Real cr[kAsmChunk][SC], ci[kAsmChunk][SC];
   __shared__ double px[kAsmChunk], py[kAsmChunk];
   __shared__ double2 ez[kAsmChunk][2];
-  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, h = lane >> 4;
+  __shared__ double2 em[kAsmWaves][kAsmTiles * 16][4 * CT];  // e^{i m alpha}, each wave's alphas and all orders
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, c = lane & 15, h = lane >> 4;
   const int k = (int)(blockIdx.x / a.a_blocks), ab = (int)(blockIdx.x - k * a.a_blocks);
-  const int tile0 = (ab * (int)(blockDim.x >> 6) + (tid >> 6)) * kAsmTiles;
+  const int tile0 = (ab * (int)(blockDim.x >> 6) + wave) * kAsmTiles;
   const double2 kp = a.kp[k], kz = a.kz[k];
   const double kturn = -kp.x / kTwoPi;        // e^{-i kappa s}: turns per nm
-  const Real klog = (Real)(kp.y * kLog2e);    // |e^{-i kappa s}| = 2^(klog s)
+  const double klog = kp.y * kLog2e;          // |e^{-i kappa s}| = 2^(klog s)
   const bool lossy = kp.y != 0.0;
   // this lane's alpha of each tile
   double ca[kAsmTiles], sa[kAsmTiles];
@@ -991,6 +1005,33 @@ __global__ void __launch_bounds__(64 * kAsmWaves) pwe_assemble_kernel(AsmArgs a)
   for (int t = 0; t < kAsmTiles; ++t)
 #pragma unroll
     for (int j = 0; j < CT; ++j) ar[t][j] = ai[t][j] = typename M::v4{0, 0, 0, 0};
+  for (int w = lane; w < kAsmTiles * 16 * 4 * CT; w += 64) {
+    const int r = w / (4 * CT), m = w - r * (4 * CT), ia = tile0 * 16 + r;
+    double es, ec;
+    sincos((double)(m + a.m_first) * (ia < a.n_a ? a.alpha[ia] : 0.0), &es, &ec);
+    em[wave][r][m] = make_double2(ec, es);
+  }
+  // the lane's share (its columns' orders) of the sum over m of e^{i m alpha}, and the running sums cleared
+  double gr[kAsmTiles][4], gi[kAsmTiles][4];
+#pragma unroll
+  for (int t = 0; t < kAsmTiles; ++t)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) gr[t][v] = gi[t][v] = 0.0;
+  auto flush = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < kAsmTiles; ++t)
+#pragma unroll
+      for (int j = 0; j < CT; ++j) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const double2 e = em[wave][t * 16 + (M::kRowIs4q ? 4 * h + v : 4 * v + h)][4 * j + (c >> 2)];
+          const double re = (double)ar[t][j][v], im = (double)ai[t][j][v];
+          gr[t][v] += re * e.x - im * e.y;
+          gi[t][v] += re * e.y + im * e.x;
+        }
+        ar[t][j] = ai[t][j] = typename M::v4{0, 0, 0, 0};
+      }
+  };
   const int64_t first = (int64_t)blockIdx.y * a.per_split;
   const int64_t last = first + a.per_split < a.n_part ? first + a.per_split : a.n_part;
   for (int64_t p0 = first; p0 < last; p0 += kAsmChunk) {
@@ -1030,6 +1071,7 @@ __global__ void __launch_bounds__(64 * kAsmWaves) pwe_assemble_kernel(AsmArgs a)
     }
     __syncthreads();
     if (tile0 * 16 >= a.n_a) continue;
+    if (sizeof(Real) == 4 && p0 > first && (p0 - first) % kAsmFlush == 0) flush();
     for (int s = 0; s < (np + 3) / 4; ++s) {
       const int p = 4 * s + h;  // (particles beyond np have zero coefficients)
       Real br[CT], bi[CT];
@@ -1044,7 +1086,7 @@ __global__ void __launch_bounds__(64 * kAsmWaves) pwe_assemble_kernel(AsmArgs a)
         Real pr, pi;
         cis_turns(kturn * sd, pr, pi);
         if (lossy) {
-          const Real mg = PweMath<Real>::exp2_(klog * (Real)sd);
+          const Real mg = exp2_split(klog * sd, Real(0));
           pr *= mg;
           pi *= mg;
         }
@@ -1058,28 +1100,20 @@ __global__ void __launch_bounds__(64 * kAsmWaves) pwe_assemble_kernel(AsmArgs a)
       }
     }
   }
-  // sum over m of e^{i m alpha}: the lane's columns of each alpha, then the lanes of the same q
+  flush();
+  // the lanes of the same q
 #pragma unroll
   for (int t = 0; t < kAsmTiles; ++t)
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
       const int ia = (tile0 + t) * 16 + (M::kRowIs4q ? 4 * h + v : 4 * v + h);
-      const double al = ia < a.n_a ? a.alpha[ia] : 0.0;
-      double gr = 0, gi = 0;
-#pragma unroll
-      for (int j = 0; j < CT; ++j) {
-        double es, ec;
-        sincos((double)(4 * j + (c >> 2) + a.m_first) * al, &es, &ec);
-        gr += (double)ar[t][j][v] * ec - (double)ai[t][j][v] * es;
-        gi += (double)ar[t][j][v] * es + (double)ai[t][j][v] * ec;
-      }
 #pragma unroll
       for (int off = 4; off < 16; off <<= 1) {
-        gr += __shfl_xor(gr, off);
-        gi += __shfl_xor(gi, off);
+        gr[t][v] += __shfl_xor(gr[t][v], off);
+        gi[t][v] += __shfl_xor(gi[t][v], off);
       }
       if (c < Q && ia < a.n_a)
-        a.part[(((size_t)blockIdx.y * Q + c) * a.n_k + k) * a.n_a + ia] = make_double2(gr, gi);
+        a.part[(((size_t)blockIdx.y * Q + c) * a.n_k + k) * a.n_a + ia] = make_double2(gr[t][v], gi[t][v]);
     }
 }
 
