@@ -45,12 +45,22 @@ class _Scatterers:
             self.coefficients[np.asarray(idx)[:, None], np.asarray(dst)[None, :]] = block[:, src]
 
 
+def _layer_numbers(layer_system, z):
+    """layer_system.layer_number of every height. One search finds them all where that is LayerSystem's own; a
+    layer system of another class, or with a layer_number of its own, is asked height by height."""
+    ask = layer_system.layer_number
+    if (isinstance(layer_system, lay.LayerSystem) and getattr(ask, '__func__', None) is lay.LayerSystem.layer_number
+            and ask.__self__ is layer_system):
+        return layer_system.layer_numbers(z)
+    return np.array([ask(h) for h in z])
+
+
 def _by_layer(particle_list, layer_system):
     """[(layer, its particles, their positions)] in the order of the layers."""
     if not len(particle_list):
         return []
     xyz = np.array([p.position for p in particle_list], dtype=np.float64)
-    layers = layer_system.layer_numbers(xyz[:, 2])
+    layers = _layer_numbers(layer_system, xyz[:, 2])
     out = []
     for i in np.unique(layers):
         idx = np.flatnonzero(layers == i)

@@ -1,0 +1,124 @@
+"""The host side of the scattered field's plane wave expansions (grouping by
+layer, direct and layer-mediated terms, far field) with the device's particle sum
+stubbed by random numbers that depend on its input: the sums against the same
+terms as expansions of their own, responded to by layer_response and added by
+PlaneWaveExpansion's checked sum, equal to the last bit, for particles in several
+layers."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from smuthi_amd import far_field, scattered_field
+from smuthi_amd.expansions import PlaneWaveExpansion, SphericalWaveExpansion, layer_response
+from smuthi_amd.layers import LayerSystem
+from smuthi_amd.particles import Sphere
+
+WL = 550.0
+SYSTEMS = [([0, 0], [1.52, 1]), ([0, 400, 0], [1.5, 2 + 0.01j, 1]), ([0, 300, 200, 0], [1.5, 1.8, 1.3, 1.0])]
+KP, AL = np.linspace(0, 0.02, 7) - 1e-4j, np.linspace(0, 6, 5)
+
+
+class _Lib:
+    def smh_pwe_assemble(self, *a):
+        n, n_k, n_a = a[1], a[7], a[11]
+
+        def doubles(p, size):
+            return np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_double)), (size,))
+        x, c = doubles(a[2], 3 * n), doubles(a[5], 8)
+        doubles(a[13], 8 * n_k * n_a)[:] = np.random.default_rng(
+            int(abs(x.sum() * 1e3) + abs(c.sum()) * 1e6)).standard_normal(8 * n_k * n_a)
+        return 0
+
+
+@pytest.fixture(autouse=True)
+def host_assembly(monkeypatch):
+    monkeypatch.setattr(scattered_field._lib, 'load', lambda: _Lib())
+    monkeypatch.setattr(scattered_field.cu, 'context', lambda: None)
+
+
+def _particles(thicknesses, seed=0):
+    rng = np.random.default_rng(seed)
+    top = float(sum(thicknesses))
+    heights = [top + 100.0, top, 150.0, top + 220.0] if top else [100.0, 130.0]  # (one on an interface)
+    parts = []
+    for i in range(12):
+        l_max = int(rng.integers(1, 4))
+        p = Sphere([1e3 * rng.random(), 1e3 * rng.random(), heights[i % len(heights)]], 1.5, 40, l_max, min(l_max, 2))
+        p.scattered_field = SphericalWaveExpansion(1.0, l_max, min(l_max, 2), 'outgoing', p.position, 0, np.inf)
+        n = len(p.scattered_field.coefficients)
+        p.scattered_field.coefficients = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+        parts.append(p)
+    return parts
+
+
+def _by_terms(parts, ls, layer, direct, response):
+    """Every term an expansion of its own, added with PlaneWaveExpansion's checks."""
+    om = 2 * np.pi / WL
+    bounds = (ls.lower_zlimit(layer), ls.upper_zlimit(layer))
+    ref = [0, 0, ls.reference_z(layer)]
+    up, dn = (PlaneWaveExpansion(om * ls.refractive_indices[layer], KP, AL, kind, ref, *bounds)
+              for kind in ('upgoing', 'downgoing'))
+    layers = [ls.layer_number(p.position[2]) for p in parts]
+    for i in sorted(set(layers)):
+        group = [p for p, q in zip(parts, layers) if q == i]
+        if not (direct and i == layer or response):
+            continue
+        s = scattered_field._Scatterers(group, np.array([p.position for p in group], dtype=float))
+        gu, gd, k, kp, al, _ = scattered_field._assemble(WL, s, ls, i, KP, AL, 'double')
+        z = [p.position[2] for p in group]
+        ref_i = [0, 0, ls.reference_z(i)]
+        pu = PlaneWaveExpansion(k, kp, al, 'upgoing', ref_i, max(z), ls.upper_zlimit(i))
+        pd = PlaneWaveExpansion(k, kp, al, 'downgoing', ref_i, ls.lower_zlimit(i), min(z))
+        pu.coefficients, pd.coefficients = gu, gd
+        if direct and i == layer:
+            up, dn = up + pu, dn + pd
+        if response:
+            ru, rd = layer_response(ls, (pu, pd), i, layer)
+            up, dn = up + ru, dn + rd
+    return up, dn
+
+
+@pytest.mark.parametrize('system', SYSTEMS)
+def test_sums_equal_the_terms_one_by_one(system):
+    ls = LayerSystem(*system)
+    parts = _particles(system[0])
+    for layer in range(ls.number_of_layers()):
+        for direct, response in ((True, True), (True, False), (False, True)):
+            got = scattered_field.scattered_field_pwe(WL, parts, ls, layer, KP, AL, direct, response, 'double')
+            for g, w in zip(got, _by_terms(parts, ls, layer, direct, response)):
+                assert np.array_equal(g.coefficients, w.coefficients)
+                assert (g.lower_z, g.upper_z) == (w.lower_z, w.upper_z)
+                assert g.kind == w.kind and np.isclose(g.k, w.k)
+
+
+class _Duck:
+    """A smuthi-shaped layer system: LayerSystem's attributes, layer_number and nothing beyond."""
+
+    def __init__(self, *system):
+        ls = LayerSystem(*system)
+        self.thicknesses, self.refractive_indices = ls.thicknesses, ls.refractive_indices
+        for name in ('number_of_layers', 'lower_zlimit', 'upper_zlimit', 'reference_z', 'layer_number', 'wavenumber'):
+            setattr(self, name, getattr(ls, name))
+
+
+class _LowerOnInterfaces(LayerSystem):
+    """Points on an interface count as below it."""
+
+    def layer_number(self, z):
+        return LayerSystem.layer_number(self, np.nextafter(z, -np.inf))
+
+
+@pytest.mark.parametrize('kind', [_Duck, _LowerOnInterfaces])
+@pytest.mark.parametrize('system', SYSTEMS)
+def test_layer_systems_of_the_users_own(kind, system):
+    ls = kind(*system)
+    parts = _particles(system[0])
+    for layer in range(ls.number_of_layers()):
+        got = scattered_field.scattered_field_pwe(WL, parts, ls, layer, KP, AL, precision='double')
+        for g, w in zip(got, _by_terms(parts, ls, layer, True, True)):
+            assert np.array_equal(g.coefficients, w.coefficients)
+    sfld = scattered_field.scattered_field_piecewise_expansion(WL, parts, ls, KP, AL)
+    spheres = [e for e in sfld.expansion_list if not isinstance(e, PlaneWaveExpansion)]
+    assert len(spheres) == len({ls.layer_number(p.position[2]) for p in parts})
+    far_field.scattered_far_field(WL, parts, ls, np.linspace(0, np.pi, 9), AL)
