@@ -57,7 +57,8 @@ def _layer_numbers(layer_system, z):
 
 def _by_layer(particle_list, layer_system):
     """[(layer, its particles, their positions)] in the order of the layers."""
-    if not len(particle_list):
+    particle_list = list(particle_list)
+    if not particle_list:
         return []
     xyz = np.array([p.position for p in particle_list], dtype=np.float64)
     layers = _layer_numbers(layer_system, xyz[:, 2])
@@ -158,6 +159,7 @@ def scattered_field_piecewise_expansion(vacuum_wavelength, particle_list, layer_
     if layer_numbers is None:
         layer_numbers = range(layer_system.number_of_layers())
     nl = layer_system.number_of_layers()
+    particle_list = list(particle_list)
     sfld = PiecewiseFieldExpansion()
     for i in layer_numbers:
         up, dn = scattered_field_pwe(vacuum_wavelength, particle_list, layer_system, i, k_parallel, azimuthal_angles,

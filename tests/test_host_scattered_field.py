@@ -122,3 +122,21 @@ def test_layer_systems_of_the_users_own(kind, system):
     spheres = [e for e in sfld.expansion_list if not isinstance(e, PlaneWaveExpansion)]
     assert len(spheres) == len({ls.layer_number(p.position[2]) for p in parts})
     far_field.scattered_far_field(WL, parts, ls, np.linspace(0, np.pi, 9), AL)
+
+
+@pytest.mark.parametrize('wrap', [iter, tuple, lambda parts: dict(enumerate(parts)).values(),
+                                  lambda parts: np.array(parts, dtype=object)])
+def test_particles_of_any_iterable(wrap):
+    ls = LayerSystem(*SYSTEMS[2])
+    parts = _particles(SYSTEMS[2][0])
+    want = scattered_field.scattered_field_pwe(WL, parts, ls, 2, KP, AL)
+    got = scattered_field.scattered_field_pwe(WL, wrap(parts), ls, 2, KP, AL)
+    assert all(np.array_equal(g.coefficients, w.coefficients) for g, w in zip(got, want))
+    polar = np.linspace(0, np.pi, 9)
+    want = far_field.scattered_far_field(WL, parts, ls, polar, AL)
+    got = far_field.scattered_far_field(WL, wrap(parts), ls, polar, AL)
+    assert np.array_equal(got.amplitude, want.amplitude)
+    want = scattered_field.scattered_field_piecewise_expansion(WL, parts, ls, KP, AL)
+    got = scattered_field.scattered_field_piecewise_expansion(WL, wrap(parts), ls, KP, AL)
+    assert len(got.expansion_list) == len(want.expansion_list)
+    assert len(got.validity_conditions) == len(parts)
