@@ -132,7 +132,10 @@ def _scattered_field_pwe(vacuum_wavelength, by_layer, scatterers, layer_system, 
         *g, k_swe, kp, al, ms = _assemble(vacuum_wavelength, scatterers[i_swe], layer_system, i_swe, k_parallel,
                                           azimuthal_angles, precision)
         scattered_field_pwe.last_kernel_ms += ms
-        if not out[0].compatible(out[0]):
+        # the terms' common grids (the assembly's), wavenumber and reference point, as PlaneWaveExpansion.__add__
+        # checks them
+        n = layer_system.refractive_indices
+        if not out[0].compatible(PlaneWaveExpansion(k_swe / n[i_swe] * n[layer_number], kp, al, 'upgoing', [0, 0, z])):
             raise ValueError('Plane wave expansion are inconsistent.')
         if direct:
             out[0].lower_z, out[1].upper_z = max(vb[0], xyz[:, 2].max()), min(vb[1], xyz[:, 2].min())

@@ -140,3 +140,15 @@ def test_particles_of_any_iterable(wrap):
     got = scattered_field.scattered_field_piecewise_expansion(WL, wrap(parts), ls, KP, AL)
     assert len(got.expansion_list) == len(want.expansion_list)
     assert len(got.validity_conditions) == len(parts)
+
+
+@pytest.mark.filterwarnings('ignore')
+@pytest.mark.parametrize('k_parallel,azimuth', [
+    (KP, AL + 0.3j), (np.where(np.arange(7) == 3, np.nan, KP), AL), (KP, np.where(np.arange(5) == 3, np.nan, AL))])
+@pytest.mark.parametrize('layer,direct,response', [(1, True, True), (1, True, False), (2, False, True)])
+def test_inconsistent_grids_are_refused(k_parallel, azimuth, layer, direct, response):
+    """Angles of which the assembly takes the real part, numbers that do not equal themselves."""
+    ls = LayerSystem([0, 400, 0], [1.5, 2, 1])
+    parts = [p for p in _particles([0, 400, 0]) if ls.layer_number(p.position[2]) == 1]
+    with pytest.raises(ValueError, match='inconsistent'):
+        scattered_field.scattered_field_pwe(WL, parts, ls, layer, k_parallel, azimuth, direct, response)
