@@ -327,8 +327,10 @@ __global__ void vol_slot_taps64_kernel(const float2* __restrict__ table, const d
 // The same rows in FP16 in the fragment order of vol_half_kernel:
 // [rows][MT][64 lanes][NC][4], lane (q, rr) of tile i holding
 // A(slot 16 (i mod MH) + rr, slot 16 c + 4 q + j) / hs[row], hs[row] the
-// smallest power of two with max |A| / hs <= 2^12 over the row; one block
-// per row.
+// smallest power of two with max |A| / hs <= 2^12 over the row, for a row of
+// zeros (distances below the smallest of the pairs) the smallest there is: the
+// kernels weight the rows of a pair relative to the largest scale among them,
+// which a row without values must not set; one block per row.
 __global__ void vol_half_taps_kernel(const float2* __restrict__ table, const double2* __restrict__ mr,
                                      const double2* __restrict__ mz, const double2* __restrict__ mrz, int vq, int B,
                                      int S, const int* __restrict__ n_of, _Float16* th, float* hs) {
@@ -369,7 +371,7 @@ __global__ void vol_half_taps_kernel(const float2* __restrict__ table, const dou
     __syncthreads();
   }
   const double mx = red[0];
-  const int e = mx > 0.0 ? (int)ceil(log2(mx)) - 12 : 0;
+  const int e = mx > 0.0 ? (int)ceil(log2(mx)) - 12 : -126;
   const double inv = ldexp(1.0, -e);
   if (threadIdx.x == 0) hs[row] = ldexpf(1.0f, e);
   for (int f = threadIdx.x; f < per_row; f += blockDim.x) th[row * per_row + f] = (_Float16)(value(f) * inv);
