@@ -2,9 +2,13 @@
 in one workgroup (up to 4096 unknowns, edge at 682 / 683 particles of 6), the
 several-launch step above, restart lengths from one step to the largest basis,
 and repeated solves (the first runs eagerly, the second captures its graphs,
-the third replays them, with eager matvecs between). The residual is taken
+the third replays them, with eager matvecs between), and solves of different
+operators by several threads on the context's one stream, while graphs are
+captured. The residual is taken
 with the plain numpy operator of the partial-sum tests; an FP64 solve to tol
 leaves tol plus the FP64 operators' own difference (1e-13)."""
+import threading
+
 import numpy as np
 import pytest
 
@@ -42,3 +46,44 @@ def test_single_solves_meet_the_tolerance(gpu, n, restart):
             first = x if first is None else first
             assert np.linalg.norm(x - first) <= 1e-8 * np.linalg.norm(first)
         op.matvec(b, 'single')
+
+
+def test_threads_solve_while_others_capture(gpu):
+    """Each thread solves with operators of its own, one to three right-hand sides, every operator four times: the
+    second run of each step captures its graph while the other threads launch on the same stream."""
+    from smuthi_amd.linear_system import CouplingMatrixRadialLookupCUDA
+
+    def system(n):
+        xy, rho, table = _system(n, n)
+        op = CouplingMatrixRadialLookupCUDA.from_table(table, rho, [Sphere([a, b, 200.0], 1.5, 50.0, 1, 1)
+                                                                    for a, b in xy], H, 'linear')
+        rng = np.random.default_rng(n)
+        d = np.hypot(xy[:, None, 0] - xy[None, :, 0], xy[:, None, 1] - xy[None, :, 1])
+        t = (0.25 / (6 * (1 / (1 + d / 500)).sum(1).max()) * np.exp(2j * np.pi * rng.uniform(size=(n, 6)))).ravel()
+        b = rng.standard_normal((3, n * 6)) + 1j * rng.standard_normal((3, n * 6))
+        want = op.solve_master(t, b, 1e-10, precision='double')
+        return op, t, b, want
+
+    work = [[system(n) for n in sizes] for sizes in ((20, 90, 41), (33, 60, 25), (70, 28, 52))]
+    failures = []
+
+    def solve(systems):
+        try:
+            for op, t, b, want in systems:
+                for repeat in range(4):
+                    for rhs, ref in ((b[0], want[0]), (b, want)):
+                        for precision in ('double', 'mixed'):
+                            x = op.solve_master(t, rhs, 1e-8, precision=precision)
+                            err = np.linalg.norm(x - ref) / np.linalg.norm(ref)
+                            if not err <= 1e-7:
+                                failures.append((op.shape, repeat, precision, err))
+        except Exception as e:
+            failures.append(e)
+
+    threads = [threading.Thread(target=solve, args=(w,)) for w in work]
+    print('solves in %d threads' % len(threads), flush=True)
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures, failures
