@@ -548,7 +548,7 @@ struct Solver {
   hipStream_t s;
   SolveWs* ws;
   int64_t n, n8, per_part;  // padded length, times KB, elements per particle
-  int restart, nsys, nblk;
+  int restart, cap, nsys, nblk;  // cap: restart length that the workspace's arrays are laid out for
   bool use_P, small;
   int64_t mv64 = 0, mv32 = 0, mv16 = 0, iters = 0;
 
@@ -560,7 +560,9 @@ struct Solver {
     nblk = (int)std::max<int64_t>(1, std::min<int64_t>((most + 1023) / 1024, std::max(8, kDotBlocks / op->n_seg)));
     use_P = op->d_P != nullptr;
     small = KB == 1 && op->n_seg == 1 && n8 <= kSmallVector;
-    if (ws->n8 == n8 && ws->restart == restart && ws->nsys == nsys && ws->nblk == nblk) return SMH_OK;
+    cap = std::max(restart, ws->restart);
+    if (ws->n8 == n8 && ws->restart >= restart && ws->nsys == nsys && ws->nblk == nblk) return SMH_OK;
+    cap = restart;
     ws->release();
     const size_t n32 = KB == 1 ? (size_t)n : (size_t)op->n_part * op->b32_S * KB;
     const bool half = KB > 1 && smh::op_has_batch(op, SMH_FP16);
@@ -659,7 +661,7 @@ struct Solver {
   }
 
   void saxpy(int nv, const double2* c, double sgn, double2* w) {
-    hipLaunchKernelGGL(saxpy_kernel<KB>, dim3(blocks_for(n8)), dim3(256), 0, s, ws->V, n8, nv, c, restart + 1, sgn, w,
+    hipLaunchKernelGGL(saxpy_kernel<KB>, dim3(blocks_for(n8)), dim3(256), 0, s, ws->V, n8, nv, c, cap + 1, sgn, w,
                        n8, per_part, (const int*)op->d_seg_of);
   }
 
@@ -668,12 +670,12 @@ struct Solver {
   // a graph).
   int arnoldi_step(int k, int precision) {
     int rc;
-    const int ldh = restart + 1;
+    const int ldh = cap + 1;
     const double2* vk = ws->V + (size_t)k * n8;
     if ((rc = master(vk, ws->w, precision, use_P))) return rc;
     if (small) {
       hipLaunchKernelGGL(arnoldi_small_kernel, dim3(1), dim3(kSmallThreads), 0, s, k, ws->V, (const double2*)ws->w,
-                         (int)n8, ws->atol, restart, ws->live, ws->H, ws->cs, ws->sn, ws->g, ws->kr, ws->nlive,
+                         (int)n8, ws->atol, cap, ws->live, ws->H, ws->cs, ws->sn, ws->g, ws->kr, ws->nlive,
                          ws->h_live);
       SMH_HIP(ctx, hipGetLastError());
       return SMH_OK;
@@ -684,7 +686,7 @@ struct Solver {
     saxpy(k + 1, ws->h2, -1.0, ws->w);
     if ((rc = dots(ws->w, 1, ws->w, ws->hn, 1))) return rc;
     hipLaunchKernelGGL(givens_kernel, dim3(blocks_for(nsys, 64)), dim3(64), 0, s, k, ws->h1, ws->h2, ldh, ws->hn,
-                       ws->atol, nsys, restart, ws->live, ws->H, ws->cs, ws->sn, ws->g, ws->kr, ws->scale, ws->nlive);
+                       ws->atol, nsys, cap, ws->live, ws->H, ws->cs, ws->sn, ws->g, ws->kr, ws->scale, ws->nlive);
     hipLaunchKernelGGL(sscale_kernel<KB>, dim3(blocks_for(n8)), dim3(256), 0, s, ws->w, ws->scale,
                        ws->V + (size_t)(k + 1) * n8, n8, per_part, (const int*)op->d_seg_of,
                        (const int*)(ws->nlive + k), ws->h_live);
@@ -766,7 +768,6 @@ struct Solver {
   int gmres(double2* x, const double2* b, const double* atol, const int* active, int maxiter, int precision,
             double* res_out, int& steps, bool x_zero, bool trust_estimate) {
     int rc;
-    const int R = restart;
     SMH_HIP(ctx, hipMemcpyAsync(ws->atol, atol, nsys * sizeof(double), hipMemcpyHostToDevice, s));
     SMH_HIP(ctx, hipMemcpyAsync(ws->active, active, nsys * sizeof(int), hipMemcpyHostToDevice, s));
     steps = 0;
@@ -778,17 +779,17 @@ struct Solver {
         hipLaunchKernelGGL(sub_kernel, dim3(blocks_for(n8)), dim3(256), 0, s, b, ws->w, ws->w, n8);
       }
       if ((rc = dots(ws->w, 1, ws->w, ws->hn, 1))) return rc;
-      hipLaunchKernelGGL(zero_int_kernel, dim3(1), dim3(256), 0, s, ws->nlive, R + 1);
+      hipLaunchKernelGGL(zero_int_kernel, dim3(1), dim3(256), 0, s, ws->nlive, cap + 1);
       hipLaunchKernelGGL(cycle_init_kernel, dim3(blocks_for(nsys, 64)), dim3(64), 0, s, ws->hn, ws->atol, ws->active,
-                         nsys, R, ws->g, ws->live, ws->scale, ws->res, ws->kr, ws->nlive);
+                         nsys, cap, ws->g, ws->live, ws->scale, ws->res, ws->kr, ws->nlive);
       // V_0 (zero for systems that do not run) and the live count
       hipLaunchKernelGGL(sscale_kernel<KB>, dim3(blocks_for(n8)), dim3(256), 0, s, ws->w, ws->scale, ws->V, n8,
-                         per_part, (const int*)op->d_seg_of, (const int*)(ws->nlive + R), ws->h_live);
+                         per_part, (const int*)op->d_seg_of, (const int*)(ws->nlive + cap), ws->h_live);
       SMH_HIP(ctx, hipGetLastError());
       if ((rc = residuals(res_out))) return rc;
       if (ws->h_live[0] == 0 || steps >= maxiter) return SMH_OK;
       int k = 0;
-      for (; k < R && steps < maxiter; ++k, ++steps) {
+      for (; k < restart && steps < maxiter; ++k, ++steps) {
         if ((rc = run_step(k, precision))) return rc;
         ++iters;
         SMH_HIP(ctx, hipStreamSynchronize(s));
@@ -799,8 +800,8 @@ struct Solver {
         }
       }
       // y = R^-1 g per system, then x += V y (or x += P V y) for all at once
-      hipLaunchKernelGGL(backsub_kernel, dim3(blocks_for(nsys, 64)), dim3(64), 0, s, nsys, R, ws->H, ws->g, ws->kr,
-                         ws->yv, R + 1, ws->res);
+      hipLaunchKernelGGL(backsub_kernel, dim3(blocks_for(nsys, 64)), dim3(64), 0, s, nsys, cap, ws->H, ws->g, ws->kr,
+                         ws->yv, cap + 1, ws->res);
       if (k > 0) {
         if (use_P) {
           hipLaunchKernelGGL(zero2_kernel, dim3(1024), dim3(256), 0, s, ws->tmp, n8);

@@ -7,6 +7,7 @@ operators by several threads on the context's one stream, while graphs are
 captured. The residual is taken
 with the plain numpy operator of the partial-sum tests; an FP64 solve to tol
 leaves tol plus the FP64 operators' own difference (1e-13)."""
+import ctypes
 import threading
 
 import numpy as np
@@ -46,6 +47,35 @@ def test_single_solves_meet_the_tolerance(gpu, n, restart):
             first = x if first is None else first
             assert np.linalg.norm(x - first) <= 1e-8 * np.linalg.norm(first)
         op.matvec(b, 'single')
+
+
+def test_shorter_restarts_keep_the_workspace(gpu):
+    """Restart lengths in turn, eager, captured and replayed: the arrays of the longest serve the shorter ones, so
+    no device memory is given back (5000 unknowns: 10 MB of basis at 120, 0.6 MB at 6)."""
+    from smuthi_amd.linear_system import CouplingMatrixRadialLookupCUDA
+    hip = ctypes.CDLL('libamdhip64.so')
+
+    def free_memory():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+    n = 834
+    xy, rho, table = _system(n, n)
+    op = CouplingMatrixRadialLookupCUDA.from_table(table, rho, [Sphere([a, b, 200.0], 1.5, 50.0, 1, 1)
+                                                                for a, b in xy], H, 'linear')
+    rng = np.random.default_rng(3)
+    d = np.hypot(xy[:, None, 0] - xy[None, :, 0], xy[:, None, 1] - xy[None, :, 1])
+    t = (0.25 / (6 * (1 / (1 + d / 500)).sum(1).max()) * np.exp(2j * np.pi * rng.uniform(size=(n, 6)))).ravel()
+    b = rng.standard_normal((3, n * 6)) + 1j * rng.standard_normal((3, n * 6))
+    for rhs in (b[0], b):
+        op.solve_master(t, rhs, 1e-9, precision='double', restart=120)
+        free = free_memory()
+        for restart in (6, 120, 2, 6, 120, 6):
+            x = op.solve_master(t, rhs, 1e-9, precision='double', restart=restart)
+            for v, r in zip(x.reshape(-1, n * 6), rhs.reshape(-1, n * 6)):
+                res = r - v + t * _reference(xy, rho, table, v.reshape(1, n, 6)).ravel()
+                assert np.linalg.norm(res) <= (1e-9 + 1e-12) * np.linalg.norm(r), restart
+            assert free_memory() - free < 2 ** 22, restart  # (captured graphs may take some)
 
 
 def test_threads_solve_while_others_capture(gpu):
