@@ -225,16 +225,16 @@ __device__ inline double2 cdiv2(double2 a, double2 b) {
 }
 
 // Start of a restart cycle (one thread per system): beta = ||r|| from the norm
-// dot, the system runs this cycle if active and beta > atol; nlive[restart]
-// counts the systems that run.
+// dot, the system runs this cycle if active, beta > atol and it has steps left;
+// nlive[restart] counts the systems that run.
 __global__ void cycle_init_kernel(const double2* __restrict__ nrm, const double* __restrict__ atol,
-                                  const int* __restrict__ active, int nsys, int restart, double2* g, int* live,
+                                  const int* __restrict__ active, const int* __restrict__ left, int nsys, int restart, double2* g, int* live,
                                   double* scale, double* res, int* kr, int* nlive) {
   const int sys = blockIdx.x * blockDim.x + threadIdx.x;
   if (sys >= nsys) return;
   const double beta = sqrt(fmax(0.0, nrm[sys].x));
   res[sys] = beta;
-  const bool c = active[sys] && beta > atol[sys] && beta > 0.0;
+  const bool c = active[sys] && beta > atol[sys] && beta > 0.0 && left[sys] > 0;
   live[sys] = c ? 1 : 0;
   kr[sys] = 0;
   scale[sys] = c ? 1.0 / beta : 0.0;
@@ -276,9 +276,11 @@ __device__ inline bool givens_step(int k, double2* col, double hn, double atol, 
 }
 
 // The step's rotations (one thread per system) and the normalisation of w;
-// nlive[k] counts the systems still running after this step.
+// nlive[k] counts the systems still running after this step (no more than left
+// steps of the cycle).
 __global__ void givens_kernel(int k, double2* h1, const double2* __restrict__ h2, int ldh,
-                              const double2* __restrict__ hn2, const double* __restrict__ atol, int nsys, int restart,
+                              const double2* __restrict__ hn2, const double* __restrict__ atol,
+                              const int* __restrict__ left, int nsys, int restart,
                               int* live, double2* H, double2* cs, double2* sn, double2* g, int* kr, double* scale,
                               int* nlive) {
   const int sys = blockIdx.x * blockDim.x + threadIdx.x;
@@ -294,7 +296,8 @@ __global__ void givens_kernel(int k, double2* h1, const double2* __restrict__ h2
     col[j] = make_double2(a.x + b.x, a.y + b.y);
   }
   const bool on = givens_step(k, col, hn, atol[sys], restart, H + (size_t)sys * (restart + 1) * restart,
-                              cs + (size_t)sys * restart, sn + (size_t)sys * restart, g + (size_t)sys * (restart + 1));
+                              cs + (size_t)sys * restart, sn + (size_t)sys * restart, g + (size_t)sys * (restart + 1)) &&
+                  k + 1 < left[sys];
   kr[sys] = k + 1;
   scale[sys] = hn > 0 ? 1.0 / hn : 0.0;
   if (!on)
@@ -313,7 +316,7 @@ __global__ void givens_kernel(int k, double2* h1, const double2* __restrict__ h2
 constexpr int kSmallThreads = 1024, kSmallPer = 4, kSmallVector = kSmallThreads * kSmallPer;
 __global__ void __launch_bounds__(kSmallThreads)
     arnoldi_small_kernel(int k, double2* V, const double2* __restrict__ wv, int n, const double* __restrict__ atol,
-                         int restart, int* live, double2* H, double2* cs, double2* sn, double2* g, int* kr,
+                         const int* __restrict__ left, int restart, int* live, double2* H, double2* cs, double2* sn, double2* g, int* kr,
                          int* nlive, int* host_live) {
   __shared__ double2 red[kSmallThreads / 64][kMaxBasis + 1];
   __shared__ double2 h[kMaxBasis + 1], col[kMaxBasis + 1], css[kMaxBasis], sns[kMaxBasis];
@@ -396,7 +399,7 @@ __global__ void __launch_bounds__(kSmallThreads)
     double f = 0.0;
     if (live[0]) {
       const double hn = sqrt(fmax(0.0, h[0].x));
-      const bool on = givens_step(k, col, hn, atol[0], restart, H, css, sns, g);
+      const bool on = givens_step(k, col, hn, atol[0], restart, H, css, sns, g) && k + 1 < left[0];
       cs[k] = css[k];
       sn[k] = sns[k];
       kr[0] = k + 1;
@@ -419,12 +422,15 @@ __global__ void __launch_bounds__(kSmallThreads)
 }
 
 // End of a cycle (one thread per system): y = R^{-1} g over the system's
-// kr steps (zero beyond), and its least-squares residual estimate |g_kr|.
+// kr steps (zero beyond), and its least-squares residual estimate |g_kr|. The
+// cycle's steps come off the system's steps left: `used` of them, or (used < 0)
+// its own.
 __global__ void backsub_kernel(int nsys, int restart, const double2* __restrict__ H, const double2* __restrict__ g,
-                               const int* __restrict__ kr, double2* yv, int ldy, double* res) {
+                               const int* __restrict__ kr, double2* yv, int ldy, double* res, int used, int* left) {
   const int sys = blockIdx.x * blockDim.x + threadIdx.x;
   if (sys >= nsys) return;
   const int m = kr[sys];
+  left[sys] -= used >= 0 ? used : m;
   const double2* Hs = H + (size_t)sys * (restart + 1) * restart;
   const double2* gs = g + (size_t)sys * (restart + 1);
   double2* y = yv + (size_t)sys * ldy;
@@ -492,8 +498,9 @@ struct SolveWs {
   double2 *V = nullptr, *w = nullptr, *t = nullptr, *partial = nullptr, *h1 = nullptr, *h2 = nullptr,
           *hn = nullptr, *H = nullptr, *cs = nullptr, *sn = nullptr, *g = nullptr, *yv = nullptr, *y64 = nullptr,
           *b = nullptr, *x = nullptr, *d = nullptr, *r = nullptr, *pv = nullptr, *tmp = nullptr;
+  // atol, res, left and active are one block: uploaded, and the middle two read back, in one copy
   double *atol = nullptr, *scale = nullptr, *res = nullptr;
-  int *live = nullptr, *kr = nullptr, *nlive = nullptr, *active = nullptr;
+  int *live = nullptr, *kr = nullptr, *nlive = nullptr, *active = nullptr, *left = nullptr;
   float2 *x32 = nullptr, *y32 = nullptr;
   void* x16 = nullptr;
   // pinned host memory: the live-system count of the last step, and the
@@ -512,7 +519,7 @@ struct SolveWs {
   void release() {
     drop_graphs();
     void* p[] = {V, w, t, partial, h1, h2, hn, H, cs, sn, g, yv, y64, b, x, d, r, pv, tmp,
-                 atol, scale, res, live, kr, nlive, active, x32, y32, x16};
+                 atol, scale, live, kr, nlive, x32, y32, x16};
     for (void* q : p)
       if (q) (void)hipFree(q);
     if (capture) (void)hipStreamDestroy(capture);
@@ -584,10 +591,9 @@ struct Solver {
         alloc((void**)&ws->x, n8 * sizeof(double2)) && alloc((void**)&ws->d, n8 * sizeof(double2)) &&
         alloc((void**)&ws->r, n8 * sizeof(double2)) &&
         (KB == 1 || (alloc((void**)&ws->pv, n8 * sizeof(double2)) && alloc((void**)&ws->tmp, n8 * sizeof(double2)))) &&
-        alloc((void**)&ws->atol, nsys * sizeof(double)) &&
-        alloc((void**)&ws->scale, nsys * sizeof(double)) && alloc((void**)&ws->res, nsys * sizeof(double)) &&
+        alloc((void**)&ws->atol, 3 * nsys * sizeof(double)) && alloc((void**)&ws->scale, nsys * sizeof(double)) &&
         alloc((void**)&ws->live, nsys * sizeof(int)) && alloc((void**)&ws->kr, nsys * sizeof(int)) &&
-        alloc((void**)&ws->nlive, (restart + 1) * sizeof(int)) && alloc((void**)&ws->active, nsys * sizeof(int)) &&
+        alloc((void**)&ws->nlive, (restart + 1) * sizeof(int)) &&
         alloc((void**)&ws->x32, n32 * sizeof(float2)) && alloc((void**)&ws->y32, n8 * sizeof(float2)) &&
         (!half || alloc(&ws->x16, n32 * 2 * sizeof(_Float16))) &&
         hipHostMalloc((void**)&ws->h_live, 4 * sizeof(int), hipHostMallocDefault) == hipSuccess &&
@@ -596,6 +602,9 @@ struct Solver {
       ws->release();
       return smh_fail(ctx, SMH_ERR_HIP, "solver allocation failed (%lld entries, restart %d)", (long long)n8, restart);
     }
+    ws->res = ws->atol + nsys;
+    ws->left = (int*)(ws->res + nsys);
+    ws->active = ws->left + nsys;
     // the FP32 input's padding slots stay zero
     hipLaunchKernelGGL(zero_f2_kernel, dim3(1024), dim3(256), 0, s, ws->x32, (int64_t)n32);
     SMH_HIP(ctx, hipGetLastError());
@@ -675,7 +684,7 @@ struct Solver {
     if ((rc = master(vk, ws->w, precision, use_P))) return rc;
     if (small) {
       hipLaunchKernelGGL(arnoldi_small_kernel, dim3(1), dim3(kSmallThreads), 0, s, k, ws->V, (const double2*)ws->w,
-                         (int)n8, ws->atol, cap, ws->live, ws->H, ws->cs, ws->sn, ws->g, ws->kr, ws->nlive,
+                         (int)n8, ws->atol, ws->left, cap, ws->live, ws->H, ws->cs, ws->sn, ws->g, ws->kr, ws->nlive,
                          ws->h_live);
       SMH_HIP(ctx, hipGetLastError());
       return SMH_OK;
@@ -686,7 +695,7 @@ struct Solver {
     saxpy(k + 1, ws->h2, -1.0, ws->w);
     if ((rc = dots(ws->w, 1, ws->w, ws->hn, 1))) return rc;
     hipLaunchKernelGGL(givens_kernel, dim3(blocks_for(nsys, 64)), dim3(64), 0, s, k, ws->h1, ws->h2, ldh, ws->hn,
-                       ws->atol, nsys, cap, ws->live, ws->H, ws->cs, ws->sn, ws->g, ws->kr, ws->scale, ws->nlive);
+                       ws->atol, ws->left, nsys, cap, ws->live, ws->H, ws->cs, ws->sn, ws->g, ws->kr, ws->scale, ws->nlive);
     hipLaunchKernelGGL(sscale_kernel<KB>, dim3(blocks_for(n8)), dim3(256), 0, s, ws->w, ws->scale,
                        ws->V + (size_t)(k + 1) * n8, n8, per_part, (const int*)op->d_seg_of,
                        (const int*)(ws->nlive + k), ws->h_live);
@@ -747,12 +756,13 @@ struct Solver {
     return SMH_OK;
   }
 
-  // the systems' residuals (or estimates) to the host
-  int residuals(double* res_out) {
-    SMH_HIP(ctx, hipMemcpyAsync(ws->h_val, ws->res, nsys * sizeof(double), hipMemcpyDeviceToHost, s));
+  // the systems' residuals (or estimates) and steps left to the host
+  int residuals(double* res_out, int* left) {
+    SMH_HIP(ctx, hipMemcpyAsync(ws->h_val, ws->res, nsys * (sizeof(double) + sizeof(int)), hipMemcpyDeviceToHost, s));
     SMH_HIP(ctx, hipStreamSynchronize(s));
     const double* v = reinterpret_cast<const double*>(ws->h_val);
     std::copy(v, v + nsys, res_out);
+    std::copy((const int*)(v + nsys), (const int*)(v + nsys) + nsys, left);
     return SMH_OK;
   }
 
@@ -763,13 +773,20 @@ struct Solver {
   // Arnoldi residual estimates reach atol or the cycle ends, without
   // recomputing the true residual (the caller takes it in FP64 and starts the
   // next sweep: a reduced-precision operator whose error sits above atol would
-  // otherwise stall the restarts). res_out[sys]: residual of x (or the
-  // estimate); steps: Arnoldi steps taken.
-  int gmres(double2* x, const double2* b, const double* atol, const int* active, int maxiter, int precision,
+  // otherwise stall the restarts). left[sys]: steps the system may take, and
+  // may still take afterwards: on lookup operators the systems share the count
+  // of the steps taken together, on the explicit matrix each counts its own
+  // (there right-hand sides solved one after the other had maxiter each, and
+  // one that ends a sweep early must not pay for the others' steps).
+  // res_out[sys]: residual of x (or the estimate); steps: Arnoldi steps taken.
+  int gmres(double2* x, const double2* b, const double* atol, const int* active, int* left, int precision,
             double* res_out, int& steps, bool x_zero, bool trust_estimate) {
     int rc;
-    SMH_HIP(ctx, hipMemcpyAsync(ws->atol, atol, nsys * sizeof(double), hipMemcpyHostToDevice, s));
-    SMH_HIP(ctx, hipMemcpyAsync(ws->active, active, nsys * sizeof(int), hipMemcpyHostToDevice, s));
+    std::vector<double> systems(3 * (size_t)nsys, 0.0);
+    std::copy(atol, atol + nsys, systems.data());
+    std::copy(left, left + nsys, (int*)(systems.data() + 2 * nsys));
+    std::copy(active, active + nsys, (int*)(systems.data() + 2 * nsys) + nsys);
+    SMH_HIP(ctx, hipMemcpyAsync(ws->atol, systems.data(), systems.size() * sizeof(double), hipMemcpyHostToDevice, s));
     steps = 0;
     for (int outer = 0;; ++outer) {
       if (outer == 0 && x_zero) {
@@ -781,15 +798,15 @@ struct Solver {
       if ((rc = dots(ws->w, 1, ws->w, ws->hn, 1))) return rc;
       hipLaunchKernelGGL(zero_int_kernel, dim3(1), dim3(256), 0, s, ws->nlive, cap + 1);
       hipLaunchKernelGGL(cycle_init_kernel, dim3(blocks_for(nsys, 64)), dim3(64), 0, s, ws->hn, ws->atol, ws->active,
-                         nsys, cap, ws->g, ws->live, ws->scale, ws->res, ws->kr, ws->nlive);
+                         ws->left, nsys, cap, ws->g, ws->live, ws->scale, ws->res, ws->kr, ws->nlive);
       // V_0 (zero for systems that do not run) and the live count
       hipLaunchKernelGGL(sscale_kernel<KB>, dim3(blocks_for(n8)), dim3(256), 0, s, ws->w, ws->scale, ws->V, n8,
                          per_part, (const int*)op->d_seg_of, (const int*)(ws->nlive + cap), ws->h_live);
       SMH_HIP(ctx, hipGetLastError());
-      if ((rc = residuals(res_out))) return rc;
-      if (ws->h_live[0] == 0 || steps >= maxiter) return SMH_OK;
+      if ((rc = residuals(res_out, left))) return rc;
+      if (ws->h_live[0] == 0) return SMH_OK;
       int k = 0;
-      for (; k < restart && steps < maxiter; ++k, ++steps) {
+      for (; k < restart; ++k, ++steps) {
         if ((rc = run_step(k, precision))) return rc;
         ++iters;
         SMH_HIP(ctx, hipStreamSynchronize(s));
@@ -801,7 +818,7 @@ struct Solver {
       }
       // y = R^-1 g per system, then x += V y (or x += P V y) for all at once
       hipLaunchKernelGGL(backsub_kernel, dim3(blocks_for(nsys, 64)), dim3(64), 0, s, nsys, cap, ws->H, ws->g, ws->kr,
-                         ws->yv, cap + 1, ws->res);
+                         ws->yv, cap + 1, ws->res, op->kind == 2 ? -1 : k, ws->left);
       if (k > 0) {
         if (use_P) {
           hipLaunchKernelGGL(zero2_kernel, dim3(1024), dim3(256), 0, s, ws->tmp, n8);
@@ -812,7 +829,7 @@ struct Solver {
         }
       }
       SMH_HIP(ctx, hipGetLastError());
-      if (trust_estimate) return residuals(res_out);
+      if (trust_estimate) return residuals(res_out, left);
     }
   }
 };
@@ -891,7 +908,7 @@ static int solve_blocks(smh_op* op, const double* t_diag, const double* rhs, dou
   int64_t steps_total = 0;
   bool converged_all = true;
   std::vector<double> bnorm(nsys), atol(nsys), res(nsys), prev_res(nsys), inner_atol(nsys), inner_res(nsys);
-  std::vector<int> active(nsys), act(nsys);
+  std::vector<int> active(nsys), act(nsys), left(nsys);
   for (int64_t r0 = 0; r0 < nrhs; r0 += KB) {
     const int nb = (int)std::min<int64_t>(KB, nrhs - r0);
     SMH_HIP(ctx, hipMemcpyAsync(op->d_pk_in, rhs + 2 * r0 * op->n_unk, (size_t)nb * op->n_unk * sizeof(double2),
@@ -904,11 +921,12 @@ static int solve_blocks(smh_op* op, const double* t_diag, const double* rhs, dou
       atol[q] = tol * bnorm[q];
       active[q] = (q % KB) < nb && bnorm[q] > 0.0;
     }
+    std::fill(left.begin(), left.end(), maxiter);
     int steps = 0;
     if (mode == SMH_SOLVE_FP64) {
       // x0 = rhs, as smuthi passes rhs as initial guess
       SMH_HIP(ctx, hipMemcpyAsync(ws->x, ws->b, S.n8 * sizeof(double2), hipMemcpyDeviceToDevice, s));
-      if ((rc = S.gmres(ws->x, ws->b, atol.data(), active.data(), maxiter, SMH_FP64, res.data(), steps, false, false)))
+      if ((rc = S.gmres(ws->x, ws->b, atol.data(), active.data(), left.data(), SMH_FP64, res.data(), steps, false, false)))
         return rc;
       steps_total += steps;
       sweeps_total += 1;
@@ -919,7 +937,6 @@ static int solve_blocks(smh_op* op, const double* t_diag, const double* rhs, dou
       bool fresh = true;
       bool fp64_residuals = mode != SMH_SOLVE_MIXED16;
       const int inner_prec = mode == SMH_SOLVE_MIXED16 ? SMH_FP16 : SMH_FP32;
-      int budget = maxiter;
       for (int sweep = 0; sweep < 50; ++sweep) {
         if (sweep > 0) {
           // FP16 inner solves: the residual that drives the next sweep comes
@@ -955,17 +972,16 @@ static int solve_blocks(smh_op* op, const double* t_diag, const double* rhs, dou
         bool any = false;
         for (int q = 0; q < nsys; ++q) {
           prev_res[q] = res[q];
-          act[q] = active[q] && res[q] > atol[q];
+          act[q] = active[q] && res[q] > atol[q] && left[q] > 0;
           inner_atol[q] = std::max(atol[q] * 0.5, (mode == SMH_SOLVE_MIXED16 ? kInnerRel16 : kInnerRel) * res[q]);
           any = any || act[q];
         }
-        if (!any || budget <= 0) break;
+        if (!any) break;
         hipLaunchKernelGGL(zero2_kernel, dim3(1024), dim3(256), 0, s, ws->d, S.n8);
         int inner_steps = 0;
-        if ((rc = S.gmres(ws->d, ws->r, inner_atol.data(), act.data(), budget, inner_prec, inner_res.data(),
+        if ((rc = S.gmres(ws->d, ws->r, inner_atol.data(), act.data(), left.data(), inner_prec, inner_res.data(),
                           inner_steps, true, true)))
           return rc;
-        budget -= inner_steps;
         steps_total += inner_steps;
         hipLaunchKernelGGL(add_kernel, dim3(blocks_for(S.n8)), dim3(256), 0, s, ws->x, ws->d, S.n8);
         sweeps_total += 1;

@@ -69,3 +69,33 @@ def test_explicit_operator_refuses_what_it_did(gpu):
         set_preconditioner(op, np.zeros((3, 6, 6), complex))
     with pytest.raises(SmhError):
         op.solve_master(np.full(op.shape[0], 0.1), x, 1e-6, precision='mixed16')
+
+
+def test_each_right_hand_side_of_a_block_has_its_own_steps(gpu):
+    """maxiter counts the steps of each right-hand side, as if it were solved alone. Noise takes most steps, in one
+    sweep of the refinement; an eigenvector with 1e-6 of noise few, in two. Together the second sweeps follow the
+    longest first one, and the block still passes with the steps that its longest member takes alone."""
+    op = _operator(24, 2)
+    W = op.coupling_matrix
+    n, tol = len(W), 1.5e-7
+    rng = np.random.default_rng(5)
+    t = 0.8 / np.abs(np.linalg.eigvals(W)).max() * np.exp(2j * np.pi * rng.uniform(size=n))
+    _, vec = np.linalg.eig(np.eye(n) - t[:, None] * W)
+
+    def noise():
+        v = rng.standard_normal(n) + 1j * rng.standard_normal(n)
+        return v / np.linalg.norm(v)
+
+    def alone(x):
+        return [op.solve_master(t, v, tol, precision='mixed', restart=100, with_stats=True)[1] for v in x]
+    hard, easy = [noise() for _ in range(24)], [vec[:, 3 * j] + 1e-6 * noise() for j in range(24)]
+    sh, se = alone(hard), alone(easy)
+    one = [(s['iterations'], j) for j, s in enumerate(sh) if s['sweeps'] == 1 and s['relative_residual'] < 0.85 * tol]
+    steps, j = max(one)
+    two = [k for k, s in enumerate(se) if s['sweeps'] == 2 and s['iterations'] < steps][:7]
+    print('steps alone %d, %s' % (steps, [se[k]['iterations'] for k in two]), flush=True)
+    assert len(two) == 7
+    x = np.stack([hard[j]] + [easy[k] for k in two])
+    got, stats, ok = op.solve_master(t, x, tol, precision='mixed', restart=100, maxiter=steps, with_stats=True)
+    assert ok and stats['relative_residual'] <= tol and stats['iterations'] > steps, stats
+    assert not op.solve_master(t, x, tol, precision='mixed', restart=100, maxiter=steps // 2, with_stats=True)[2]
