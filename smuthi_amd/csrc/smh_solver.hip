@@ -308,12 +308,16 @@ __global__ void givens_kernel(int k, double2* h1, const double2* __restrict__ h2
 
 // Everything of an Arnoldi step that follows the matvec, for one system whose
 // vector fits a workgroup's registers (kSmallVector entries): CGS2 against
-// V_0..V_k, the norm, the rotations and V_{k+1}. Bound by the latency of its
-// dependent passes over V from L2 (1500 unknowns, k = 8: about 10 us); the
-// launches it replaces (two dots, two reductions, two updates, norm, rotation,
-// scaling) took 35 us of a step at that size, and spread over more workgroups
-// they are the faster ones above it.
+// V_0..V_k, the norm, the rotations and V_{k+1}. Bound by its dependent passes
+// over V, which one CU reads from its XCD's L2 (4 MB): beyond kSmallBasis
+// entries of basis the launches it replaces (two dots, two reductions, two
+// updates, norm, rotation, scaling), which spread them over the chip, are the
+// faster ones. A whole step of 4092 unknowns: 81 us against 100 below k = 4, 237
+// against 265 below k = 48, 300 against 333 below 64, but 536 against 437 from k
+// = 64 to 96; of 2100 unknowns 61 against 71 below k = 4, 429 against 450 below
+// k = 126; of 600 unknowns 45 against 60 and 336 against 406.
 constexpr int kSmallThreads = 1024, kSmallPer = 4, kSmallVector = kSmallThreads * kSmallPer;
+constexpr int64_t kSmallBasis = (int64_t)1 << 18;
 __global__ void __launch_bounds__(kSmallThreads)
     arnoldi_small_kernel(int k, double2* V, const double2* __restrict__ wv, int n, const double* __restrict__ atol,
                          const int* __restrict__ left, int restart, int* live, double2* H, double2* cs, double2* sn, double2* g, int* kr,
@@ -682,7 +686,7 @@ struct Solver {
     const int ldh = cap + 1;
     const double2* vk = ws->V + (size_t)k * n8;
     if ((rc = master(vk, ws->w, precision, use_P))) return rc;
-    if (small) {
+    if (small && (k + 1) * n8 <= kSmallBasis) {
       hipLaunchKernelGGL(arnoldi_small_kernel, dim3(1), dim3(kSmallThreads), 0, s, k, ws->V, (const double2*)ws->w,
                          (int)n8, ws->atol, ws->left, cap, ws->live, ws->H, ws->cs, ws->sn, ws->g, ws->kr, ws->nlive,
                          ws->h_live);

@@ -1,6 +1,6 @@
 """Solves of one right-hand side on the device: systems whose Arnoldi step runs
-in one workgroup (up to 4096 unknowns, edge at 682 / 683 particles of 6), the
-several-launch step above, restart lengths from one step to the largest basis,
+in one workgroup (up to 4096 unknowns, edge at 682 / 683 particles of 6, and up
+to 64 steps of 4092), the several-launch step above, restart lengths from one step to the largest basis,
 and repeated solves (the first runs eagerly, the second captures its graphs,
 the third replays them, with eager matvecs between), and solves of different
 operators by several threads on the context's one stream, while graphs are
@@ -47,6 +47,33 @@ def test_single_solves_meet_the_tolerance(gpu, n, restart):
             first = x if first is None else first
             assert np.linalg.norm(x - first) <= 1e-8 * np.linalg.norm(first)
         op.matvec(b, 'single')
+
+
+def test_steps_on_both_sides_of_the_basis_limit(gpu):
+    """A cycle of 100 steps that does not converge: the first 64 run in one workgroup, the others in several
+    launches. Its residual is the true one of its solution, and the smallest over the same Krylov space that a block
+    solve (several launches throughout) finds, up to the FP64 roundings of 100 steps on a basis orthogonalised twice
+    (100 x 1e-16 x the growth of |x| over |b|, below 1e-9)."""
+    from smuthi_amd.linear_system import CouplingMatrixRadialLookupCUDA
+    n = 682
+    xy, rho, table = _system(n, n)
+    op = CouplingMatrixRadialLookupCUDA.from_table(table, rho, [Sphere([a, b, 200.0], 1.5, 50.0, 1, 1)
+                                                                for a, b in xy], H, 'linear')
+    rng = np.random.default_rng(1)
+    d = np.hypot(xy[:, None, 0] - xy[None, :, 0], xy[:, None, 1] - xy[None, :, 1])
+    t = (4000 / (6 * (1 / (1 + d / 500)).sum(1).max()) * np.exp(2j * np.pi * rng.uniform(size=(n, 6)))).ravel()
+    b = rng.standard_normal((2, n * 6)) + 1j * rng.standard_normal((2, n * 6))
+    kw = dict(precision='double', restart=100, maxiter=100, with_stats=True)
+    worst = []
+    for repeat in range(3):
+        alone = [op.solve_master(t, v, 1e-12, **kw) for v in b]
+        for (x, stats, ok), v in zip(alone, b):
+            res = np.linalg.norm(v - x + t * _reference(xy, rho, table, x.reshape(1, n, 6)).ravel())
+            assert not ok and stats['iterations'] == 100
+            assert abs(res / np.linalg.norm(v) - stats['relative_residual']) <= 1e-9
+        worst.append(max(s['relative_residual'] for _, s, _ in alone))
+    block = op.solve_master(t, b, 1e-12, **kw)[1]['relative_residual']
+    assert np.abs(np.array(worst) / block - 1).max() <= 1e-6, (worst, block)
 
 
 def test_shorter_restarts_keep_the_workspace(gpu):
