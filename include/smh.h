@@ -281,7 +281,10 @@ int smh_op_bench_matvec_batch(smh_op *op, int precision, int iters, double *kern
  * matvec), and keeps the fastest grouping (*best = its index). The FP16
  * and FP32 8-RHS kernels share one grouping. Results stay within each
  * kernel's accuracy (the grouping changes summation order and fixed-point
- * scales only). Drops the solver's captured graphs. No counterpart in
+ * scales only). Drops the solver's captured graphs. The 8-RHS kernels of
+ * cubic volume lookups have no work items: their one launch is timed once,
+ * matvec_ms holds that time for every candidate, *best is 0 and the graphs
+ * stay. No counterpart in
  * smuthi, whose CUDA kernels launch one thread per matrix row
  * (linear_system_cuda.py:26-405, cuda_blocksize). */
 int smh_op_autotune(smh_op *op, int batch, int precision, int iters, int n_cand, const int *items_per_cu,

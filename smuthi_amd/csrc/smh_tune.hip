@@ -45,7 +45,6 @@ int regroup(smh_op* op, const std::vector<smh_op::Binning*>& bins, int per_cu, i
   smh_ctx* ctx = op->ctx;
   size_t need = 0;
   for (smh_op::Binning* bn : bins) {
-    if (!bn->slab_pair.empty()) continue;  // (volume, batched: entries are taken from queues, not grouped)
     if (int rc = group_work_items(op, *bn, per_cu, order_mode)) return rc;
     need = std::max(need, (size_t)bn->n_items * bn->part_bytes);
   }
@@ -86,17 +85,26 @@ extern "C" int smh_op_autotune(smh_op* op, int batch, int precision, int iters, 
     SMH_CHECK(ctx, bn->Rc > 0 && bn->n_entries > 0, SMH_ERR_UNSUPPORTED, "no %s kernel for this operator",
               pi ? "FP64" : "FP32");
   SMH_HIP(ctx, hipSetDevice(ctx->device));
+  auto time = [&](double* ms) {
+    double kms = 0;
+    return batch ? smh_op_bench_matvec_batch(op, precision, iters, &kms, ms)
+                 : smh_op_bench_matvec(op, precision, iters, &kms, ms);
+  };
+  if (!bins[0]->slab_pair.empty()) {
+    // the slab kernels (cubic volume lookups, batched) deal their units out by a fixed stride: every candidate is
+    // the same launch, timed once, and the solver's graphs stay
+    if (int rc = time(matvec_ms)) return rc;
+    std::fill(matvec_ms + 1, matvec_ms + n_cand, matvec_ms[0]);
+    if (best) *best = 0;
+    return SMH_OK;
+  }
   // captured solver graphs hold the item arrays' addresses and grid sizes
   smh::solver_drop_graphs(op);
   int pick = -1;
   for (int c = 0; c < n_cand; ++c) {
     if (int rc = regroup(op, bins, items_per_cu[c], launch_order[c])) return rc;
-    double kms = 0, tms = 0;
-    const int rc = batch ? smh_op_bench_matvec_batch(op, precision, iters, &kms, &tms)
-                         : smh_op_bench_matvec(op, precision, iters, &kms, &tms);
-    if (rc) return rc;
-    matvec_ms[c] = tms;
-    if (pick < 0 || tms < matvec_ms[pick]) pick = c;
+    if (int rc = time(matvec_ms + c)) return rc;
+    if (pick < 0 || matvec_ms[c] < matvec_ms[pick]) pick = c;
   }
   if (int rc = regroup(op, bins, items_per_cu[pick], launch_order[pick])) return rc;
   if (best) *best = pick;

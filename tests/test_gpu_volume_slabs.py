@@ -86,3 +86,23 @@ def test_half_next_to_rows_of_zeros(gpu, kind, size):
     V = rng.standard_normal((8, op.shape[0])) + 1j * rng.standard_normal((8, op.shape[0]))
     want = op.matvec(V, 'double')
     assert np.linalg.norm(op.matvec(V, 'half') - want) < 1e-3 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize('kind,grouped', [('linear', True), ('spline', False), ('catmull-rom', False)])
+def test_autotune_times_one_launch_once(gpu, kind, grouped):
+    """The slab kernels have no launch shapes to choose from: every candidate has the one launch's time, and the
+    first is named. The single-vector and bilinear kernels are timed candidate by candidate."""
+    op, rng = _operator(60, 2, 2, kind, None, 5)
+    V = rng.standard_normal((8, op.shape[0])) + 1j * rng.standard_normal((8, op.shape[0]))
+    cand = [(4, 0), (16, 1), (8, 0), (32, 1), (16, 0)]
+    for precision in ('half', 'single', 'double'):
+        before = op.matvec(V, precision)
+        res = op.autotune(batch=True, precision=precision, iters=2, candidates=cand)
+        times = set(res['matvec_ms'].values())
+        assert min(times) > 0
+        if grouped:
+            assert len(times) > 1
+        else:
+            assert len(times) == 1 and res['best'] == cand[0]
+            assert np.array_equal(op.matvec(V, precision), before)
+    assert len(set(op.autotune(batch=False, precision='single', iters=2, candidates=cand)['matvec_ms'].values())) > 1
