@@ -81,8 +81,8 @@ __global__ void residual_parts_kernel(const double2* __restrict__ b, const doubl
 // Bound by the chain of pivots: a panel's rows stay in the registers of one
 // workgroup (two per thread), so that a pivot costs two barriers and no memory
 // access. 1800 unknowns (60 spheres, l_max 3): 13.2 ms in some 4000 launches of
-// rocSOLVER's getrf, 5.4 ms in 226 launches here, 28 us with two rows per thread
-// and 19 with one; errors against 64 bits as getrf's (80 to 2016 unknowns). With
+// rocSOLVER's getrf, 5.6 ms in 226 launches here, 29 us with two rows per thread
+// and 20 with one; errors against 64 bits as getrf's (80 to 2016 unknowns). With
 // more than 2048 rows the panel no longer fits the registers, and a pass over the matrix per eight columns no
 // longer the last-level cache: getrf.
 constexpr int kLuPanel = 8, kLuRows = 1024, kLuWaves = kLuRows / 64;
@@ -102,12 +102,15 @@ __device__ inline double2 cfma(double2 a, double2 l, double2 u) {  // a + l u
   return a;
 }
 
-// Largest key of the row of 16 lanes, in all of them
+// Largest value (of non-negative doubles, by their bits) and smallest index of the row of 16 lanes, in all of them
+template <int kCtrl>
+__device__ __forceinline__ unsigned dpp(unsigned v) {
+  return (unsigned)__builtin_amdgcn_mov_dpp((int)v, kCtrl, 0xF, 0xF, false);
+}
 template <int kCtrl>
 __device__ __forceinline__ unsigned long long max_dpp(unsigned long long k) {
-  const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(k & 0xffffffffu), kCtrl, 0xF, 0xF, false);
-  const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(k >> 32), kCtrl, 0xF, 0xF, false);
-  const unsigned long long o = ((unsigned long long)hi << 32) | lo;
+  const unsigned long long o =
+      ((unsigned long long)dpp<kCtrl>((unsigned)(k >> 32)) << 32) | dpp<kCtrl>((unsigned)(k & 0xffffffffu));
   return o > k ? o : k;
 }
 __device__ __forceinline__ unsigned long long max_row(unsigned long long k) {
@@ -115,6 +118,12 @@ __device__ __forceinline__ unsigned long long max_row(unsigned long long k) {
   k = max_dpp<0x124>(k);
   k = max_dpp<0x122>(k);
   return max_dpp<0x121>(k);
+}
+__device__ __forceinline__ unsigned min_row(unsigned i) {
+  i = min(i, dpp<0x128>(i));
+  i = min(i, dpp<0x124>(i));
+  i = min(i, dpp<0x122>(i));
+  return min(i, dpp<0x121>(i));
 }
 __device__ __forceinline__ unsigned long long max_xor(unsigned long long k, int d) {
   const unsigned long long o = __shfl_xor(k, d);
@@ -139,6 +148,7 @@ __global__ void __launch_bounds__(kLuRows) lu_step_kernel(double2* __restrict__ 
   __shared__ double2 sv[kLuPanel][2 * kLuPanel], us[kLuPanel][kLuPanel], l11[kLuPanel][kLuPanel];
   __shared__ double2 prow[kLuPanel], orow[kLuPanel];
   __shared__ unsigned long long redk[kLuWaves];
+  __shared__ unsigned redi[kLuWaves];
   __shared__ int pivots[kLuPanel];
   const int tid = threadIdx.x, N = (int)n, strips = (N + kLuPanel - 1) / kLuPanel;
   const int sk = k >= 0 ? k / kLuPanel : -1;  // strip of the factored panel
@@ -221,22 +231,37 @@ __global__ void __launch_bounds__(kLuRows) lu_step_kernel(double2* __restrict__ 
 #pragma unroll
   for (int j = 0; j < kLuPanel; ++j) {
     if (j >= w) break;
-    // pivot: the largest |re| + |im| of the rows from j on, by its upper 32 bits (a row within
-    // 1e-6 of the largest serves as well), the first of equals
-    unsigned long long key = 0xffffffffu - (unsigned)j;
+    // pivot: the largest |re| + |im| of the rows from j on, the first of equals (no row but NaN: j)
+    constexpr unsigned kNone = 0xffffffffu;
+    unsigned long long key = 0;
+    int best = -1;  // the lane's q
 #pragma unroll
     for (int q = 0; q < R; ++q) {
       const int i = tid + q * kLuRows;
       const double v = fabs(a[q][j].x) + fabs(a[q][j].y);
-      const unsigned long long kq =
-          ((unsigned long long)__double_as_longlong(v) & ~0xffffffffull) | (0xffffffffu - (unsigned)i);
-      if (i >= j && row0 + i < N && v >= 0.0 && kq > key) key = kq;
+      const unsigned long long kq = (unsigned long long)__double_as_longlong(v);
+      if (i >= j && row0 + i < N && v >= 0.0 && (best < 0 || kq > key)) {
+        key = kq;
+        best = q;
+      }
     }
-    key = max_xor(max_xor(max_row(key), 16), 32);
-    if ((tid & 63) == 0) redk[tid >> 6] = key;
+    const unsigned long long most = max_xor(max_xor(max_row(key), 16), 32);
+    unsigned index = kNone;
+#pragma unroll
+    for (int q = R - 1; q >= 0; --q) {
+      const unsigned long long lanes = __ballot(best == q && key == most);
+      if (lanes) index = (unsigned)((tid & ~63) + q * kLuRows + __ffsll((long long)lanes) - 1);
+    }
+    if ((tid & 63) == 0) {
+      redk[tid >> 6] = most;
+      redi[tid >> 6] = index;
+    }
     __syncthreads();
-    key = max_row(redk[tid & (kLuWaves - 1)]);
-    const int at = (int)(0xffffffffu - (unsigned)(key & 0xffffffffu));
+    const unsigned long long wave_key = redk[tid & (kLuWaves - 1)];
+    const unsigned wave_index = redi[tid & (kLuWaves - 1)];
+    // (a wave without rows has the key 0 and no index)
+    const unsigned first = min_row(wave_key == max_row(wave_key) ? wave_index : kNone);
+    const int at = first == kNone ? j : (int)first;
 #pragma unroll
     for (int q = 0; q < R; ++q)
       if (tid + q * kLuRows == at) {
