@@ -37,7 +37,7 @@ struct SweArgs {
   const double* part;   // [n_part][6]: x, y, z, radius^2, z lower, z upper
   const double2* coef;  // [n_part][B], H: b_(1-tau) staged at tau; unrolled kernels in swe_pair_offset order, else (tau, l, m)
   const double* pts;    // [n_pts][3]
-  void* out;            // [splits][3][n_pts] complex of Real
+  void* out;            // [splits][3][n_pts] complex of Real; one split: [3][n_pts] double2, the result
   int64_t n_part, n_pts;
   int64_t per_split;    // particles per blockIdx.y
   double k_re, k_im;
@@ -66,6 +66,23 @@ __host__ __device__ inline double legendre_mm_prefactor(int m) {
   double res = 1.0;
   for (int t = 2; t <= 2 * m; t += 2) res += res / t;
   return sqrt(res / 2.0);
+}
+
+// A point's sum over the workgroup's particles. The only split's is the result,
+// and no second launch follows (a single wave's field: 56 us a call, 72 with it).
+template <typename C>
+__device__ inline void swe_store(const SweArgs& a, int64_t ip, C ex, C ey, C ez) {
+  if (gridDim.y == 1) {
+    double2* out = reinterpret_cast<double2*>(a.out) + ip;
+    out[0] = make_double2((double)ex.re, (double)ex.im);
+    out[a.n_pts] = make_double2((double)ey.re, (double)ey.im);
+    out[2 * a.n_pts] = make_double2((double)ez.re, (double)ez.im);
+    return;
+  }
+  C* out = reinterpret_cast<C*>(a.out) + 3 * (int64_t)blockIdx.y * a.n_pts + ip;
+  out[0] = ex;
+  out[a.n_pts] = ey;
+  out[2 * a.n_pts] = ez;
 }
 
 // Bound by VALU issue: per pair about 100 instructions of FP64 geometry and
@@ -236,10 +253,7 @@ __global__ void __launch_bounds__(kSwePoints) swe_field_kernel(SweArgs a) {
     }
   }
   if (live) {
-    C* out = reinterpret_cast<C*>(a.out) + 3 * (int64_t)blockIdx.y * a.n_pts + ip;
-    out[0] = ex;
-    out[a.n_pts] = ey;
-    out[2 * a.n_pts] = ez;
+    swe_store(a, ip, ex, ey, ez);
   }
 }
 
@@ -420,10 +434,7 @@ __global__ void __launch_bounds__(kSwePoints) swe_field_any_kernel(SweArgs a, in
     }
   }
   if (live) {
-    C* out = reinterpret_cast<C*>(a.out) + 3 * (int64_t)blockIdx.y * a.n_pts + ip;
-    out[0] = ex;
-    out[a.n_pts] = ey;
-    out[2 * a.n_pts] = ez;
+    swe_store(a, ip, ex, ey, ez);
   }
 }
 
@@ -516,13 +527,13 @@ extern "C" int smh_swe_field(smh_ctx* ctx, int64_t n_part, const double* pos, co
   const size_t csize = precision == SMH_FP32 ? sizeof(float2) : sizeof(double2);
   void* buf[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
   const size_t sizes[5] = {part.size() * 8, cf.size() * 8, (size_t)3 * n_pts * 8, (size_t)3 * n_pts * 16,
-                           (size_t)splits * 3 * n_pts * csize};
+                           splits > 1 ? (size_t)splits * 3 * n_pts * csize : 0};
   auto release = [&]() {
     for (void* q : buf)
       if (q) hipFree(q);
   };
   for (int i = 0; i < 5; ++i)
-    if (hipMalloc(&buf[i], sizes[i]) != hipSuccess) {
+    if (sizes[i] > 0 && hipMalloc(&buf[i], sizes[i]) != hipSuccess) {
       release();
       return smh_fail(ctx, SMH_ERR_HIP, "SWE field device allocation failed");
     }
@@ -537,7 +548,7 @@ extern "C" int smh_swe_field(smh_ctx* ctx, int64_t n_part, const double* pos, co
   a.part = (const double*)buf[0];
   a.coef = (const double2*)buf[1];
   a.pts = (const double*)buf[2];
-  a.out = buf[4];
+  a.out = splits > 1 ? buf[4] : buf[3];
   a.n_part = n_part;
   a.n_pts = n_pts;
   a.per_split = per_split;
@@ -554,7 +565,7 @@ extern "C" int smh_swe_field(smh_ctx* ctx, int64_t n_part, const double* pos, co
   void* args_any[] = {&a, &lmax_, &mmax_, &B_, &chunk};
   if (e == hipSuccess)
     e = hipLaunchKernel(fn, dim3(nb, (unsigned)splits), dim3(kSwePoints), lds ? args_any : args_fixed, lds, s);
-  if (e == hipSuccess) {
+  if (e == hipSuccess && splits > 1) {
     const unsigned sb = (unsigned)((3 * n_pts + 255) / 256);
     if (precision == SMH_FP32)
       hipLaunchKernelGGL(swe_sum_kernel<float>, dim3(sb), dim3(256), 0, s, (const cplx<float>*)buf[4], splits,
