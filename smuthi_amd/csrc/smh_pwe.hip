@@ -760,11 +760,6 @@ extern "C" int smh_pwe_field(smh_ctx* ctx, int kind, int64_t n_k, const double* 
     for (int64_t j = 0; j < n_a; ++j)
       wa[j] = n_a == 1 ? 0.0 : 0.5 * ((j + 1 < n_a ? alpha[j + 1] : alpha[j]) - (j > 0 ? alpha[j - 1] : alpha[j]));
   }
-  std::vector<double> ca(n_a), sa(n_a);
-  for (int64_t j = 0; j < n_a; ++j) {
-    ca[j] = std::cos(alpha[j]);
-    sa[j] = std::sin(alpha[j]);
-  }
   // leaves and their origins; z origin on the side toward which every term decays
   std::vector<PwePoint> pt(n_pts);
   for (int64_t j = 0; j < n_pts; ++j) pt[j] = {{xyz[3 * j], xyz[3 * j + 1], xyz[3 * j + 2]}, j};
@@ -779,8 +774,32 @@ extern "C" int smh_pwe_field(smh_ctx* ctx, int kind, int64_t n_k, const double* 
     kmax = std::max(kmax, std::hypot(kp[2 * k], kp[2 * k + 1]));
     kim = std::max(kim, std::fabs(kp[2 * k + 1]));
   }
-  std::vector<double> pts((size_t)3 * n_pts), org((size_t)4 * n_leaves);
-  std::vector<int> idx(n_pts);
+  // device buffers; the first kUp of them are one block, filled here and uploaded in one copy (each copy of a few KB
+  // takes a call as long as a kernel)
+  enum { KP, KZ, WK, CA, SA, WA, AL, PTS, ORG, LEAF, IDX, LIST, kUp, F_ = kUp, OUT, PART, G_, TRIG, N_BUF };
+  size_t sizes[N_BUF], up_off[kUp + 1] = {0};
+  sizes[KP] = sizes[KZ] = sizes[WK] = (size_t)n_k * 16;
+  sizes[CA] = sizes[SA] = sizes[WA] = sizes[AL] = (size_t)n_a * 8;
+  sizes[PTS] = (size_t)3 * n_pts * 8;
+  sizes[ORG] = (size_t)4 * n_leaves * 8;
+  sizes[LEAF] = bounds.size() * 4;
+  sizes[IDX] = (size_t)n_pts * 4;
+  sizes[LIST] = (size_t)n_leaves * 4;
+  for (int i = 0; i < kUp; ++i) up_off[i + 1] = up_off[i] + (sizes[i] + 15) / 16 * 16;
+  std::vector<double> block(up_off[kUp] / 8);
+  auto in = [&](int i) { return block.data() + up_off[i] / 8; };
+  std::memcpy(in(KP), kp, sizes[KP]);
+  std::memcpy(in(KZ), kz, sizes[KZ]);
+  std::memcpy(in(WK), wk.data(), sizes[WK]);
+  std::memcpy(in(WA), wa.data(), sizes[WA]);
+  std::memcpy(in(AL), alpha, sizes[AL]);
+  std::memcpy(in(LEAF), bounds.data(), sizes[LEAF]);
+  for (int64_t j = 0; j < n_a; ++j) {
+    in(CA)[j] = std::cos(alpha[j]);
+    in(SA)[j] = std::sin(alpha[j]);
+  }
+  double *pts = in(PTS), *org = in(ORG);
+  int* idx = (int*)in(IDX);
   // leaves by kernel: order 0, harmonics with up to 31 orders, up to 63, one term per azimuth. The harmonics pay where
   // their orders (about 20 instructions each, and most kappa have fewer than the largest) are below half the
   // azimuths (26 instructions and three or four transcendental ones each); growth of e^{|Im kappa| rho} would
@@ -801,8 +820,12 @@ extern "C" int smh_pwe_field(smh_ctx* ctx, int kind, int64_t n_k, const double* 
     o[0] = 0.5 * (lo[0] + hi[0]);
     o[1] = 0.5 * (lo[1] + hi[1]);
     o[2] = up ? lo[2] : (down ? hi[2] : 0.5 * (lo[2] + hi[2]));
-    o[3] = 0.0;
-    for (int j = bounds[l]; j < bounds[l + 1]; ++j) o[3] = std::max(o[3], std::hypot(pt[j].x[0] - o[0], pt[j].x[1] - o[1]));
+    double r2 = 0.0;
+    for (int j = bounds[l]; j < bounds[l + 1]; ++j) {
+      const double dx = pt[j].x[0] - o[0], dy = pt[j].x[1] - o[1];
+      r2 = std::max(r2, dx * dx + dy * dy);
+    }
+    o[3] = std::sqrt(r2);
     const int m = max_order(precision, kmax * o[3]);
     const bool harmonics = m >= 0 && 2 * m <= n_a && kim * o[3] <= 1.0;
     list[!harmonics ? 3 : (m == 0 ? 0 : (precision == SMH_FP32 && m < 32 ? 1 : 2))].push_back(l);
@@ -818,53 +841,35 @@ extern "C" int smh_pwe_field(smh_ctx* ctx, int kind, int64_t n_k, const double* 
   const size_t lds = (size_t)2 * n_a * rs + (size_t)kc * n_a * 6 * rs;
   SMH_CHECK(ctx, lds <= 160 * 1024, SMH_ERR_UNSUPPORTED, "too many azimuth samples (%lld)", (long long)n_a);
   const int trig_rows = (int)(n_a + 3) / 4 * 4;
-  std::vector<int> order;
-  for (const std::vector<int>& l : list) order.insert(order.end(), l.begin(), l.end());
-  enum { F_, KP, KZ, CA, SA, PTS, LEAF, ORG, OUT, PART, G_, WK, WA, AL, TRIG, IDX, LIST, N_BUF };
-  void* buf[N_BUF] = {nullptr};
+  const bool harmonic = !list[1].empty() || !list[2].empty();
+  int* order = (int*)in(LIST);
+  for (const std::vector<int>& l : list) order = std::copy(l.begin(), l.end(), order);
   const size_t waves = (size_t)n_k * n_a;
-  size_t sizes[N_BUF];
   sizes[F_] = 3 * waves * 16;
-  sizes[KP] = sizes[KZ] = sizes[WK] = (size_t)n_k * 16;
-  sizes[CA] = sizes[SA] = sizes[WA] = sizes[AL] = (size_t)n_a * 8;
-  sizes[PTS] = pts.size() * 8;
-  sizes[LEAF] = bounds.size() * 4;
-  sizes[ORG] = org.size() * 8;
   sizes[OUT] = (size_t)3 * n_pts * 16;
   sizes[PART] = splits * sizes[OUT];
   sizes[G_] = 2 * waves * 16;
-  sizes[TRIG] = (size_t)trig_rows * 2 * (kMaxM + 1) * rs;
-  sizes[IDX] = idx.size() * 4;
-  sizes[LIST] = order.size() * 4;
+  sizes[TRIG] = harmonic ? (size_t)trig_rows * 2 * (kMaxM + 1) * rs : 0;
+  char* d_up = nullptr;
+  void* buf[N_BUF] = {nullptr};
   auto release = [&]() {
-    for (void* b : buf)
-      if (b) hipFree(b);
+    if (d_up) (void)hipFree(d_up);
+    for (int i = kUp; i < N_BUF; ++i)
+      if (buf[i]) (void)hipFree(buf[i]);
   };
-  for (int i = 0; i < N_BUF; ++i)
-    if (hipMalloc(&buf[i], sizes[i]) != hipSuccess) {
-      release();
-      return smh_fail(ctx, SMH_ERR_HIP, "PWE device allocation failed");
-    }
+  bool ok = hipMalloc(&d_up, up_off[kUp]) == hipSuccess;
+  for (int i = 0; i < kUp && ok; ++i) buf[i] = d_up + up_off[i];
+  for (int i = kUp; i < N_BUF && ok; ++i) ok = sizes[i] == 0 || hipMalloc(&buf[i], sizes[i]) == hipSuccess;
+  if (!ok) {
+    release();
+    return smh_fail(ctx, SMH_ERR_HIP, "PWE device allocation failed");
+  }
   hipStream_t s = ctx->stream;
-  const void* src[N_BUF] = {nullptr};
-  src[KP] = kp;
-  src[KZ] = kz;
-  src[CA] = ca.data();
-  src[SA] = sa.data();
-  src[PTS] = pts.data();
-  src[LEAF] = bounds.data();
-  src[ORG] = org.data();
-  src[G_] = g;
-  src[WK] = wk.data();
-  src[WA] = wa.data();
-  src[AL] = alpha;
-  src[IDX] = idx.data();
-  src[LIST] = order.data();
-  for (int i = 0; i < N_BUF; ++i)
-    if (src[i] && hipMemcpyAsync(buf[i], src[i], sizes[i], hipMemcpyHostToDevice, s) != hipSuccess) {
-      release();
-      return smh_fail(ctx, SMH_ERR_HIP, "PWE upload failed");
-    }
+  if (hipMemcpyAsync(d_up, block.data(), up_off[kUp], hipMemcpyHostToDevice, s) != hipSuccess ||
+      hipMemcpyAsync(buf[G_], g, sizes[G_], hipMemcpyHostToDevice, s) != hipSuccess) {
+    release();
+    return smh_fail(ctx, SMH_ERR_HIP, "PWE upload failed");
+  }
   PweArgs a;
   a.F = (const double2*)buf[F_];
   a.kp = (const double2*)buf[KP];
@@ -895,7 +900,9 @@ extern "C" int smh_pwe_field(smh_ctx* ctx, int kind, int64_t n_k, const double* 
                        (int)n_a, (const double2*)buf[G_], a.kp, a.kz, a.ca, a.sa, (const double2*)buf[WK],
                        (const double*)buf[WA], make_double2(k_re, k_im), (double2*)buf[F_]);
     const unsigned tb = (unsigned)((trig_rows * (kMaxM + 1) + 255) / 256);
-    if (precision == SMH_FP32)
+    if (!harmonic)
+      ;  // (only the harmonics read it)
+    else if (precision == SMH_FP32)
       hipLaunchKernelGGL(pwe_trig_kernel<float>, dim3(tb), dim3(256), 0, s, (int)n_a, trig_rows, (const double*)buf[AL],
                          (float*)buf[TRIG]);
     else
