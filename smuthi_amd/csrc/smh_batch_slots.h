@@ -100,14 +100,17 @@ void slot_tables(int* out) {
 }
 
 // Shape of the slot kernels. A wave holds one entry's tap fragments in
-// registers, T terms x tiles x K-steps values per lane. Blocks too large for
-// that are cut into parts, each a pass over the entry's pairs. FP32: P32 parts
-// of the result tiles (a tile's Re and Im rows together) within 128 registers,
-// each rotating and adding its own rows (2501 spheres, l_max 4, 3 parts: a
-// block product takes 17.0 ms, 18.4 with parts of the K-steps, which repeat the
-// rotation and the LDS additions of all rows). FP64: P64 parts of an even
-// number of K-steps within 64 values (10000 spheres, l_max 3, 2 parts: 184 ms, 199 with parts of the
-// tiles, which repeat the input's loads and rotation).
+// registers, T terms x tiles x K-steps values per lane (fits: the FP32 kernel's
+// in one set of at most 128). Larger blocks split the K-steps into parts, each
+// a pass over the entry's pairs with its own epilogue: P32 parts of whole
+// float4 groups (4 K-steps) within 128 FP32 registers, P64 parts of an even
+// number of K-steps within 64 FP64 values (0: no such split). The parts' sums
+// meet in the accumulators' 64-bit words. Parts of the result tiles instead, each
+// with all K-steps, rotate and add every row once, but the K-steps' sums meet in
+// FP32: 2501 spheres, l_max 4, 3 parts, FP32: a block product 17.0 ms against
+// 18.4, error 2.166e-7 against 2.154e-7 (1500 to 4000 spheres: 0.5 % larger
+// throughout). FP64, 10000 spheres, l_max 3, 2 parts: 184 ms, 199 with parts of
+// the tiles, which repeat the input's loads and rotation.
 template <int L, int M, int T>
 struct SlotShape {
   static constexpr int S = SvwfIdx<L, M>::Bh, NS = S / 4, MT = 2 * S / 16, MH = MT / 2;
@@ -115,18 +118,13 @@ struct SlotShape {
   static constexpr int LO = 2 * kBatchRhs * SC;  // int64 accumulator words per receiver
   static constexpr int SY = 2 * LO;         // LDS int32 words per receiver
   static constexpr int FRB = MT * NS * 64;  // floats per tap row
-  static constexpr int tile_parts(int budget) {
-    for (int p = 1; p <= MH; ++p)
-      if (MH % p == 0 && T * 2 * (MH / p) * NS <= budget) return p;
-    return MH;
-  }
-  static constexpr int step_parts(int budget) {
+  static constexpr bool fits = T * MT * NS <= 128;
+  static constexpr int parts(int budget, int step) {
     for (int p = 1; p <= NS; ++p)
-      if (NS % p == 0 && (NS / p) % 2 == 0 && T * MT * (NS / p) <= budget) return p;
+      if (NS % p == 0 && (NS / p) % step == 0 && T * MT * (NS / p) <= budget) return p;
     return 0;
   }
-  static constexpr int P32 = tile_parts(128), P64 = step_parts(64);
-  static constexpr bool fits32 = T * 2 * (MH / P32) * NS <= 128;
+  static constexpr int P32 = parts(128, 4), P64 = parts(64, 2);
 };
 
 // cos(k phi), sin(k phi) for k <= K from cos phi, sin phi (angle addition)
@@ -189,9 +187,9 @@ __global__ void __launch_bounds__(512) batch_slots_kernel(RadialKArgs a) {
   constexpr int S = Sh::S, NS = Sh::NS, MT = Sh::MT, MH = Sh::MH, SC = Sh::SC, LO = Sh::LO;
   constexpr int KB = kBatchRhs;
   static_assert(KB * 2 == 16, "16 result columns = kBatch right-hand sides x (re, im)");
-  // result tiles in P parts (one register set of tap fragments per part)
-  constexpr int P = Sh::P32, MHP = MH / P;
-  static_assert(Sh::fits32, "tap fragments exceed the register budget");
+  // K-steps in P parts (one register set of tap fragments per part)
+  constexpr int P = Sh::P32, NSP = NS / (P > 0 ? P : 1);
+  static_assert(P > 0, "tap fragments exceed the register budget");
   static_assert(MMAX <= 4, "phase selection covers |m| <= 4");
   constexpr SlotOrder<LMAX, MMAX> so{};
   static_assert(so.ok, "slot order");
@@ -204,7 +202,9 @@ __global__ void __launch_bounds__(512) batch_slots_kernel(RadialKArgs a) {
   const int item = a.order ? a.order[blockIdx.x] : (int)blockIdx.x;
   float sh = 0.f;
   double ish = 0.0;
-  fixed_scale64(a.item_lsum[item], *a.xmax, a.item_en[item], sh, ish);
+  // each pair adds once per part to each word of its receiver
+  constexpr int PB = P <= 1 ? 0 : (P <= 2 ? 1 : (P <= 4 ? 2 : (P <= 8 ? 3 : 4)));  // ceil(log2 P)
+  fixed_scale64(a.item_lsum[item], *a.xmax, a.item_en[item] + PB, sh, ish);
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int2 it = a.items[item];
@@ -256,35 +256,35 @@ __global__ void __launch_bounds__(512) batch_slots_kernel(RadialKArgs a) {
     const int p_end = en.z;
 #pragma unroll
     for (int h = 0; h < P; ++h) {
-      // polynomial coefficients tv[t][ti][s] = c_t(row rr of the part's tile ti, slot 4 s + q) of the entry's
-      // bin: tile h MHP + ti (ti < MHP, Re L) or MH + h MHP + ti - MHP (Im L) (VOL: the values of the entry's tap t)
-      float tv[T][2 * MHP][NS];
+      // K-steps s0 .. s0 + NSP - 1 of this part
+      const int s0 = h * NSP;
+      // polynomial coefficients tv[t][i][s] = c_t(tile i row rr, slot 4 (s0 + s) + q) of the entry's bin
+      // (VOL: the values of the entry's tap t)
+      float tv[T][MT][NSP];
 #pragma unroll
       for (int t = 0; t < T; ++t) {
         const size_t trow =
             VOL ? (size_t)(en.x + vol_tap_offset(a.vmode, a.vslice, t, a.len_z)) : (size_t)bin * T + t;
         const float4* row = tt4 + trow * (Sh::FRB / 4);
 #pragma unroll
-        for (int ti = 0; ti < 2 * MHP; ++ti) {
-          const int i = ti < MHP ? h * MHP + ti : MH + h * MHP + ti - MHP;
+        for (int i = 0; i < MT; ++i)
 #pragma unroll
-          for (int s4 = 0; s4 < NS / 4; ++s4) {
-            const float4 v = row[(i * (NS / 4) + s4) * 64 + lane];
-            tv[t][ti][4 * s4 + 0] = v.x;
-            tv[t][ti][4 * s4 + 1] = v.y;
-            tv[t][ti][4 * s4 + 2] = v.z;
-            tv[t][ti][4 * s4 + 3] = v.w;
+          for (int s4 = 0; s4 < NSP / 4; ++s4) {
+            const float4 v = row[(i * (NS / 4) + s0 / 4 + s4) * 64 + lane];
+            tv[t][i][4 * s4 + 0] = v.x;
+            tv[t][i][4 * s4 + 1] = v.y;
+            tv[t][i][4 * s4 + 2] = v.z;
+            tv[t][i][4 * s4 + 3] = v.w;
           }
-        }
       }
-      auto load_x = [&](const Rec& r, float4 (&xs)[NS / 2]) {
+      auto load_x = [&](const Rec& r, float4 (&xs)[NSP / 2]) {
         const float4* xp =
-            reinterpret_cast<const float4*>(xg + (int64_t)(r.ij & kPairMask) * S * KB + xlane);
+            reinterpret_cast<const float4*>(xg + (int64_t)(r.ij & kPairMask) * S * KB + xlane) + s0 / 2;
 #pragma unroll
-        for (int k = 0; k < NS / 2; ++k) xs[k] = xp[k];
+        for (int k = 0; k < NSP / 2; ++k) xs[k] = xp[k];
       };
       Rec rec_n = recs[en.y];
-      float4 xc[NS / 2];
+      float4 xc[NSP / 2];
       load_x(rec_n, xc);
       for (int p = 0; p < p_end; ++p) {
         const Rec rec = rec_n;
@@ -305,17 +305,17 @@ __global__ void __launch_bounds__(512) batch_slots_kernel(RadialKArgs a) {
         for (int k = 1; k <= MMAX; ++k) ez[k] = xor_sign(sn[k], zmask);
 
         // B operand per K-step: (e^{i m2 phi} x[slot 4 s + q][rhs]).re or .im
-        float z[NS];
+        float z[NSP];
 #pragma unroll
-        for (int s = 0; s < NS; ++s) {
+        for (int s = 0; s < NSP; ++s) {
           const float4 x4 = xc[s >> 1];
           const float xr = (s & 1) ? x4.z : x4.x, xi = (s & 1) ? x4.w : x4.y;
           const float av0 = zp ? xi : xr, bv0 = zp ? xr : xi;
-          const int am = so.absm[s];
+          const int am = so.absm[s0 + s];
           if (am == 0) {
             z[s] = av0;
           } else {
-            const int sg = so.sgn[s];
+            const int sg = so.sgn[s0 + s];
             const float e = sg > 0 ? ez[am] : (sg < 0 ? -ez[am] : xor_sign(ez[am], qmask));
             z[s] = fmaf(cs[am], av0, e * bv0);
           }
@@ -323,17 +323,13 @@ __global__ void __launch_bounds__(512) batch_slots_kernel(RadialKArgs a) {
         // the input of the next pair goes into the same registers
         load_x(rec_n, xc);
 
-        // (long rows: a sum per four K-steps, added at the end, keeps the chains of FP32 sums short)
-        constexpr int NA = P > 1 ? NS / 4 : 1;
-        typename Mfma<float>::v4 acc[2 * MHP], sum[2 * MHP][NA];
+        typename Mfma<float>::v4 acc[MT];
 #pragma unroll
-        for (int i = 0; i < 2 * MHP; ++i)
+        for (int i = 0; i < MT; ++i) acc[i] = typename Mfma<float>::v4{0, 0, 0, 0};
 #pragma unroll
-          for (int k = 0; k < NA; ++k) sum[i][k] = typename Mfma<float>::v4{0, 0, 0, 0};
+        for (int s = 0; s < NSP; ++s) {
 #pragma unroll
-        for (int s = 0; s < NS; ++s) {
-#pragma unroll
-          for (int i = 0; i < 2 * MHP; ++i) {
+          for (int i = 0; i < MT; ++i) {
             float v;
             if constexpr (VOL) {
               v = wt[0] * tv[0][i][s];
@@ -344,21 +340,14 @@ __global__ void __launch_bounds__(512) batch_slots_kernel(RadialKArgs a) {
 #pragma unroll
               for (int t = T - 2; t >= 0; --t) v = fmaf(v, w, tv[t][i][s]);
             }
-            sum[i][s % NA] = Mfma<float>::op(v, z[s], sum[i][s % NA]);
+            acc[i] = Mfma<float>::op(v, z[s], acc[i]);
           }
-        }
-#pragma unroll
-        for (int i = 0; i < 2 * MHP; ++i) {
-          acc[i] = sum[i][0];
-#pragma unroll
-          for (int k = 1; k < NA; ++k) acc[i] += sum[i][k];
         }
 
         // y (rhs, re|im) of rows 16 i + 4 q + v, rotated by e^{-i m1 phi}, scaled by S_hi
         unsigned long long* yrow = yacc + (size_t)(rec.ij >> kPairShift) * LO + colbase;
 #pragma unroll
-        for (int ti = 0; ti < MHP; ++ti) {
-          const int i = h * MHP + ti;
+        for (int i = 0; i < MH; ++i) {
           float er = 0.f, ei = 0.f;
 #pragma unroll
           for (int am = 0; am <= MMAX; ++am) {
@@ -375,7 +364,7 @@ __global__ void __launch_bounds__(512) batch_slots_kernel(RadialKArgs a) {
 #pragma unroll
           for (int v = 0; v < 4; ++v) {
             const float eps = v < 2 ? elo : ehi;
-            const float al = acc[ti][v], be = acc[ti + MHP][v];
+            const float al = acc[i][v], be = acc[i + MH][v];
             const float own = fmaf(al, er, be * eps);
             const float snd = fmaf(be, er, -(al * eps));
             const float val = fma_xor1(own, sgnz, snd);
@@ -392,7 +381,7 @@ __global__ void __launch_bounds__(512) batch_slots_kernel(RadialKArgs a) {
     const int il = j / (2 * KB * S), k = j - il * 2 * KB * S;
     const int c = k / S, sl2 = k - c * S;
     const int w0 = il * LO + c * SC + sl2;
-    const long long sum = (long long)(yacc[w0] - (unsigned long long)n_adds[il] * kMagic64Bits);  // modulo 2^64
+    const long long sum = (long long)(yacc[w0] - (unsigned long long)n_adds[il] * P * kMagic64Bits);  // modulo 2^64
     yp[j] = (float)((double)sum * ish);
   }
 }

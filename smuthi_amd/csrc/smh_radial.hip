@@ -387,7 +387,7 @@ KernelInfo pick(int l, int m) {
 template <int L, int Mx, int T, typename Real>
 KernelInfo batch_kernel_info() {
   KernelInfo k;
-  if constexpr (std::is_same<Real, float>::value && SlotShape<L, Mx, T>::fits32 && Mx <= 4) {
+  if constexpr (std::is_same<Real, float>::value && SlotShape<L, Mx, T>::P32 > 0 && Mx <= 4) {
     k.fn = reinterpret_cast<void*>(&batch_slots_kernel<L, Mx, T>);
     k.threads = 512;
     k.sy = SlotShape<L, Mx, T>::SY;  // int32 words (one int64 word per result)
@@ -425,7 +425,7 @@ KernelInfo pick_batch(int l, int m) {
 // (its binning and slot order)
 template <int L, int Mx, int T>
 void* half_fn() {
-  if constexpr (SlotShape<L, Mx, 4>::fits32 && Mx <= 4 && half_tile_parts(T, SvwfIdx<L, Mx>::B) > 0)
+  if constexpr (SlotShape<L, Mx, 4>::P32 > 0 && Mx <= 4 && half_tile_parts(T, SvwfIdx<L, Mx>::B) > 0)
     return reinterpret_cast<void*>(&batch_half_kernel<L, Mx, T>);
   else
     return nullptr;
