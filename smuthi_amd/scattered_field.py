@@ -5,6 +5,7 @@ scatterers, the outgoing SWE -> PWE conversion
 libsmh launch (smh_pwe_assemble); the direct part and the layer response
 (layers.py:141-191) are combined on the host.
 """
+import copy
 import ctypes
 
 import numpy as np
@@ -135,7 +136,10 @@ def _scattered_field_pwe(vacuum_wavelength, by_layer, scatterers, layer_system, 
         # the terms' common grids (the assembly's), wavenumber and reference point, as PlaneWaveExpansion.__add__
         # checks them
         n = layer_system.refractive_indices
-        if not out[0].compatible(PlaneWaveExpansion(k_swe / n[i_swe] * n[layer_number], kp, al, 'upgoing', [0, 0, z])):
+        term = copy.copy(out[0])
+        term.k, term.k_parallel, term.azimuthal_angles = k_swe / n[i_swe] * n[layer_number], kp, al
+        term.reference_point = list(out[0].reference_point)
+        if not out[0].compatible(term):
             raise ValueError('Plane wave expansion are inconsistent.')
         if direct:
             out[0].lower_z, out[1].upper_z = max(vb[0], xyz[:, 2].max()), min(vb[1], xyz[:, 2].min())
