@@ -82,10 +82,10 @@ __host__ __device__ constexpr int half_tile_parts(int T, int B) {
   return 0;
 }
 
-// VOL: volume lookups. The table holds the tap rows in this kernel's
-// fragment order ([rows][MT][64 lanes][NC][4] FP16, one row per tap row of the
-// volume lookup), each row divided by its own power of two hscale[row]; an
-// entry's T taps of z slice a.vslice sit at rows en.x + vol_tap_offset, and a
+// VOL: bilinear volume lookups (cubic ones: smh_batch_volume.h). The table holds
+// the tap rows in this kernel's fragment order ([rows][MT][64 lanes][NC][4]
+// FP16, one row per node), each row divided by its own power of two
+// hscale[row]; an entry's T = 4 taps sit at rows en.x + vol_tap_offset, and a
 // pair weights them with vol_tap_weight(w, w2) hscale[row] / (the largest of
 // the entry's four scales), which then scales the result. The weights go to
 // the input side (one MFMA per tap), so the taps are summed in FP32.
@@ -306,7 +306,7 @@ __global__ void __launch_bounds__(kHalfThreads) batch_half_kernel(RadialKArgs a,
       if constexpr (VOL) {
 #pragma unroll
         for (int t = 0; t < T; ++t) {
-          const _Float16 h = (_Float16)(vol_tap_weight<float>(a.vmode, a.vslice, t, rec.w, rec.w2) * rel[t]);
+          const _Float16 h = (_Float16)(vol_tap_weight<float>(kVolBilinear, 0, t, rec.w, rec.w2) * rel[t]);
           wt[t] = half4_t{h, h, h, h};
         }
       }
@@ -382,7 +382,7 @@ __global__ void __launch_bounds__(kHalfThreads) batch_half_kernel(RadialKArgs a,
     const int4 en = a.entries[e];
     int rows[T];
 #pragma unroll
-    for (int t = 0; t < T; ++t) rows[t] = VOL ? en.x + vol_tap_offset(a.vmode, a.vslice, t, a.len_z) : 0;
+    for (int t = 0; t < T; ++t) rows[t] = VOL ? en.x + vol_tap_offset(kVolBilinear, 0, t, a.len_z) : 0;
 #pragma unroll
     for (int h = 0; h < TP; ++h) {
       load_coef(bin_of(en), rows, tv, h);

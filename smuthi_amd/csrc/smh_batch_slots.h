@@ -176,11 +176,10 @@ __device__ inline float fma_xor1(float v, float c, float other) {
   return fmaf(c, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(other), 0xB1, 0xF, 0xF, false)), v);
 }
 
-// VOL: volume lookups. The table holds tap rows in the same slot fragment
-// order ([rows][MT][NS/4][64 lanes][4], one row per tap row of the volume
-// lookup: node * vq + moment kind); an entry's T taps for z slice a.vslice sit
-// at rows en.x + vol_tap_offset(a.vmode, a.vslice, t, a.len_z), and a pair
-// weights them with vol_tap_weight(w, w2) instead of Horner in w.
+// VOL: bilinear volume lookups (cubic ones: smh_batch_volume.h). The table holds
+// tap rows in the same slot fragment order ([rows][MT][NS/4][64 lanes][4], one
+// row per node); an entry's T = 4 taps sit at rows en.x + vol_tap_offset, and a
+// pair weights them with vol_tap_weight(w, w2) instead of Horner in w.
 template <int LMAX, int MMAX, int T, bool VOL = false>
 __global__ void __launch_bounds__(512) batch_slots_kernel(RadialKArgs a) {
   using Sh = SlotShape<LMAX, MMAX, T>;
@@ -264,7 +263,7 @@ __global__ void __launch_bounds__(512) batch_slots_kernel(RadialKArgs a) {
 #pragma unroll
       for (int t = 0; t < T; ++t) {
         const size_t trow =
-            VOL ? (size_t)(en.x + vol_tap_offset(a.vmode, a.vslice, t, a.len_z)) : (size_t)bin * T + t;
+            VOL ? (size_t)(en.x + vol_tap_offset(kVolBilinear, 0, t, a.len_z)) : (size_t)bin * T + t;
         const float4* row = tt4 + trow * (Sh::FRB / 4);
 #pragma unroll
         for (int i = 0; i < MT; ++i)
@@ -294,7 +293,7 @@ __global__ void __launch_bounds__(512) batch_slots_kernel(RadialKArgs a) {
         float wt[T];  // VOL: the pair's tap weights
         if constexpr (VOL) {
 #pragma unroll
-          for (int t = 0; t < T; ++t) wt[t] = vol_tap_weight<float>(a.vmode, a.vslice, t, rec.w, rec.w2);
+          for (int t = 0; t < T; ++t) wt[t] = vol_tap_weight<float>(kVolBilinear, 0, t, rec.w, rec.w2);
         }
         // cos / sin of k phi, k = 1..MMAX
         float cs[MMAX + 1], sn[MMAX + 1];

@@ -149,7 +149,7 @@ struct RadialKArgs {
   int n_items, n_entries, interp, Rc;
   int len_z;                // 2-D lookups: table rows per distance node (tap t sits at (t/2) len_z + t%2)
   int row_s = 1, row_o = 0;  // entry tap row = row_s * bin + row_o (kernels on per-bin coefficient rows)
-  int vmode = 1, vslice = 0;  // volume lookups: interpolation mode and z slice (vol_tap_offset)
+  int vmode = 1, vslice = 0;  // single-vector volume lookups: interpolation mode and z slice (vol_tap_offset)
   // block -> work item (null: identity). Items sorted by first table row and
   // dealt so that the blocks one XCD runs (blockIdx mod 8) walk neighbouring
   // bins together and share the tap rows in that XCD's L2.
@@ -256,13 +256,15 @@ struct RadialShape {
 // Volume lookups over nodes (distance r, z index j). vmode 1, bilinear: one
 // launch per table, nodes at row r * len_z + j, taps (r, j), (r, j+1),
 // (r+1, j), (r+1, j+1). vmode 2 (tensor Catmull-Rom) and 3 (tensor not-a-knot
-// spline) run as four launches per table, one per z tap s ("slice"), each a
-// 4-tap interpolation along rho weighted by the slice's z weight:
+// spline) have four z taps s ("slices"), each a 4-tap interpolation along rho
+// weighted by the slice's z weight; single vectors take one launch per table
+// and slice:
 //   Catmull-Rom: tap t at node (r + t - 1, j + s - 1), one row per node;
 //   spline: four rows per node (value, rho moment, z moment, mixed moment,
 //   moments Mh = h^2/6 S''), tap t = (node r + t/2, rho kind t%2), slice
 //   s = (node j + s/2, z kind s%2), weights of tap_weight() in each direction.
 // Offsets are relative to the entry's row (node (r, j)).
+constexpr int kVolBilinear = 1;
 __host__ __device__ inline int vol_tap_offset(int vmode, int s, int t, int len_z) {
   if (vmode == 2) return (t - 1) * len_z + (s - 1);
   if (vmode == 3) return 4 * ((t >> 1) * len_z + (s >> 1)) + (t & 1) + 2 * (s & 1);

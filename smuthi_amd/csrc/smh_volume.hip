@@ -533,7 +533,7 @@ KernelInfo vol_chunk_kernel_info(VolBatch form) {
       k.sy = Sh::SY;
       break;
     case kVolFp64Rows32:
-      k.fn = reinterpret_cast<void*>(&batch_slots64_kernel<L, Mx, 4, true, true>);
+      k.fn = reinterpret_cast<void*>(&batch_slots64_kernel<L, Mx, 4, true>);
       k.threads = kSlots64Threads;
       k.sy = Sh::LO;  // doubles
       break;
@@ -1107,7 +1107,6 @@ int vol_apply_batch(smh_op* op, int precision, const void* x_pad, void* y_pad, b
       a.interp = op->interp;
       a.Rc = bn.Rc;
       a.len_z = (int)op->len_z;
-      a.vmode = op->vmode;
       a.row_s = 1;
       a.row_o = 0;
       if (int rc_ = op_set_lds(op, k.fn, bn.lds)) return rc_;
