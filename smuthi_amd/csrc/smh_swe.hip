@@ -518,7 +518,8 @@ extern "C" int smh_swe_field(smh_ctx* ctx, int64_t n_part, const double* pos, co
           }
         }
   }
-  // particles split so that about eight workgroups a CU run (256 x 8; a split sums at least kSweChunk particles)
+  // particles split so that about eight workgroups a CU run (256 x 8), into no more splits than chunks of kSweChunk,
+  // and evenly (33 particles: 17 and 16)
   const unsigned nb = (unsigned)((n_pts + kSwePoints - 1) / kSwePoints);
   const int64_t want = std::max<int64_t>(1, std::min<int64_t>((8 * (int64_t)ctx->num_cu + nb - 1) / nb,
                                                               (n_part + kSweChunk - 1) / kSweChunk));
