@@ -352,10 +352,11 @@ inline void fill_zero(void* p, size_t bytes, hipStream_t s) {
 // per CU in k items each, a CU spends W + k kItemCost and waits about half an
 // item at the end: the sum is least at k = sqrt(W / (2 kItemCost)) (1023
 // spheres, l_max 2, FP64: 4 items per CU, where 16 write and read 260 MB of
-// partials). The FP64 kBatch-RHS kernel keeps small items: it adds with FP64
-// atomics in no fixed order, and where an item holds few pairs of a receiver
-// the residuals that certify a solve repeat to the last bit. The autotuner
-// (smh_op_autotune) may regroup.
+// partials). The FP64 kBatch-RHS kernel keeps small items: it adds an item's
+// pairs with FP64 atomics in no fixed order, and the fewer pairs of a receiver
+// an item holds, the less the sums that certify a solve differ from run to run
+// (with larger items by more than 1e-12 of a batched solution). The
+// autotuner (smh_op_autotune) may regroup.
 constexpr int kMaxItemsPerCu = 16;
 constexpr double kItemCost = 8.0, kItemCostBatch = 12.0;
 inline int default_items_per_cu(double cost_per_cu, bool batch, bool fp64) {

@@ -830,7 +830,8 @@ extern "C" int smh_pwe_field(smh_ctx* ctx, int kind, int64_t n_k, const double* 
     const bool harmonics = m >= 0 && 2 * m <= n_a && kim * o[3] <= 1.0;
     list[!harmonics ? 3 : (m == 0 ? 0 : (precision == SMH_FP32 && m < 32 ? 1 : 2))].push_back(l);
   }
-  // kappa ranges: about eight workgroups per CU, at least 16 kappa each
+  // kappa ranges: about eight workgroups per CU, no more ranges than 16s of kappa, whole eights of kappa each (the
+  // last one what is left)
   const int want = (int)std::max<int64_t>(1, std::min<int64_t>((8 * (int64_t)ctx->num_cu + n_leaves - 1) / n_leaves,
                                                                (n_k + 15) / 16));
   const int per_split = (int)((n_k + want - 1) / want + 7) / 8 * 8;
