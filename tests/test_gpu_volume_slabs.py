@@ -11,6 +11,8 @@ order, sqrt(n taps) 1e-16 of the result, 1e-12 with room. FP32 rounds weights,
 taps, phases and products to 2^-24, some of each per term, averaged over the
 terms: 3e-6 as in the oracle tests. FP16 operands: 2^-11 per operand, 3e-3 as
 there."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -28,8 +30,26 @@ def gpu():
     return cuda
 
 
-def _operator(n, l_max, m_max, kind, heights, seed, size=1.0, zero_below=0.0):
+def _ensembles(offsets):
+    """Class of volume operators over the ensembles of particles [offsets[e], offsets[e + 1])."""
+    from smuthi_amd import _lib, cuda
     from smuthi_amd.volume import CouplingMatrixVolumeLookupCUDA
+
+    class Ensembles(CouplingMatrixVolumeLookupCUDA):
+        def _create(self, xyz):
+            off = np.ascontiguousarray(offsets, dtype=np.int64)
+            self._op = ctypes.c_void_p()
+            _lib.check(_lib.load().smh_volume_create_ensembles(
+                cuda.context(), len(off) - 1, off.ctypes.data_as(ctypes.POINTER(ctypes.c_int64)), _lib.dptr(xyz),
+                _lib.iptr(self._lmax), _lib.iptr(self._mmax), self.l_max, self.m_max, float(self.rho_array[0]),
+                float(self.sum_z_array[0]), float(self.diff_z_array[0]), float(self.resolution), len(self.rho_array),
+                len(self.sum_z_array), self._interp, ctypes.byref(self._op)), cuda.context(), 'create')
+    return Ensembles
+
+
+def _operator(n, l_max, m_max, kind, heights, seed, size=1.0, zero_below=0.0, offsets=None):
+    from smuthi_amd.volume import CouplingMatrixVolumeLookupCUDA
+    make = CouplingMatrixVolumeLookupCUDA if offsets is None else _ensembles(offsets)
     rng = np.random.default_rng(seed)
     m = int(np.ceil(np.sqrt(n)))
     site = rng.permutation(m * m)[:n]
@@ -50,7 +70,7 @@ def _operator(n, l_max, m_max, kind, heights, seed, size=1.0, zero_below=0.0):
     kw = {'linear': dict(interpolator_kind='linear'),
           'catmull-rom': dict(interpolator_kind='cubic', cubic_interpolant='catmull-rom'),
           'spline': dict(interpolator_kind='cubic', cubic_interpolant='spline')}[kind]
-    return CouplingMatrixVolumeLookupCUDA.from_tables(table(sz), table(dz), rho, sz, dz, parts, H, **kw), rng
+    return make.from_tables(table(sz), table(dz), rho, sz, dz, parts, H, **kw), rng
 
 
 @pytest.mark.parametrize('n,l_max,m_max,kind,heights', [
@@ -74,6 +94,27 @@ def test_batched_matvecs_match_single_vector(gpu, n, l_max, m_max, kind, heights
             assert err.max() < tol, (precision, err)
             # cubic: sums in a fixed order, the same to the last bit
             assert kind == 'linear' or np.array_equal(got, op.matvec(V, precision))
+
+
+@pytest.mark.parametrize('kind,l_max', [('linear', 2), ('catmull-rom', 3), ('spline', 1)])
+def test_ensembles_of_different_sizes(gpu, kind, l_max):
+    """Pairs of one ensemble only: one operator over 1, 37, 2 and 60 particles against the operator over all hundred,
+    applied to the vectors of one ensemble at a time."""
+    off = [0, 1, 38, 40, 100]
+    op, rng = _operator(100, l_max, l_max, kind, None, 9, offsets=off)
+    whole, _ = _operator(100, l_max, l_max, kind, None, 9)
+    B = op.blocksize
+    V = rng.standard_normal((8, op.shape[0])) + 1j * rng.standard_normal((8, op.shape[0]))
+    want = np.zeros_like(V)
+    for a, b in zip(off[:-1], off[1:]):
+        part = np.zeros_like(V)
+        part[:, a * B:b * B] = V[:, a * B:b * B]
+        want[:, a * B:b * B] = np.stack([whole.matvec(v, 'double') for v in part])[:, a * B:b * B]
+    for precision, tol in (('double', 1e-12), ('single', 3e-6), ('half', 3e-3)):
+        got = op.matvec(V, precision)
+        for a, b in zip(off[:-1], off[1:]):
+            g, w = got[:, a * B:b * B], want[:, a * B:b * B]
+            assert np.linalg.norm(g - w) < tol * np.linalg.norm(w), (precision, a)
 
 
 @pytest.mark.parametrize('kind', ['linear', 'catmull-rom', 'spline'])
