@@ -6,6 +6,8 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -15,6 +17,10 @@ struct smh_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  // solver steps are recorded into graphs on this stream, by one thread at a
+  // time; nothing runs on it
+  hipStream_t capture = nullptr;
+  std::shared_ptr<std::mutex> capture_lock = std::make_shared<std::mutex>();
   std::string last_error;
   int num_cu = 0;
   size_t lds_per_block = 0;

@@ -19,6 +19,15 @@ int smh_fail(smh_ctx* ctx, int code, const char* fmt, ...) {
   return code;
 }
 
+// Streams and events of a context, and the context.
+static void release(smh_ctx* ctx) {
+  hipEventDestroy(ctx->ev0);
+  hipEventDestroy(ctx->ev1);
+  hipStreamDestroy(ctx->capture);
+  hipStreamDestroy(ctx->stream);
+  delete ctx;
+}
+
 extern "C" int smh_init(int device, smh_ctx** out) {
   if (!out) return SMH_ERR_ARG;
   *out = nullptr;
@@ -29,6 +38,7 @@ extern "C" int smh_init(int device, smh_ctx** out) {
   ctx->device = device;
   hipError_t e = hipSetDevice(device);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&ctx->capture, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipEventCreate(&ctx->ev0);
   if (e == hipSuccess) e = hipEventCreate(&ctx->ev1);
   hipDeviceProp_t prop;
@@ -41,10 +51,7 @@ extern "C" int smh_init(int device, smh_ctx** out) {
   void* sp = nullptr;
   if (e == hipSuccess) e = hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch));
   if (e != hipSuccess || sp == nullptr) {
-    hipEventDestroy(ctx->ev0);
-    hipEventDestroy(ctx->ev1);
-    hipStreamDestroy(ctx->stream);
-    delete ctx;
+    release(ctx);
     return SMH_ERR_HIP;
   }
   ctx->scratch = static_cast<char*>(sp);
@@ -53,10 +60,7 @@ extern "C" int smh_init(int device, smh_ctx** out) {
   snprintf(ctx->arch, sizeof(ctx->arch), "%s", prop.gcnArchName);
   if (strncmp(ctx->arch, "gfx950", 6) != 0) {
     fprintf(stderr, "smh: device %d is %s, kernels are built for gfx950\n", device, ctx->arch);
-    hipEventDestroy(ctx->ev0);
-    hipEventDestroy(ctx->ev1);
-    hipStreamDestroy(ctx->stream);
-    delete ctx;
+    release(ctx);
     return SMH_ERR_UNSUPPORTED;
   }
   *out = ctx;
@@ -67,10 +71,7 @@ void smh_ctx_release_if_idle(smh_ctx* ctx) {
   if (!ctx || !ctx->destroy_requested || ctx->live_ops > 0) return;
   hipSetDevice(ctx->device);
   hipStreamSynchronize(ctx->stream);
-  hipEventDestroy(ctx->ev0);
-  hipEventDestroy(ctx->ev1);
-  hipStreamDestroy(ctx->stream);
-  delete ctx;
+  release(ctx);
 }
 
 extern "C" int smh_destroy(smh_ctx* ctx) {
@@ -81,10 +82,7 @@ extern "C" int smh_destroy(smh_ctx* ctx) {
   }
   hipSetDevice(ctx->device);
   hipStreamSynchronize(ctx->stream);
-  hipEventDestroy(ctx->ev0);
-  hipEventDestroy(ctx->ev1);
-  hipStreamDestroy(ctx->stream);
-  delete ctx;
+  release(ctx);
   return SMH_OK;
 }
 

@@ -511,7 +511,6 @@ struct SolveWs {
   // systems' norms or residuals
   int* h_live = nullptr;
   double2* h_val = nullptr;
-  hipStream_t capture = nullptr;  // the graphs' steps are recorded on it, nothing runs there
   std::map<int, hipGraphExec_t> graphs;
   std::set<int> ran;  // steps that have run since the graphs were dropped
 
@@ -526,7 +525,6 @@ struct SolveWs {
                  atol, scale, live, kr, nlive, x32, y32, x16};
     for (void* q : p)
       if (q) (void)hipFree(q);
-    if (capture) (void)hipStreamDestroy(capture);
     if (h_live) (void)hipHostFree(h_live);
     if (h_val) (void)hipHostFree(h_val);
     *this = SolveWs();
@@ -723,13 +721,13 @@ struct Solver {
     if (it == ws->graphs.end()) {
       // the matvec counters count launches: the replay below counts this step's one matvec
       const int64_t c64 = mv64, c32 = mv32, c16 = mv16;
-      // recorded on a stream of the workspace's own: threads with other operators share the context's stream,
+      // recorded on the stream that only captures use: threads with other operators share the context's other one,
       // whose work would end up in this graph, and whose synchronizations fail, during the capture
-      if (!ws->capture) SMH_HIP(ctx, hipStreamCreateWithFlags(&ws->capture, hipStreamNonBlocking));
-      SMH_HIP(ctx, hipStreamBeginCapture(ws->capture, hipStreamCaptureModeRelaxed));
+      std::unique_lock<std::mutex> one(*ctx->capture_lock);
+      SMH_HIP(ctx, hipStreamBeginCapture(ctx->capture, hipStreamCaptureModeRelaxed));
       smh_ctx* const home = ctx;
       smh_ctx recording = *ctx;
-      recording.stream = s = ws->capture;
+      recording.stream = s = ctx->capture;
       op->ctx = ctx = &recording;
       const int rc = arnoldi_step(k, precision);
       op->ctx = ctx = home;
@@ -739,7 +737,8 @@ struct Solver {
       mv32 = c32;
       mv16 = c16;
       hipGraph_t graph = nullptr;
-      const hipError_t e = hipStreamEndCapture(ws->capture, &graph);
+      const hipError_t e = hipStreamEndCapture(ctx->capture, &graph);
+      one.unlock();
       if (rc || e != hipSuccess) {
         if (graph) (void)hipGraphDestroy(graph);
         return rc ? rc : smh_fail(ctx, SMH_ERR_HIP, "graph capture failed: %s", hipGetErrorString(e));
