@@ -284,9 +284,8 @@ int smh_op_bench_matvec_batch(smh_op *op, int precision, int iters, double *kern
  * scales only). Drops the solver's captured graphs. The 8-RHS kernels of
  * cubic volume lookups have no work items: their one launch is timed once,
  * matvec_ms holds that time for every candidate, *best is 0 and the graphs
- * stay. No counterpart in
- * smuthi, whose CUDA kernels launch one thread per matrix row
- * (linear_system_cuda.py:26-405, cuda_blocksize). */
+ * stay. No counterpart in smuthi, whose CUDA kernels launch one thread per
+ * matrix row (linear_system_cuda.py:26-405, cuda_blocksize). */
 int smh_op_autotune(smh_op *op, int batch, int precision, int iters, int n_cand, const int *items_per_cu,
                     const int *launch_order, double *matvec_ms, int *best);
 
@@ -308,7 +307,9 @@ int smh_op_half_interp(smh_op *op, int *terms, double *lin_ratio);
  * (solver_type 'gmres') starts from x0 = rhs as smuthi does;
  * SMH_SOLVE_MIXED / MIXED16 refine from x0 = 0. They stop at
  * ||rhs - M x|| <= tol ||rhs|| measured in FP64 and return SMH_ERR_NOCONV
- * when maxiter Arnoldi steps do not get there. SMH_SOLVE_LU (solver_type
+ * when maxiter Arnoldi steps do not get there: steps of each right-hand side,
+ * where lookup operators solve blocks of them the steps taken together.
+ * SMH_SOLVE_LU (solver_type
  * 'LU', linear_system.py:259-268, explicit operators only) factors M on the
  * device once per T (kept on the operator) and solves directly; tol, restart
  * and maxiter are not used. stats (out, 8 doubles): Arnoldi steps, FP64

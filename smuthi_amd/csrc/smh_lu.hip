@@ -81,7 +81,7 @@ __global__ void residual_parts_kernel(const double2* __restrict__ b, const doubl
 // Bound by the chain of pivots: a panel's rows stay in the registers of one
 // workgroup (two per thread), so that a pivot costs two barriers and no memory
 // access. 1800 unknowns (60 spheres, l_max 3): 13.2 ms in some 4000 launches of
-// rocSOLVER's getrf, 5.6 ms in 226 launches here, 29 us with two rows per thread
+// rocSOLVER's getrf, 5.7 ms in 226 launches here, 31 us with two rows per thread
 // and 20 with one; errors against 64 bits as getrf's (80 to 2016 unknowns). With
 // more than 2048 rows the panel no longer fits the registers, and a pass over the matrix per eight columns no
 // longer the last-level cache: getrf.
