@@ -73,14 +73,30 @@ struct PweMath<double> {
   static __device__ inline double exp2_(double x) { return exp2(x); }
 };
 
-// e^{i 2 pi t} for any t
-__device__ inline void cis_turns(double t, double& c, double& s) { sincospi(2.0 * (t - rint(t)), &s, &c); }
-__device__ inline void cis_turns(double t, float& c, float& s) { PweMath<float>::cis_rev((float)(t - rint(t)), c, s); }
+// A wavenumber in turns (over 2 pi) per length, to twice FP64's digits, and the
+// fraction of a turn of k s: the product less its whole turns is rounded once,
+// at the size of the fraction (a rounded product would leave FP64 phases 1e-16
+// of the whole argument, some hundred radians over an array).
+struct Turns {
+  double hi, lo;
+};
+__device__ inline Turns turns_of(double k) {
+  constexpr double kInvHi = 0.15915494309189535, kInvLo = -9.839338337591243e-18;  // 1 / (2 pi)
+  const double hi = k * kInvHi;
+  return {hi, fma(k, kInvLo, fma(k, kInvHi, -hi))};
+}
+__device__ inline double turn_fraction(Turns k, double s) {
+  return fma(k.lo, s, fma(k.hi, s, -rint(k.hi * s)));
+}
+
+// e^{i 2 pi t} of a fraction of a turn
+__device__ inline void cis_turns(double t, double& c, double& s) { sincospi(2.0 * t, &s, &c); }
+__device__ inline void cis_turns(double t, float& c, float& s) { PweMath<float>::cis_rev((float)t, c, s); }
 
 // e^{i kz dz}, the argument reduced in FP64 (leaves may be tall)
 template <typename Real>
 __device__ inline void z_phase(double2 kz, double dz, Real& c, Real& s) {
-  cis_turns(kz.x / kTwoPi * dz, c, s);
+  cis_turns(turn_fraction(turns_of(kz.x), dz), c, s);
   if (kz.y != 0.0) {
     const Real m = PweMath<Real>::exp2_((Real)(-kz.y * kLog2e * dz));
     c *= m;
@@ -193,12 +209,12 @@ __global__ void __launch_bounds__(256) pwe_column_kernel(PweArgs a) {
   const int k_end = min(a.n_k, ((int)blockIdx.y + 1) * a.per_split);
   for (int k = (int)blockIdx.y * a.per_split + wave; k < k_end; k += 4) {
     const double2 kp = a.kp[k], kz = a.kz[k];
-    const double kturn = kp.x / kTwoPi;
+    const Turns kturn = turns_of(kp.x);
     double A[6] = {0, 0, 0, 0, 0, 0};
     for (int j = lane; j < a.n_a; j += 64) {
       const double sxy = x0 * a.ca[j] + y0 * a.sa[j];
       double er, ei;
-      cis_turns(kturn * sxy, er, ei);
+      cis_turns(turn_fraction(kturn, sxy), er, ei);
       if (kp.y != 0.0) {
         const double mag = exp(-kp.y * sxy);
         er *= mag;
@@ -467,7 +483,7 @@ __global__ void __launch_bounds__(256) pwe_harmonics_kernel(PweArgs a) {
         const double2 kp = a.kp[k], kz = a.kz[k];
         const double sxy = x0 * a.ca[a0 + ia] + y0 * a.sa[a0 + ia];
         double er, ei;
-        cis_turns((kp.x * sxy + kz.x * z0) / kTwoPi, er, ei);
+        cis_turns(turn_fraction(turns_of(kp.x), sxy) + turn_fraction(turns_of(kz.x), z0), er, ei);
         if (kp.y != 0.0 || kz.y != 0.0) {
           const double mag = exp(-(kp.y * sxy + kz.y * z0));
           er *= mag;
@@ -954,16 +970,16 @@ extern "C" int smh_pwe_field(smh_ctx* ctx, int kind, int64_t n_k, const double* 
 // FP64 sincos of the phases (about 60 instructions per particle and alpha)
 // beside as much time in the MFMA: 90 x 361 waves, 1000 particles, l_max 3, FP64:
 // 1.34 ms when a thread summed all orders of one alpha in registers.
-// FP32 sums go through the sum over m into FP64 ones every kAsmFlush particles:
+// The MFMA's sums go through the sum over m into FP64 ones every kAsmFlush particles:
 // where the waves alone fill the chip, one workgroup sums all particles, and one
 // running FP32 sum of 10000 of them is off by 2.5e-6 (1000 x 361 waves over 60 um,
-// 15.3 ms), in this form by 3.0e-7 (16.7 ms).
+// 15.3 ms), in this form by 3.0e-7 (16.7 ms). FP64, 2000 particles: 6.6 -> 6.8 ms.
 // A launch covers kAsmOrders orders m at most; more run as several launches,
 // each adding its orders' share into g.
 namespace {
 
 constexpr int kAsmChunk = 32;   // particles staged at a time
-constexpr int kAsmFlush = 4 * kAsmChunk;  // particles of one FP32 sum
+constexpr int kAsmFlush = 4 * kAsmChunk;  // particles of one sum on the MFMA
 constexpr int kAsmTiles = 2;    // alpha tiles per wave
 constexpr int kAsmWaves = 4;
 constexpr int kAsmOrders = 12;  // orders per launch: 4 (dir, pol) each in 3 column tiles
@@ -998,7 +1014,7 @@ __global__ void __launch_bounds__(64 * kAsmWaves, sizeof(Real) == 4 ? 3 : 2) pwe
   const int k = (int)(blockIdx.x / a.a_blocks), ab = (int)(blockIdx.x - k * a.a_blocks);
   const int tile0 = (ab * (int)(blockDim.x >> 6) + wave) * kAsmTiles;
   const double2 kp = a.kp[k], kz = a.kz[k];
-  const double kturn = -kp.x / kTwoPi;        // e^{-i kappa s}: turns per nm
+  const Turns kturn = turns_of(-kp.x);        // e^{-i kappa s}
   const double klog = kp.y * kLog2e;          // |e^{-i kappa s}| = 2^(klog s)
   const bool lossy = kp.y != 0.0;
   // this lane's alpha of each tile
@@ -1079,7 +1095,7 @@ __global__ void __launch_bounds__(64 * kAsmWaves, sizeof(Real) == 4 ? 3 : 2) pwe
     }
     __syncthreads();
     if (tile0 * 16 >= a.n_a) continue;
-    if (sizeof(Real) == 4 && p0 > first && (p0 - first) % kAsmFlush == 0) flush();
+    if (p0 > first && (p0 - first) % kAsmFlush == 0) flush();
     for (int s = 0; s < (np + 3) / 4; ++s) {
       const int p = 4 * s + h;  // (particles beyond np have zero coefficients)
       Real br[CT], bi[CT];
@@ -1092,7 +1108,7 @@ __global__ void __launch_bounds__(64 * kAsmWaves, sizeof(Real) == 4 ? 3 : 2) pwe
       for (int t = 0; t < kAsmTiles; ++t) {
         const double sd = px[p] * ca[t] + py[p] * sa[t];
         Real pr, pi;
-        cis_turns(kturn * sd, pr, pi);
+        cis_turns(turn_fraction(kturn, sd), pr, pi);
         if (lossy) {
           const Real mg = exp2_split(klog * sd, Real(0));
           pr *= mg;

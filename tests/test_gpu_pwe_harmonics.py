@@ -73,3 +73,20 @@ def test_fields_match_oracle(gpu, shape, n_k, n_a, neff, lossy):
         for precision, tol in (('double', 1e-10), ('single', 3e-6 if shape not in ('sparse', 'wide patch') else 5e-5)):
             got = np.stack(getattr(made[1], field)(*args, precision=precision))
             assert np.abs(got - want).max() <= tol * np.abs(want).max(), (field, precision)
+
+
+def test_fp64_phases_of_columns_far_out(gpu):
+    """A discrete plane wave at azimuth 0 on columns 30 to 60 um out and up to 30 um high: kappa x and k_z z are
+    products of FP64 numbers, and their phases, several hundred radians, keep an absolute error of a few 1e-16 (not of
+    their own size, 1e-13)."""
+    from smuthi_amd.expansions import PlaneWaveExpansion
+    x, z = np.meshgrid([30123.4, -44567.8, 59876.5], np.linspace(100.0, 30000.0, 40))
+    x, z = x.ravel(), z.ravel()
+    for kappa in K * np.array([0.31, 0.64, 0.977]):
+        pwe = PlaneWaveExpansion(K, [kappa], [0.0], 'upgoing', [0, 0, 0], 0, np.inf)
+        pwe.coefficients[0] = 0.8 - 0.3j
+        got = pwe.electric_field(x, np.zeros_like(x), z, precision='double')[1]
+        phase = np.longdouble(kappa) * x.astype(np.longdouble) + \
+            np.longdouble(pwe.k_z()[0].real) * z.astype(np.longdouble)
+        want = (0.8 - 0.3j) * (np.cos(phase) + 1j * np.sin(phase)).astype(complex)
+        assert np.linalg.norm(got - want) <= 2e-15 * np.linalg.norm(want)

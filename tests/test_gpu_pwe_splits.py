@@ -83,6 +83,32 @@ def test_workgroups_of_several_chunks(n, l_max):
                 assert np.abs(got[d, :, k] - want).max() <= tol * np.abs(want).max(), (prec, k, d)
 
 
+def test_fp64_phases_over_a_wide_array():
+    """One particle 41 um out at azimuth 0, where kappa x is a product of two FP64 numbers: its phase, some 600
+    radians, keeps an absolute error of a few 1e-16 (not of its own size, 7e-14)."""
+    from smuthi_amd import _lib, cuda, fields
+    assert cuda.enable_gpu(), 'MI355X not available'
+    rng = np.random.default_rng(2)
+    n_k = 200
+    B = fields.blocksize(1, 1)
+    _, _, m = fields.index_arrays(1, 1)
+    xyz, z_ref = np.array([[41234.567, 0.0, 100.0]]), 100.0
+    kp = (K * rng.uniform(0.5, 1.4, n_k)).astype(complex)
+    kz = fields.k_z(k_parallel=kp, k=K).astype(complex)
+
+    def c(*s):
+        return np.ascontiguousarray(rng.standard_normal(s) + 1j * rng.standard_normal(s))
+    coef, btab, al = c(1, B), c(n_k, 2, 2, B), np.zeros(1)
+    got, ms = np.zeros((2, 2, n_k, 1), complex), ctypes.c_double()
+    _lib.check(_lib.load().smh_pwe_assemble(cuda.context(), 1, _lib.dptr(xyz), 1, 1, _lib.dptr(coef), z_ref, n_k,
+                                            _lib.dptr(kp), _lib.dptr(kz), _lib.dptr(btab), 1, _lib.dptr(al),
+                                            _lib.dptr(got), _lib.FP64, ctypes.byref(ms)), cuda.context(), 'assemble')
+    phase = kp.real.astype(np.longdouble) * np.longdouble(xyz[0, 0])
+    wave = (np.cos(phase) - 1j * np.sin(phase)).astype(complex)
+    want = (btab @ coef[0]).transpose(1, 2, 0) * wave
+    assert np.linalg.norm(got[..., 0] - want) <= 2e-15 * np.linalg.norm(want)
+
+
 def test_fp32_keeps_its_digits_over_many_particles():
     """4000 particles over 60 um that one workgroup sums (the waves alone fill the chip), lossless and lossy
     kappa. Coefficients, phases (native sine and cosine, 1e-7) and the sums of 128 particles are rounded to 32
