@@ -26,8 +26,8 @@ namespace {
 
 int blocks_of(int64_t n, int t = 256) { return (int)std::min<int64_t>((n + t - 1) / t, 1 << 20); }
 
-// M = I - diag(t) W on the padded index, row-major [n][n]
-__global__ void master_dense_kernel(const double2* __restrict__ W, const double2* __restrict__ t, int64_t n,
+// M = I - diag(t) W on the padded index, row-major [n][n], or (unit 0) M - I
+__global__ void master_dense_kernel(const double2* __restrict__ W, const double2* __restrict__ t, int64_t n, double unit,
                                     double2* __restrict__ M) {
   const int64_t total = n * n;
   for (int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; f < total; f += (int64_t)gridDim.x * blockDim.x) {
@@ -35,7 +35,7 @@ __global__ void master_dense_kernel(const double2* __restrict__ W, const double2
     const double2 w = W[f], a = t[r];
     double re = -(a.x * w.x - a.y * w.y);
     const double im = -(a.x * w.y + a.y * w.x);
-    if (r == c) re += 1.0;
+    if (r == c) re += unit;
     M[f] = make_double2(re, im);
   }
 }
@@ -81,8 +81,9 @@ __global__ void residual_parts_kernel(const double2* __restrict__ b, const doubl
 // Bound by the chain of pivots: a panel's rows stay in the registers of one
 // workgroup (two per thread), so that a pivot costs two barriers and no memory
 // access. 1800 unknowns (60 spheres, l_max 3): 13.2 ms in some 4000 launches of
-// rocSOLVER's getrf, 5.7 ms in 226 launches here, 31 us with two rows per thread
-// and 20 with one; errors against 64 bits as getrf's (80 to 2016 unknowns). With
+// rocSOLVER's getrf, 6.0 ms in 226 launches here, 34 us with two rows per thread
+// and 21 with one; solutions' errors against refined ones 4 to 8 % below getrf's
+// (spheres, 240 to 1800 unknowns: 4.7e-16 to 7.1e-16). With
 // more than 2048 rows the panel no longer fits the registers, and a pass over the matrix per eight columns no
 // longer the last-level cache: getrf.
 constexpr int kLuPanel = 8, kLuRows = 1024, kLuWaves = kLuRows / 64;
@@ -142,14 +143,20 @@ __device__ inline double2 csub(double2 a, double2 l, double2 u) {  // a - l u
 // the first launch, which only factors strip 0. Rows below the panel number at
 // most R * kLuRows. Block b < gridDim.x takes strip k / kLuPanel + 1 (b = 0,
 // if there is one) or one of the others.
+// The trailing matrix is kept without the identity of A = I - ..: a row's 1, in
+// the column it had before all exchanges (its origin), is added when its
+// column's panel is factored or its row becomes one of U. The roundings of
+// the updates, one per panel, are then of the coupling's size instead of 1.
+// origin: every row's before (in) and after (out) the factored panel's exchanges.
 template <int R>
 __global__ void __launch_bounds__(kLuRows) lu_step_kernel(double2* __restrict__ A, int64_t n, int k, LuPerm* perms,
+                                                          const int* __restrict__ origin_in, int* origin_out,
                                                           int* ipiv, int* info) {
   __shared__ double2 sv[kLuPanel][2 * kLuPanel], us[kLuPanel][kLuPanel], l11[kLuPanel][kLuPanel];
   __shared__ double2 prow[kLuPanel], orow[kLuPanel];
   __shared__ unsigned long long redk[kLuWaves];
   __shared__ unsigned redi[kLuWaves];
-  __shared__ int pivots[kLuPanel];
+  __shared__ int pivots[kLuPanel], origin[2 * kLuRows], moved[2 * kLuPanel];
   const int tid = threadIdx.x, N = (int)n, strips = (N + kLuPanel - 1) / kLuPanel;
   const int sk = k >= 0 ? k / kLuPanel : -1;  // strip of the factored panel
   int strip = sk + 1 < strips ? ((int)blockIdx.x == 0 ? sk + 1 : (int)blockIdx.x - 1) : (int)blockIdx.x;
@@ -163,6 +170,9 @@ __global__ void __launch_bounds__(kLuRows) lu_step_kernel(double2* __restrict__ 
     const int r = tid & (2 * kLuPanel - 1), c = tid / (2 * kLuPanel), count = pm.count;
     const bool mine = c < w && r < count;
     if (mine) sv[c][r] = C[c * n + pm.row[r]];
+    if (tid < count) moved[tid] = origin_in[pm.row[pm.src[tid]]];  // origins of the rows that have moved
+    if (strip == sk + 1)
+      for (int i = row0 - wk + tid; i < N; i += kLuRows) origin[i] = origin_in[i];
     if (strip > sk && tid < kLuPanel * kLuPanel) {
       const int i = tid / kLuPanel, j = tid % kLuPanel;  // L(j, i) of the panel's triangle
       l11[j][i] = A[(int64_t)(k + i) * n + k + j];
@@ -176,6 +186,7 @@ __global__ void __launch_bounds__(kLuRows) lu_step_kernel(double2* __restrict__ 
 #pragma unroll
       for (int j = 0; j < kLuPanel; ++j) {
         u[j] = sv[tid][pm.src[j]];
+        if (moved[j] == c0 + tid) u[j].x += 1.0;
 #pragma unroll
         for (int i = 0; i < j; ++i) u[j] = csub(u[j], l11[j][i], u[i]);
         us[j][tid] = u[j];
@@ -183,6 +194,7 @@ __global__ void __launch_bounds__(kLuRows) lu_step_kernel(double2* __restrict__ 
       }
     }
     __syncthreads();
+    if (strip == sk + 1 && tid < count) origin[pm.row[tid]] = moved[tid];
     // the rows below: C -= L U
     double2 l[R][kLuPanel];
 #pragma unroll
@@ -219,6 +231,7 @@ __global__ void __launch_bounds__(kLuRows) lu_step_kernel(double2* __restrict__ 
       }
     }
     if (strip != sk + 1) return;
+    __syncthreads();
   }
   // factor the strip: row row0 + tid + q kLuRows in a[q] (row0 = c0; written above by this thread)
   double2 a[R][kLuPanel];
@@ -227,6 +240,13 @@ __global__ void __launch_bounds__(kLuRows) lu_step_kernel(double2* __restrict__ 
     const int i = row0 + tid + q * kLuRows;
 #pragma unroll
     for (int cc = 0; cc < kLuPanel; ++cc) a[q][cc] = cc < w && i < N ? C[cc * n + i] : make_double2(0.0, 0.0);
+    if (i < N) {
+      const int o = k >= 0 ? origin[i] : i;
+      origin_out[i] = o;
+#pragma unroll
+      for (int cc = 0; cc < kLuPanel; ++cc)
+        if (cc < w && o == c0 + cc) a[q][cc].x += 1.0;
+    }
   }
 #pragma unroll
   for (int j = 0; j < kLuPanel; ++j) {
@@ -338,9 +358,9 @@ __global__ void __launch_bounds__(kLuRows) lu_step_kernel(double2* __restrict__ 
   }
 }
 
-// ipiv [n], info [1] and perms [strips] on the device; info is the first zero
-// pivot's column (1-based), or 0
-void lu_factor(double2* A, int64_t n, int* ipiv, int* info, LuPerm* perms, hipStream_t s) {
+// Factors I + A. ipiv [n], info [1], perms [strips] and origin [2 n] on the
+// device; info is the first zero pivot's column (1-based), or 0
+void lu_factor(double2* A, int64_t n, int* ipiv, int* info, LuPerm* perms, int* origin, hipStream_t s) {
   const int strips = (int)((n + kLuPanel - 1) / kLuPanel);
   (void)hipMemsetAsync(info, 0, sizeof(int), s);
   for (int st = -1; st < strips; ++st) {
@@ -348,7 +368,8 @@ void lu_factor(double2* A, int64_t n, int* ipiv, int* info, LuPerm* perms, hipSt
     const int blocks = st < 0 ? 1 : strips - 1;  // all strips but the factored one
     if (blocks == 0) break;
     const auto kern = n - (k + kLuPanel) > kLuRows ? lu_step_kernel<2> : lu_step_kernel<1>;
-    hipLaunchKernelGGL(kern, dim3(blocks), dim3(kLuRows), 0, s, A, n, k, perms, ipiv, info);
+    hipLaunchKernelGGL(kern, dim3(blocks), dim3(kLuRows), 0, s, A, n, k, perms, (const int*)origin + (st & 1) * n,
+                       origin + ((st + 1) & 1) * n, ipiv, info);
   }
 }
 
@@ -387,9 +408,10 @@ int lu_solve(smh_op* op, const double* t_diag, const double* rhs, double* x, int
   double* d_parts = nullptr;
   int* d_info = nullptr;
   LuPerm* d_perms = nullptr;
+  int* d_origin = nullptr;
   constexpr int kParts = 256;
   auto done = [&](int code) {
-    void* p[] = {d_t, d_b, d_x, d_y, d_parts, d_info, d_perms};
+    void* p[] = {d_t, d_b, d_x, d_y, d_parts, d_info, d_perms, d_origin};
     for (void* q : p)
       if (q) (void)hipFree(q);
     return code;
@@ -423,12 +445,14 @@ int lu_solve(smh_op* op, const double* t_diag, const double* rhs, double* x, int
       LU_HIP(hipMalloc(&op->d_piv, (size_t)n * sizeof(int)));
     }
     op->lu_t.clear();
+    const bool own = n <= 2 * kLuRows;
     hipLaunchKernelGGL(master_dense_kernel, dim3(blocks_of(n * n)), dim3(256), 0, s, (const double2*)op->d_W64,
-                       (const double2*)d_t, n, op->d_lu);
+                       (const double2*)d_t, n, own ? 0.0 : 1.0, op->d_lu);
     LU_HIP(hipGetLastError());
-    if (n <= 2 * kLuRows) {
+    if (own) {
       LU_HIP(hipMalloc(&d_perms, (size_t)((n + kLuPanel - 1) / kLuPanel) * sizeof(LuPerm)));
-      lu_factor(op->d_lu, n, op->d_piv, d_info, d_perms, s);
+      LU_HIP(hipMalloc(&d_origin, (size_t)2 * n * sizeof(int)));
+      lu_factor(op->d_lu, n, op->d_piv, d_info, d_perms, d_origin, s);
       LU_HIP(hipGetLastError());
     } else {
       const rocblas_status st = rocsolver_zgetrf(h, (rocblas_int)n, (rocblas_int)n,
