@@ -352,15 +352,17 @@ __global__ void __launch_bounds__(256) explicit_gemv_kernel(const void* __restri
 // reads 64 contiguous bytes of its row, which are its K values of the turn's
 // MFMA 16x16x4 steps (the column order inside a turn is the lanes' own, the same
 // for W and X). The 16 result columns are (vector, re | im): Re W meets (Re x,
-// Im x), Im W meets (-Im x, Re x), the other half of the lane pair. Even and odd
-// steps and the two products keep sums of their own, the waves' sums are added
-// at the end. Bound by HBM on W, read once for all vectors: the next turn's
+// Im x), Im W meets (-Im x, Re x), the other half of the lane pair. The sums stay
+// as short as those of one vector's product (a wavefront per row), whose error
+// is the bound: FP32 chains of eight terms go to FP64 sums, FP64 has a sum per
+// step of a turn, and the waves' sums are added pairwise (one running sum of
+// each kind: errors 20 to 29 % larger at 320 to 640 unknowns). Bound by HBM on W, read once for all vectors: the next turn's
 // loads are in flight during the products, and eight waves of four such
 // workgroups keep about 130 KB per CU outstanding. The columns are cut into
 // gridDim.y shares, whose sums explicit_gemm_sum_kernel adds: 9000 unknowns
 // are 563 workgroups for the rows alone, two on some CUs and three on others
-// (FP32: 264 us, 2.45 TB/s; with 4 shares 210 us, 3.1 TB/s; FP64 316 -> 252 us,
-// 5.1 TB/s).
+// (FP32: 264 us, with 4 shares 210; FP64 316 -> 252 us, 5.1 TB/s). In FP32 the
+// short chains are the faster ones as well: 210 -> 137 us, 4.7 TB/s.
 constexpr int kGemmWaves = 8, kGemmShares = 8;
 template <typename Real>
 __global__ void __launch_bounds__(64 * kGemmWaves)
@@ -369,16 +371,38 @@ __global__ void __launch_bounds__(64 * kGemmWaves)
   using M = smh::Mfma<Real>;
   using R2 = typename smh::Vec2<Real>::t;
   constexpr int J = 64 / (int)sizeof(R2), kCols = 4 * J;  // columns per lane and per turn
-  __shared__ Real part[kGemmWaves][16][16];
+  constexpr bool kF32 = sizeof(Real) == 4;
+  constexpr int kSums = kF32 ? 2 : J;  // sums of each product
+  __shared__ double part[kGemmWaves][16][16];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, q = lane >> 4, c = lane & 15;
   const int64_t row0 = (int64_t)blockIdx.x * 16;
   const int64_t row = min(row0 + c, n - 1);  // rows beyond n repeat the last one (not stored)
   const R2* W = (const R2*)Wv + row * n;
   const Real* x = (const Real*)xv + c;  // this lane's column (vector, re | im) of X
   const Real sgn = (c & 1) ? Real(1) : Real(-1);
-  typename M::v4 acc[4];
+  typename M::v4 acc[2][kSums];
+  double sum[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-  for (int i = 0; i < 4; ++i) acc[i] = typename M::v4{0, 0, 0, 0};
+  for (int i = 0; i < kSums; ++i) acc[0][i] = acc[1][i] = typename M::v4{0, 0, 0, 0};
+  // the sums into the wave's FP64 one, pairwise
+  auto gather = [&]() {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      double t[2 * kSums];
+#pragma unroll
+      for (int i = 0; i < kSums; ++i) {
+        t[2 * i] = (double)acc[0][i][v];
+        t[2 * i + 1] = (double)acc[1][i][v];
+      }
+#pragma unroll
+      for (int d = 1; d < 2 * kSums; d *= 2)
+#pragma unroll
+        for (int i = 0; i + d < 2 * kSums; i += 2 * d) t[i] += t[i + d];
+      sum[v] += t[0];
+    }
+#pragma unroll
+    for (int i = 0; i < kSums; ++i) acc[0][i] = acc[1][i] = typename M::v4{0, 0, 0, 0};
+  };
   auto load = [&](int64_t c0, R2 (&w)[J], Real (&b)[J]) {
     const int64_t k0 = c0 + q * J;
     if constexpr (sizeof(Real) == 4) {
@@ -400,8 +424,9 @@ __global__ void __launch_bounds__(64 * kGemmWaves)
   auto multiply = [&](const R2 (&w)[J], const Real (&b)[J]) {
 #pragma unroll
     for (int j = 0; j < J; ++j) {
-      acc[j & 1] = M::op(w[j].x, b[j], acc[j & 1]);
-      acc[2 + (j & 1)] = M::op(w[j].y, sgn * smh::lane_xor1(b[j]), acc[2 + (j & 1)]);
+      acc[0][j % kSums] = M::op(w[j].x, b[j], acc[0][j % kSums]);
+      acc[1][j % kSums] = M::op(w[j].y, sgn * smh::lane_xor1(b[j]), acc[1][j % kSums]);
+      if (kF32 && j % 4 == 3) gather();
     }
   };
   const int64_t turns = n / kCols;
@@ -433,18 +458,20 @@ __global__ void __launch_bounds__(64 * kGemmWaves)
     }
     multiply(w, b);
   }
+  if (!kF32) gather();
 #pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const int r = M::kRowIs4q ? 4 * q + v : 4 * v + q;
-    part[wave][r][c] = (acc[0][v] + acc[1][v]) + (acc[2][v] + acc[3][v]);
-  }
+  for (int v = 0; v < 4; ++v) part[wave][M::kRowIs4q ? 4 * q + v : 4 * v + q][c] = sum[v];
   __syncthreads();
   if (threadIdx.x < 256) {
     const int r = threadIdx.x >> 4, k = threadIdx.x & 15;
-    Real s = part[0][r][k];
+    double t[kGemmWaves];
 #pragma unroll
-    for (int w = 1; w < kGemmWaves; ++w) s += part[w][r][k];
-    if (row0 + r < n) ((Real*)yv)[((int64_t)blockIdx.y * n + row0 + r) * 16 + k] = s;
+    for (int w = 0; w < kGemmWaves; ++w) t[w] = part[w][r][k];
+#pragma unroll
+    for (int d = 1; d < kGemmWaves; d *= 2)
+#pragma unroll
+      for (int w = 0; w < kGemmWaves; w += 2 * d) t[w] += t[w + d];
+    if (row0 + r < n) ((Real*)yv)[((int64_t)blockIdx.y * n + row0 + r) * 16 + k] = (Real)t[0];
   }
 }
 
@@ -452,9 +479,9 @@ template <typename Real>
 __global__ void explicit_gemm_sum_kernel(const Real* __restrict__ part, int64_t n16, int shares, Real* __restrict__ y) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n16) return;
-  Real s = part[e];
-  for (int k = 1; k < shares; ++k) s += part[k * n16 + e];
-  y[e] = s;
+  double s = (double)part[e];
+  for (int k = 1; k < shares; ++k) s += (double)part[k * n16 + e];
+  y[e] = (Real)s;
 }
 
 }  // namespace
