@@ -90,9 +90,10 @@ constexpr int kLuPanel = 8, kLuRows = 1024, kLuWaves = kLuRows / 64;
 
 // Row exchanges of a panel, as one permutation of the rows it touches:
 // row[t] takes the value of row[src[t]]; row[j] = first column + j, j < width.
+// origin[t]: of the row that comes to row[t] (lu_step_kernel).
 struct LuPerm {
   int count;
-  int row[2 * kLuPanel], src[2 * kLuPanel];
+  int row[2 * kLuPanel], src[2 * kLuPanel], origin[2 * kLuPanel];
 };
 
 __device__ inline double2 cfma(double2 a, double2 l, double2 u) {  // a + l u
@@ -170,7 +171,7 @@ __global__ void __launch_bounds__(kLuRows) lu_step_kernel(double2* __restrict__ 
     const int r = tid & (2 * kLuPanel - 1), c = tid / (2 * kLuPanel), count = pm.count;
     const bool mine = c < w && r < count;
     if (mine) sv[c][r] = C[c * n + pm.row[r]];
-    if (tid < count) moved[tid] = origin_in[pm.row[pm.src[tid]]];  // origins of the rows that have moved
+    if (tid < count) moved[tid] = pm.origin[tid];
     if (strip == sk + 1)
       for (int i = row0 - wk + tid; i < N; i += kLuRows) origin[i] = origin_in[i];
     if (strip > sk && tid < kLuPanel * kLuPanel) {
@@ -349,10 +350,12 @@ __global__ void __launch_bounds__(kLuRows) lu_step_kernel(double2* __restrict__ 
       if (tid == j) src = sb;
       if (tid == b) src = sj;
     }
+    const int from = __shfl(row, src);
     LuPerm& pm = perms[strip];
     if (tid < count) {
       pm.row[tid] = row;
       pm.src[tid] = src;
+      pm.origin[tid] = k >= 0 ? origin[from] : from;
     }
     if (tid == 0) pm.count = count;
   }
